@@ -426,7 +426,6 @@ __global__ void k_fill_u64(unsigned long long *p, uint64_t n, unsigned long long
 // ------------------------------------------------------------------- main tile
 
 constexpr int BM = 128, BN = 128; // output tile of every MatMul kernel here
-constexpr unsigned kGfx950Cus = 256; // compute units of a gfx950 device (MI350X, MI355X)
 
 // Tile shape of the vector-unit kernel: 128 x 128 outputs per 256-thread workgroup (8 x 8
 // per thread); binary64 stages twice as deep a k-slab, halving its barriers.
@@ -1710,7 +1709,8 @@ bool matmul_bt_wanted(int dtype, uint64_t rows, uint64_t inner, uint64_t cols, b
     // 4096^3 -2%), and 4.5-7% slower on the 64 x 64 tiles of smaller grids (1024^3 NT 57.1
     // against 54.6 us).
     return rows % 128 == 0 && cols % 128 == 0 && (rows / 128) * (cols / 128) >= 256 &&
-           inner * cols <= kBtMaxElems;
+           inner * cols <= kBtMaxElems &&
+           (dtype != 0 || mid_tile_f32(rows, cols, inner, true) == MidTile::k128);
 }
 
 // The exponent screen of op(A) rows and op(B) columns, both jobs in one launch.

@@ -17,8 +17,8 @@
 //    both terms are), and x + (+0) = x + (-0) for every x != -0.
 // The two blocks of one MFMA carry k and k+1 for the same 32x32 output tile, so one
 // instruction yields 2048 products and a lane adds its 16 cells' k-product, then their
-// (k+1)-product. Small grids of whole 64x64 tiles use v_mfma_f32_16x16x1_4b_f32 the same
-// way (k_strict_gemm_mfma16): its four blocks carry k..k+3 for one 16x16 output tile.
+// (k+1)-product. Outputs that do not divide into full rounds of 128x128 tiles use
+// v_mfma_f32_16x16x1_4b_f32 the same way (matmul_mid.hip).
 //
 // Fault screening (non-finite result, exponent prefilter) and the exact replay of suspect
 // cells are shared with the VALU kernel; these kernels record a workgroup's first suspect
@@ -61,13 +61,6 @@ __device__ __forceinline__ void load_lds16(const float *base, uint32_t off, floa
                  : "memory", "m0");
 }
 __device__ __forceinline__ void wait_lds_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-// Wait until at most N of this wave's vector memory loads are outstanding: loads complete in
-// the order they were issued, so every load before the last N has landed.
-template <int N> __device__ __forceinline__ void wait_loads_but()
-{
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
 // WHOLE: every slab of every tile is whole (M, N, K multiples of the tile and slab, 16-byte
 // loads allowed), so staging runs on advancing pointers with no bound checks.
 // CHECK: the RejectSubnormal form with the partial-sum check (sck), its own instantiation so
@@ -222,11 +215,10 @@ __global__ __launch_bounds__(Cfg::kThreads, Cfg::kWavesPerSimd) void k_strict_ge
         // and issues its first MFMA before the barrier that ends slab kt: the MFMA runs while
         // the wave waits there, and no slab starts from an empty pipeline.
         //
-        // With two subtiles a wave (SN = 2), lane col of subtile j owns tile column
-        // wn + 2 col + j, so its two B operands of a k row sit side by side and one 8-byte LDS
-        // read, at an immediate offset from the lane's base, fetches both. With one (SN = 1) it
-        // owns column wn + col.
-        static_assert(SM == 1 && (SN == 1 || SN == 2), "the pipeline below is written for one or two subtiles a wave");
+        // Lane col of subtile j owns tile column wn + 2 col + j, so its two B operands of a k
+        // row sit side by side and one 8-byte LDS read, at an immediate offset from the lane's
+        // base, fetches both.
+        static_assert(SM == 1 && SN == 2, "the pipeline below is written for two subtiles a wave");
         //
         // Direct loads: each wave moves 1 KiB of op(A) and 1 KiB of op(B) per slab, lane l's 16
         // bytes landing at the wave's LDS base + 16 l. Stage layouts (floats):
@@ -274,7 +266,7 @@ __global__ __launch_bounds__(Cfg::kThreads, Cfg::kWavesPerSimd) void k_strict_ge
             lo_b = row_run(BN, (uint64_t)N);
             db = (size_t)BK * N;
             lb = 256 * wv;
-            b_off = row_off(BN, SN == 2 ? wn + 2 * col : wn + col);
+            b_off = row_off(BN, wn + 2 * col);
         }
         // Stage the next slab into stage ST: direct loads, or global -> registers (the stash
         // to LDS follows at the end of the slab).
@@ -307,12 +299,10 @@ __global__ __launch_bounds__(Cfg::kThreads, Cfg::kWavesPerSimd) void k_strict_ge
         // Software pipeline over the slab, unrolled: each MFMA is issued, then the products of
         // the one before it are folded. sched_barrier pins that order (left to the scheduler,
         // the same sequence measured about 8% slower). Each k-pair's operands are read from
-        // LDS ahead into register slots used in turn: one pair ahead into two slots with two
-        // subtiles (their MFMAs alternate within a pair), two pairs ahead into three slots
-        // with one (each pair's MFMA is issued before the previous pair is folded). Lanes
-        // 0-31 carry k = 2j, lanes 32-63 carry k = 2j + 1 (the MFMA's two blocks).
+        // LDS one pair ahead into two register slots used in turn. Lanes 0-31 carry k = 2j,
+        // lanes 32-63 carry k = 2j + 1 (the MFMA's two blocks).
         constexpr int NP = BK / 2;
-        constexpr int kSlots = SN == 2 ? 2 : 3, D = kSlots - 1;
+        constexpr int kSlots = 2, D = kSlots - 1;
         static_assert((3 * NP) % kSlots == 0, "a trip of three slabs ends on slot 0");
         // Register slot of pair j of the trip's slab c (j may run into the next slab).
         auto slot = [](int c, int j) { return (c * NP + j) % kSlots; };
@@ -322,19 +312,13 @@ __global__ __launch_bounds__(Cfg::kThreads, Cfg::kWavesPerSimd) void k_strict_ge
                 oa[g] = (&sa(st_c)[0][0])[a_off + (TA ? 2 * BM * j : 4 * BM * (j >> 1) + 2 * (j & 1))];
             else
                 oa[g] = sa(st_c)[2 * j + half][wm + col];
-            if constexpr (SN == 2) {
-                float2 v;
-                if constexpr (kDirectB)
-                    v = *reinterpret_cast<const float2 *>(&sb(st_c)[0][0] + b_off + 2 * BN * j);
-                else
-                    v = *reinterpret_cast<const float2 *>(&sb(st_c)[2 * j + half][wn + 2 * col]);
-                ob[g][0] = v.x;
-                ob[g][SN - 1] = v.y;
-            } else if constexpr (kDirectB) {
-                ob[g][0] = (&sb(st_c)[0][0])[b_off + 2 * BN * j];
-            } else {
-                ob[g][0] = sb(st_c)[2 * j + half][wn + col];
-            }
+            float2 v;
+            if constexpr (kDirectB)
+                v = *reinterpret_cast<const float2 *>(&sb(st_c)[0][0] + b_off + 2 * BN * j);
+            else
+                v = *reinterpret_cast<const float2 *>(&sb(st_c)[2 * j + half][wn + 2 * col]);
+            ob[g][0] = v.x;
+            ob[g][1] = v.y;
         };
         v32f p;
         if (ktiles > 0) {
@@ -359,27 +343,15 @@ __global__ __launch_bounds__(Cfg::kThreads, Cfg::kWavesPerSimd) void k_strict_ge
                 else if (has_next)
                     rd(nxt_c, slot(cur, j + D), j + D - NP);
                 const int g = slot(cur, j), g1 = slot(cur, j + 1);
-                if constexpr (SN == 2) {
-                    const v32f q = mma(oa[g], ob[g][SN - 1]);
-                    __builtin_amdgcn_sched_barrier(0);
-                    fold(acc[0], p, ck);
-                    __builtin_amdgcn_sched_barrier(0);
-                    if (j + 1 < NP || has_next)
-                        p = mma(oa[g1], ob[g1][0]);
-                    __builtin_amdgcn_sched_barrier(0);
-                    fold(acc[SN - 1], q, ck);
-                    __builtin_amdgcn_sched_barrier(0);
-                } else {
-                    v32f q;
-                    const bool more = j + 1 < NP || has_next;
-                    if (more)
-                        q = mma(oa[g1], ob[g1][0]);
-                    __builtin_amdgcn_sched_barrier(0);
-                    fold(acc[0], p, ck);
-                    __builtin_amdgcn_sched_barrier(0);
-                    if (more)
-                        p = q;
-                }
+                const v32f q = mma(oa[g], ob[g][1]);
+                __builtin_amdgcn_sched_barrier(0);
+                fold(acc[0], p, ck);
+                __builtin_amdgcn_sched_barrier(0);
+                if (j + 1 < NP || has_next)
+                    p = mma(oa[g1], ob[g1][0]);
+                __builtin_amdgcn_sched_barrier(0);
+                fold(acc[1], q, ck);
+                __builtin_amdgcn_sched_barrier(0);
             }
             if (kt + 2 < ktiles)
                 stash_slab(nn_c);
@@ -428,43 +400,22 @@ __global__ __launch_bounds__(Cfg::kThreads, Cfg::kWavesPerSimd) void k_strict_ge
                 for (int jj = 0; jj < SN; jj++)
                     ob[j][jj] = Bs[cur][2 * j + half][wn + 32 * jj + col];
             };
-            static_assert(SM == 1 && (SN == 1 || SN == 2), "the pipeline below is written for one or two subtiles a wave");
-            if constexpr (SN == 2) {
-                rd(0);
-                v32f p = mma(oa[0][0], ob[0][0]);
+            static_assert(SM == 1 && SN == 2, "the pipeline below is written for two subtiles a wave");
+            rd(0);
+            v32f p = mma(oa[0][0], ob[0][0]);
 #pragma unroll
-                for (int j = 0; j < NP; j++) {
-                    if (j + 1 < NP)
-                        rd(j + 1);
-                    const v32f q = mma(oa[j][0], ob[j][SN - 1]);
-                    __builtin_amdgcn_sched_barrier(0);
-                    fold(acc[0], p, ck);
-                    __builtin_amdgcn_sched_barrier(0);
-                    if (j + 1 < NP)
-                        p = mma(oa[j + 1][0], ob[j + 1][0]);
-                    __builtin_amdgcn_sched_barrier(0);
-                    fold(acc[SN - 1], q, ck);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            } else {
-                // One subtile: each pair's MFMA is issued before the previous pair is folded,
-                // operands read two pairs ahead.
-                rd(0);
-                rd(1);
-                v32f p = mma(oa[0][0], ob[0][0]);
-#pragma unroll
-                for (int j = 0; j < NP; j++) {
-                    if (j + 2 < NP)
-                        rd(j + 2);
-                    v32f q;
-                    if (j + 1 < NP)
-                        q = mma(oa[j + 1][0], ob[j + 1][0]);
-                    __builtin_amdgcn_sched_barrier(0);
-                    fold(acc[0], p, ck);
-                    __builtin_amdgcn_sched_barrier(0);
-                    if (j + 1 < NP)
-                        p = q;
-                }
+            for (int j = 0; j < NP; j++) {
+                if (j + 1 < NP)
+                    rd(j + 1);
+                const v32f q = mma(oa[j][0], ob[j][1]);
+                __builtin_amdgcn_sched_barrier(0);
+                fold(acc[0], p, ck);
+                __builtin_amdgcn_sched_barrier(0);
+                if (j + 1 < NP)
+                    p = mma(oa[j + 1][0], ob[j + 1][0]);
+                __builtin_amdgcn_sched_barrier(0);
+                fold(acc[1], q, ck);
+                __builtin_amdgcn_sched_barrier(0);
             }
             if (kt + 1 < ktiles)
                 stage.stash(As[cur ^ 1], Bs[cur ^ 1], tid);
@@ -478,30 +429,11 @@ __global__ __launch_bounds__(Cfg::kThreads, Cfg::kWavesPerSimd) void k_strict_ge
     }
 
     // Epilogue: for subtile (i, j) the lane owns rows m0+wm+32i+8(r/4)+4*half+(r%4) of column
-    // n0+wn+2col+j (three stages, two subtiles: both columns in one 8-byte store, every cell
+    // n0+wn+2col+j (three stages: both columns in one 8-byte store, every cell
     // inside M x N) or n0+wn+32j+col.
     const bool sub = CHECK && ((subl.flush() >> lane) & 1);
     uint64_t key = kNoFault;
-    if constexpr (kStages == 3 && SN == 1) {
-        const int c = n0 + wn + col;
-        const int cexp = check_risk ? exp_of(col_exp[c]) : 0;
-        if (sub) // the lane's cells: rows m0 + wm .. m0 + wm + 31 of column c
-            flag_sum_block(sck, m0 + wm, c);
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const int row = m0 + wm + 8 * (r >> 2) + 4 * half + (r & 3);
-            const float v = acc[0][r];
-            C[(size_t)row * N + c] = v;
-            bool bad = !finite_bits(v) || sub;
-            if (check_risk)
-                bad |= exp_of(row_exp[row]) + cexp < thr;
-            const uint64_t cell = (uint64_t)row * N + c;
-            if (bad)
-                key = cell < key ? cell : key;
-        }
-        block_record_min<Cfg::kThreads / 64>(key, suspect);
-        return;
-    } else if constexpr (kStages == 3) {
+    if constexpr (kStages == 3) {
         const int c = n0 + wn + 2 * col;
         const int cexp0 = check_risk ? exp_of(col_exp[c]) : 0;
         const int cexp1 = check_risk ? exp_of(col_exp[c + 1]) : 0;
@@ -650,205 +582,6 @@ __global__ __launch_bounds__(Cfg::kThreads, Cfg::kWavesPerSimd) void k_strict_ge
     block_record_min<Cfg::kThreads / 64>(key, suspect);
 }
 
-// ------------------------------------------------------- 16 x 16 waves, whole tiles
-// Outputs too small to give every SIMD several 32 x 32 waves (fewer 128 x 128 tiles than
-// CUs): 64 x 64 tiles of sixteen 16 x 16 waves, four times the waves of 32 x 32 subtiles.
-// v_mfma_f32_16x16x1_4b_f32 multiplies, in block b, A lane 16 b + i by B lane 16 b + j, and
-// lane L's register 4 b + q holds block b's (i = 4 (L / 16) + q, j = L % 16). The four blocks
-// carry k0 .. k0 + 3, so each lane folds, for each of its four cells q, registers q, 4 + q,
-// 8 + q and 12 + q in k order: 16 adds per 1024 products, the same ceiling as the 32 x 32
-// engine. Both operands load straight into LDS in every layout:
-//  * k-contiguous (op(A) untransposed, op(B) transposed): k quads, element (k, x) at
-//    256 (k / 4) + 4 x + k % 4; one wave instruction fills a quad (64 rows of 16 bytes), and
-//    a lane's operand read (x = w + L % 16, k = 4 q + L / 16) covers 64 consecutive words;
-//  * x-contiguous (op(A) transposed, op(B) untransposed): k rows of 64 floats, row k rotated
-//    by 16 (k % 4), element (k, x) at 64 k + (x + 16 (k % 4)) % 64; one instruction fills four
-//    rows, each lane fetching the global run that lands rotated, and the read (four rows, 16
-//    columns each) meets 64 distinct banks.
-typedef float v16f __attribute__((ext_vector_type(16)));
-
-template <bool TA, bool TB, bool CHECK = false>
-__global__ __launch_bounds__(1024, 2) void k_strict_gemm_mfma16(
-    const float *__restrict__ A, const float *__restrict__ B, float *__restrict__ C, int M,
-    int N, int K, const unsigned long long *__restrict__ row_exp,
-    const unsigned long long *__restrict__ col_exp, int thr, int check_risk,
-    unsigned long long *suspect, SumCheck sck, NodeGate gate)
-{
-    if (block_gate_closed(gate))
-        return;
-    constexpr int T = 64, BK = 16, SZ = T * BK; // tile side, slab, floats a stage
-    __shared__ __align__(16) float As0[SZ], As1[SZ], As2[SZ];
-    __shared__ __align__(16) float Bs0[SZ], Bs1[SZ], Bs2[SZ];
-    auto sa = [&](auto st_c) -> float * {
-        constexpr int st = decltype(st_c)::value;
-        return st == 0 ? As0 : (st == 1 ? As1 : As2);
-    };
-    auto sb = [&](auto st_c) -> float * {
-        constexpr int st = decltype(st_c)::value;
-        return st == 0 ? Bs0 : (st == 1 ? Bs1 : Bs2);
-    };
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = 16 * (wv >> 2), wn = 16 * (wv & 3);
-    int tm, tn;
-    tile_of(blockIdx.x, M / T, N / T, tm, tn);
-    const int m0 = tm * T, n0 = tn * T;
-    // RejectSubnormal with the partial-sum check: each form takes its own tiles, as in
-    // k_strict_gemm_mfma.
-    if (sck.flag != nullptr &&
-        tile_exp_sum_below<T, T>(row_exp, col_exp, m0, n0, M, N, sck.thr) != CHECK)
-        return;
-    SubLanes subl;
-    const int cls = kClassSubnormal;
-    __shared__ unsigned char fine_ss[kSumMaxSuperSlabs];
-    SumGate<BK> sgate{nullptr, false};
-    bool chk = true; // the current slab's sums are checked (checking form)
-    if constexpr (CHECK) {
-        if (sck.tbl_a != nullptr) {
-            tile_fine_superslabs<T, T>(sck, m0, n0, M, N, K, fine_ss);
-            sgate.fine = fine_ss;
-        }
-    }
-
-    // Loads: waves 0-3 move op(A), waves 4-7 op(B), one 1 KiB instruction each a slab
-    // (quad g or rows 4 g .. 4 g + 3 of the slab, g = wave % 4).
-    const bool loads = wv < 8, load_a = wv < 4;
-    const int g = wv & 3;
-    const bool kcontig = load_a ? !TA : TB;        // this wave's operand is k-contiguous
-    const float *X = load_a ? A : B;
-    const int ld = load_a ? (TA ? M : K) : (TB ? K : N);
-    const int x0 = load_a ? m0 : n0;
-    const float *gx = nullptr; // wave-uniform base, advancing BK along k a slab
-    uint32_t lo = 0;          // the lane's byte offset from it
-    size_t dk = 0;
-    if (loads) {
-        if (kcontig) {
-            gx = X + (size_t)x0 * ld + 4 * g;
-            lo = (uint32_t)lane * (uint32_t)ld * 4u;
-            dk = BK;
-        } else {
-            const int r = lane >> 4, c = lane & 15;
-            gx = X + (size_t)(4 * g) * ld + x0;
-            lo = (uint32_t)((r * ld + 4 * ((c - 4 * r) & 15)) * 4);
-            dk = (size_t)BK * ld;
-        }
-    }
-    // In both layouts instruction g fills floats 256 g .. 256 g + 255 of the stage.
-    auto load_slab = [&](auto st_c) {
-        if (loads) {
-            load_lds16(gx, lo, (load_a ? sa(st_c) : sb(st_c)) + 256 * g);
-            gx += dk;
-        }
-    };
-    // The lane's operand offsets in a stage (quad q adds 256 q in both layouts).
-    const int i = lane & 15, b = lane >> 4;
-    const int oa = !TA ? 4 * (wm + i) + b : 64 * b + ((wm + i + 16 * b) & 63);
-    const int ob = TB ? 4 * (wn + i) + b : 64 * b + ((wn + i + 16 * b) & 63);
-
-    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    v16f zero;
-#pragma unroll
-    for (int r = 0; r < 16; r++)
-        zero[r] = 0.0f;
-    // Fold one MFMA's products: each cell q adds its k0, k0 + 1, k0 + 2, k0 + 3 products in
-    // turn; the four cells' chains interleave.
-    auto fold = [&](const v16f &p, auto ck) {
-        constexpr bool CK = decltype(ck)::value;
-#pragma unroll
-        for (int blk = 0; blk < 4; blk++) {
-#pragma unroll
-            for (int q = 0; q < 4; q++)
-                acc[q] = acc[q] + p[4 * blk + q];
-            if constexpr (CK) {
-                if (chk)
-                    check_subnormal4(subl, acc[0], acc[1], acc[2], acc[3], cls);
-            }
-        }
-        asm volatile("" : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]));
-    };
-    const int ktiles = K / BK;
-    if (ktiles > 0) {
-        load_slab(std::integral_constant<int, 0>{});
-        if (ktiles > 1)
-            load_slab(std::integral_constant<int, 1>{});
-    }
-    wait_lds_loads();
-    __syncthreads();
-    auto slab = [&](auto cur_c, int kt, auto ck) __attribute__((always_inline)) {
-        constexpr int cur = decltype(cur_c)::value;
-        if (kt + 2 < ktiles)
-            load_slab(std::integral_constant<int, (cur + 2) % 3>{});
-        const float *as = sa(cur_c), *bs = sb(cur_c);
-        float a[4], bb[4];
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            a[q] = as[oa + 256 * q];
-            bb[q] = bs[ob + 256 * q];
-        }
-        v16f p = __builtin_amdgcn_mfma_f32_16x16x1f32(a[0], bb[0], zero, 0, 0, 0);
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            v16f nx;
-            if (q + 1 < 4)
-                nx = __builtin_amdgcn_mfma_f32_16x16x1f32(a[q + 1], bb[q + 1], zero, 0, 0, 0);
-            __builtin_amdgcn_sched_barrier(0);
-            fold(p, ck);
-            __builtin_amdgcn_sched_barrier(0);
-            if (q + 1 < 4)
-                p = nx;
-        }
-        // The next slab must be in LDS before the barrier publishes it; a loading wave's
-        // one load for slab kt + 2, issued this slab, may stay in flight.
-        if (loads && kt + 2 < ktiles)
-            wait_loads_but<1>();
-        else
-            wait_lds_loads();
-        __syncthreads();
-    };
-    auto off_grid = [&]() {
-        bool o = false;
-#pragma unroll
-        for (int q = 0; q < 4; q++)
-            o |= sum_off_grid(acc[q]);
-        return __builtin_amdgcn_ballot_w64(o) != 0;
-    };
-    auto gated = [&](auto cur_c, int kt, auto ck) __attribute__((always_inline)) {
-        if constexpr (decltype(ck)::value)
-            chk = sgate.at(kt, off_grid);
-        slab(cur_c, kt, ck);
-    };
-    auto run = [&](auto ck) {
-        for (int kt = 0; kt < ktiles; kt += 3) {
-            gated(std::integral_constant<int, 0>{}, kt, ck);
-            if (kt + 1 < ktiles)
-                gated(std::integral_constant<int, 1>{}, kt + 1, ck);
-            if (kt + 2 < ktiles)
-                gated(std::integral_constant<int, 2>{}, kt + 2, ck);
-        }
-    };
-    run(std::integral_constant<bool, CHECK>{});
-    // Epilogue: cells (m0 + wm + 4 (lane / 16) + q, n0 + wn + lane % 16).
-    const bool sub = CHECK && ((subl.flush() >> lane) & 1);
-    uint64_t key = kNoFault;
-    const int c = n0 + wn + i;
-    const int cexp = check_risk ? exp_of(col_exp[c]) : 0;
-    if (sub) // rows m0 + wm .. m0 + wm + 15 of column c: one 32 x 32 block
-        flag_sum_block(sck, m0 + wm, c);
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const int row = m0 + wm + 4 * b + q;
-        const float v = acc[q];
-        C[(size_t)row * N + c] = v;
-        bool bad = !finite_bits(v) || sub;
-        if (check_risk)
-            bad |= exp_of(row_exp[row]) + cexp < thr;
-        const uint64_t cell = (uint64_t)row * N + c;
-        if (bad)
-            key = cell < key ? cell : key;
-    }
-    block_record_min<16>(key, suspect);
-}
-
 static inline bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
 
 // Measurement aid: a copy of known traffic whose reads are global_load_lds_dwordx4, the load
@@ -899,22 +632,20 @@ static void mfma_dispatch(hipStream_t s, const float *A, const float *B, float *
     const bool offsets32 = 4 * span_a <= UINT32_MAX && (TB || 4 * span_b <= UINT32_MAX);
     const bool whole = va && vb && M % Cfg::BM == 0 && N % Cfg::BN == 0 && K % Cfg::BK == 0 &&
                        ((uintptr_t)C & 7u) == 0 && offsets32;
-    if constexpr (Cfg::SN == 2) {
-        // The whole-tile epilogue evaluates an elementwise node with the product.
-        if (whole && epi && (epi->op == kStepRelu || epi->op == kStepReluBackward)) {
-            if (epi->op == kStepRelu) {
-                hipLaunchKernelGGL((k_strict_gemm_mfma<Cfg, TA, TB, true, true, true, false, kStepRelu>), grid, block, 0, s, A, B, C, M, N, K, re, ce, thr, risk, suspect, sck, gate, *epi);
-                if (sck.flag)
-                    hipLaunchKernelGGL((k_strict_gemm_mfma<Cfg, TA, TB, true, true, true, true, kStepRelu>), grid, block, 0, s, A, B, C, M, N, K, re, ce, thr, risk, suspect, sck, gate, *epi);
-            } else {
-                hipLaunchKernelGGL((k_strict_gemm_mfma<Cfg, TA, TB, true, true, true, false, kStepReluBackward>), grid, block, 0, s, A, B, C, M, N, K, re, ce, thr, risk, suspect, sck, gate, *epi);
-                if (sck.flag)
-                    hipLaunchKernelGGL((k_strict_gemm_mfma<Cfg, TA, TB, true, true, true, true, kStepReluBackward>), grid, block, 0, s, A, B, C, M, N, K, re, ce, thr, risk, suspect, sck, gate, *epi);
-            }
-            if (epi_done)
-                *epi_done = true;
-            return;
+    // The whole-tile epilogue evaluates an elementwise node with the product.
+    if (whole && epi && (epi->op == kStepRelu || epi->op == kStepReluBackward)) {
+        if (epi->op == kStepRelu) {
+            hipLaunchKernelGGL((k_strict_gemm_mfma<Cfg, TA, TB, true, true, true, false, kStepRelu>), grid, block, 0, s, A, B, C, M, N, K, re, ce, thr, risk, suspect, sck, gate, *epi);
+            if (sck.flag)
+                hipLaunchKernelGGL((k_strict_gemm_mfma<Cfg, TA, TB, true, true, true, true, kStepRelu>), grid, block, 0, s, A, B, C, M, N, K, re, ce, thr, risk, suspect, sck, gate, *epi);
+        } else {
+            hipLaunchKernelGGL((k_strict_gemm_mfma<Cfg, TA, TB, true, true, true, false, kStepReluBackward>), grid, block, 0, s, A, B, C, M, N, K, re, ce, thr, risk, suspect, sck, gate, *epi);
+            if (sck.flag)
+                hipLaunchKernelGGL((k_strict_gemm_mfma<Cfg, TA, TB, true, true, true, true, kStepReluBackward>), grid, block, 0, s, A, B, C, M, N, K, re, ce, thr, risk, suspect, sck, gate, *epi);
         }
+        if (epi_done)
+            *epi_done = true;
+        return;
     }
     if (whole)
         { hipLaunchKernelGGL((k_strict_gemm_mfma<Cfg, TA, TB, true, true, true>), grid, block, 0, s, A, B, C, M, N, K, re, ce, thr, risk, suspect, sck, gate, GemmEpilogue{}); if (sck.flag) hipLaunchKernelGGL((k_strict_gemm_mfma<Cfg, TA, TB, true, true, true, true>), grid, block, 0, s, A, B, C, M, N, K, re, ce, thr, risk, suspect, sck, gate, GemmEpilogue{}); }
@@ -946,11 +677,6 @@ static void mfma_launch(hipStream_t s, int M, int N, int K, bool ta, bool tb, co
 // 32 x 32, a 256 x 128 tile, 4-wave tiles of 128 x 64 and 64 x 64, and BK = 32 (which
 // spills with the pinned slab).
 using GemmCfg = MfmaCfg<4, 2, 1, 2, 16, 4>;
-// Outputs of fewer 128 x 128 tiles than CUs: 64 x 64 tiles of four 32 x 32 waves spread the
-// same work over four times the workgroups (one wave a SIMD on more CUs rather than two on
-// fewer).
-using SmallCfg = MfmaCfg<2, 2, 1, 1, 16, 4>;
-
 hipError_t launch_gemm_mfma_f32(hipStream_t s, int M, int N, int K, bool ta, bool tb,
                                 const float *A, const float *B, float *C,
                                 const unsigned long long *row_exp,
@@ -958,29 +684,11 @@ hipError_t launch_gemm_mfma_f32(hipStream_t s, int M, int N, int K, bool ta, boo
                                 unsigned long long *suspect, SumCheck sck, NodeGate gate,
                                 const GemmEpilogue *epi, bool *epi_done)
 {
-    const uint64_t big_tiles = (uint64_t)((M + GemmCfg::BM - 1) / GemmCfg::BM) * ((N + GemmCfg::BN - 1) / GemmCfg::BN);
-    // 16 x 16 waves: whole 64 x 64 tiles, 16-byte loads, lane offsets within 32 bits, and
-    // at most one round of their workgroups (two 16-wave workgroups a CU): measured 25-30%
-    // faster than the 4-wave 64 x 64 tile at 1024^3, 512 x 4096 x 512 and 768 x 2048 x 768,
-    // 3% slower at 1920 x 1024 x 1920 (900 tiles).
-    const auto fits32 = [](uint64_t bytes) { return bytes <= UINT32_MAX; };
-    const uint64_t lda = ta ? (uint64_t)M : (uint64_t)K, ldb = tb ? (uint64_t)K : (uint64_t)N;
-    const bool w16 = M % 64 == 0 && N % 64 == 0 && K % 16 == 0 && aligned16(A) && aligned16(B) &&
-                     (uint64_t)(M / 64) * (N / 64) <= 512 &&
-                     fits32(ta ? (3 * lda + 64) * 4 : 64 * lda * 4) &&
-                     fits32(tb ? 64 * ldb * 4 : (3 * ldb + 64) * 4);
-    if (big_tiles < 256 && w16) {
-        const dim3 grid((unsigned)((M / 64) * (N / 64)));
-        if (!ta && !tb) { hipLaunchKernelGGL((k_strict_gemm_mfma16<false, false>), grid, dim3(1024), 0, s, A, B, C, M, N, K, row_exp, col_exp, thr, risk, suspect, sck, gate); if (sck.flag) hipLaunchKernelGGL((k_strict_gemm_mfma16<false, false, true>), grid, dim3(1024), 0, s, A, B, C, M, N, K, row_exp, col_exp, thr, risk, suspect, sck, gate); }
-        else if (!ta && tb) { hipLaunchKernelGGL((k_strict_gemm_mfma16<false, true>), grid, dim3(1024), 0, s, A, B, C, M, N, K, row_exp, col_exp, thr, risk, suspect, sck, gate); if (sck.flag) hipLaunchKernelGGL((k_strict_gemm_mfma16<false, true, true>), grid, dim3(1024), 0, s, A, B, C, M, N, K, row_exp, col_exp, thr, risk, suspect, sck, gate); }
-        else if (ta && !tb) { hipLaunchKernelGGL((k_strict_gemm_mfma16<true, false>), grid, dim3(1024), 0, s, A, B, C, M, N, K, row_exp, col_exp, thr, risk, suspect, sck, gate); if (sck.flag) hipLaunchKernelGGL((k_strict_gemm_mfma16<true, false, true>), grid, dim3(1024), 0, s, A, B, C, M, N, K, row_exp, col_exp, thr, risk, suspect, sck, gate); }
-        else { hipLaunchKernelGGL((k_strict_gemm_mfma16<true, true>), grid, dim3(1024), 0, s, A, B, C, M, N, K, row_exp, col_exp, thr, risk, suspect, sck, gate); if (sck.flag) hipLaunchKernelGGL((k_strict_gemm_mfma16<true, true, true>), grid, dim3(1024), 0, s, A, B, C, M, N, K, row_exp, col_exp, thr, risk, suspect, sck, gate); }
-        return hipGetLastError();
-    }
-    if (big_tiles < 256)
-        mfma_launch<SmallCfg>(s, M, N, K, ta, tb, A, B, C, row_exp, col_exp, thr, risk, suspect, sck, gate);
-    else
-        mfma_launch<GemmCfg>(s, M, N, K, ta, tb, A, B, C, row_exp, col_exp, thr, risk, suspect, sck, gate, epi, epi_done);
+    const bool whole = M % GemmCfg::BM == 0 && N % GemmCfg::BN == 0 && K % GemmCfg::BK == 0;
+    const MidTile tile = mid_tile_f32((uint64_t)M, (uint64_t)N, (uint64_t)K, whole);
+    if (tile != MidTile::k128 && mid_fits_f32((uint64_t)M, (uint64_t)N, (uint64_t)K, ta, tb))
+        return launch_gemm_mid_f32(s, tile, M, N, K, ta, tb, A, B, C, row_exp, col_exp, thr, risk, suspect, sck, gate);
+    mfma_launch<GemmCfg>(s, M, N, K, ta, tb, A, B, C, row_exp, col_exp, thr, risk, suspect, sck, gate, epi, epi_done);
     return hipGetLastError();
 }
 

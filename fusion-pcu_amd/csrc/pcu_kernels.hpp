@@ -192,6 +192,20 @@ hipError_t launch_gemm_mfma_f32(hipStream_t s, int M, int N, int K, bool ta, boo
                                 unsigned long long *suspect, SumCheck sck, NodeGate gate,
                                 const GemmEpilogue *epi = nullptr, bool *epi_done = nullptr);
 
+constexpr unsigned kGfx950Cus = 256; // compute units of a gfx950 device (MI350X, MI355X)
+
+// Output tile of the matrix-core engine: 128 x 128 (matmul_mfma.hip), or the smaller tiles of
+// matmul_mid.hip. `whole`: M, N and K are multiples of the 128 x 128 tile and its slab.
+enum class MidTile { k32, k64, k128 };
+MidTile mid_tile_f32(uint64_t M, uint64_t N, uint64_t K, bool whole);
+// Whether matmul_mid.hip can address the operands.
+bool mid_fits_f32(uint64_t M, uint64_t N, uint64_t K, bool ta, bool tb);
+hipError_t launch_gemm_mid_f32(hipStream_t s, MidTile tile, int M, int N, int K, bool ta, bool tb,
+                               const float *A, const float *B, float *C,
+                               const unsigned long long *row_exp, const unsigned long long *col_exp,
+                               int thr, int risk, unsigned long long *suspect, SumCheck sck,
+                               NodeGate gate);
+
 // C[rows x cols] = op(A) * op(B), k ascending, each multiply and add rounded on its own.
 // Every kernel of the op skips its work once `gate` shows that an earlier program node
 // faulted (that earlier fault is reported).

@@ -1,0 +1,78 @@
+"""The strict F32 MatMul's smaller tiles at the sizes where they can go wrong: the edges of the
+32 x 32 and 64 x 64 tiles, slabs of 32 k and their remainders, operands whose rows are and are
+not 16-byte aligned, in every layout, under every policy, with and without faults. Outputs are
+bit-exact and first faults exact against the oracle."""
+import numpy as np
+import pytest
+
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx(pcu_pkg):
+    c = pcu_pkg.Context(0)
+    # The screened tile kernels at every size (the default engine computes the smallest
+    # outputs in one fused launch).
+    c.set_matmul_engine("mfma_products")
+    yield c
+    c.close()
+
+
+def _check(ctx, pcu_pkg, a, b, tl, tr, policy):
+    ref, rf = oracle.matmul(a, b, tl, tr, policy=policy)
+    try:
+        got = ctx.strict_matmul(ctx.upload(a), ctx.upload(b), tl, tr, policy).numpy()
+        fault = None
+    except pcu_pkg.PcuExecutionError as e:
+        f = e.tensor_fault
+        fault = (f.element_index, f.reduction_index, int(f.step), int(f.kind))
+    want = None if rf is None else (rf.element_index, rf.reduction_index, rf.step, rf.kind)
+    assert fault == want, (a.shape, b.shape, tl, tr, policy)
+    if want is None:
+        np.testing.assert_array_equal(got.view(np.uint32), ref.view(np.uint32))
+
+
+def _operands(rng, m, k, n, tl, tr):
+    a = rng.uniform(-1, 1, (k, m) if tl else (m, k)).astype(np.float32)
+    b = rng.uniform(-1, 1, (n, k) if tr else (k, n)).astype(np.float32)
+    return a, b
+
+
+# 32 x 32 tiles (few cells) and 64 x 64 tiles (more than three 32 x 32 tiles a CU).
+@pytest.mark.parametrize("m,n", [(1, 1), (31, 33), (32, 64), (36, 68), (65, 127), (896, 1024),
+                                 (900, 1028), (897, 1031)])
+@pytest.mark.parametrize("tl", [False, True])
+@pytest.mark.parametrize("tr", [False, True])
+def test_tile_edges_and_slab_remainders(ctx, pcu_pkg, m, n, tl, tr):
+    rng = np.random.default_rng(m * 7 + n)
+    small = m * n < 100000
+    # None, one, two, three, four and five slabs of 32, whole and with 1 to 31 k over.
+    for k in (1, 4, 31, 32, 33, 64, 68, 95, 96, 100, 127, 128, 132, 161) if small else (4, 61, 96, 132, 163):
+        a, b = _operands(rng, m, k, n, tl, tr)
+        _check(ctx, pcu_pkg, a, b, tl, tr, 0)
+
+
+@pytest.mark.parametrize("m,k,n", [(70, 100, 90), (68, 132, 92), (901, 70, 1030), (904, 100, 1032)])
+@pytest.mark.parametrize("policy", [0, 1, 2])
+@pytest.mark.parametrize("layout", [(False, False), (False, True), (True, False), (True, True)])
+def test_tiles_first_fault_and_partial_sums(ctx, pcu_pkg, m, k, n, policy, layout):
+    """Operands next to the tiles' edges replaced by values that fault (not a number, an
+    overflow, a tiny product) or leave a subnormal partial sum (rejected under policy 1 only):
+    in the last row, column and k, inside the slab remainder."""
+    tl, tr = layout
+    rng = np.random.default_rng(m + 10 * policy + 100 * tl + 1000 * tr)
+    for special in (np.nan, np.float32(3e38), np.float32(1e-30), None):
+        a, b = _operands(rng, m, k, n, tl, tr)
+        av, bv = (a.T if tl else a), (b.T if tr else b)
+        if special is None:
+            # One cell's sum is 2^-130 after the first k of the remainder, exactly.
+            kk = k - 3
+            av[m - 1, :], bv[:, n - 1] = 0, 0
+            av[m - 1, kk], bv[kk, n - 1] = np.float32(2.0 ** -70), np.float32(2.0 ** -60)
+            av[m - 1, kk + 1], bv[kk + 1, n - 1] = 1, 1
+        else:
+            av[m - 1, k - 1] = special
+            bv[k - 1, n - 1] = special
+        _check(ctx, pcu_pkg, a, b, tl, tr, policy)
