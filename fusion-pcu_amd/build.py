@@ -37,7 +37,7 @@ COMMON = [
     f"-I{CSRC}",
 ]
 
-SOURCES = ["elementwise.hip", "matmul.hip", "matmul_mfma.hip", "matmul_mid.hip", "runtime.cpp", "graph.cpp"]
+SOURCES = ["elementwise.hip", "matmul.hip", "matmul_mfma.hip", "matmul_mid.hip", "matmul_small.hip", "runtime.cpp", "graph.cpp"]
 
 
 def _compile(src: str) -> str:

@@ -23,10 +23,9 @@
 //                 flagged have their K products classified in parallel by a wave. Both stop
 //                 once the earliest fault found lies before the cells still to visit. The
 //                 fault-free path returns at once.
-// Small outputs (engine auto) take one fused launch instead, k_strict_gemm_fused: each
-// 16 x 16 block screens its own rows and columns, computes its cells and searches its
-// suspect cells exactly.
+// Small outputs (engine auto) take one fused launch instead (matmul_small.hip).
 #include "pcu_device.hpp"
+#include "pcu_gemm_search.hpp"
 #include "pcu_gemm_stage.hpp"
 #include "pcu_kernels.hpp"
 
@@ -1164,106 +1163,6 @@ __global__ __launch_bounds__(256, 2) void k_gemm_tiny_scan(
 
 // --------------------------------------------------------------- exact replay
 
-// Lane l's value of v, on every lane (l uniform across the wave).
-__device__ __forceinline__ float lane_value(float v, int l)
-{
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
-}
-__device__ __forceinline__ double lane_value(double v, int l)
-{
-    const uint64_t x = bits_of(v);
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)x, l);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(x >> 32), l);
-    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
-}
-
-// First fault of one output cell, found by a whole wave (every lane returns the same). One
-// pass over k in chunks of 64, the next chunk's operands loaded while the current one is
-// classified: the lanes form the chunk's products and classify them, which gives the
-// chunk's first faulting Multiply. When `walk_adds` is set (a non-finite result, where a sum
-// can overflow, or RejectSubnormal, where a subnormal sum faults), every lane then folds the
-// chunk's products before that Multiply in k order, as the contract orders the sums. Those
-// products are finite, so a sum there can only fault by overflowing (the running sum turns,
-// and stays, infinite) or, under RejectSubnormal, by being subnormal: the chunk is folded
-// with plain adds and that check, and only a chunk that trips it is folded again with the
-// exact add classifier to name the step. A Multiply at k comes before the Add at k. Returns
-// kNoFault or the packed fault word.
-template <typename T>
-__device__ __forceinline__ uint64_t cell_first_fault(const T *__restrict__ A, const T *__restrict__ B,
-                                                     uint64_t M, uint64_t N, uint64_t K, int ta,
-                                                     int tb, uint64_t cell, int policy,
-                                                     bool walk_adds)
-{
-    const int lane = threadIdx.x & 63;
-    const uint64_t r = cell / N, c = cell % N;
-    auto load = [&](uint64_t k0, T &a, T &b) {
-        const uint64_t k = k0 + lane;
-        a = (T)0;
-        b = (T)0;
-        if (k < K) {
-            a = ta ? A[k * M + r] : A[r * K + k];
-            b = tb ? B[c * K + k] : B[k * N + c];
-        }
-    };
-    const bool reject_sub = policy == kPolicyRejectSubnormal;
-    T total = (T)0;
-    T a, b;
-    load(0, a, b);
-    for (uint64_t k0 = 0; k0 < K; k0 += 64) {
-        T na = (T)0, nb = (T)0;
-        if (k0 + 64 < K)
-            load(k0 + 64, na, nb);
-        const T p = a * b;
-        uint32_t kind = kOk;
-        if (k0 + lane < K)
-            kind = classify_mul(a, b, p, policy);
-        const uint64_t mask = __ballot(kind != kOk);
-        const int l_m = mask ? __ffsll((long long)mask) - 1 : 64;
-        if (walk_adds) {
-            const int in_k = K - k0 < 64 ? (int)(K - k0) : 64;
-            const int here = l_m < in_k ? l_m : in_k; // products summed before any fault
-            T t = total;
-            bool sub = false;
-            if (here == 64) {
-#pragma unroll
-                for (int j = 0; j < 64; j++) {
-                    t = t + lane_value(p, j);
-                    sub |= reject_sub && subnormal(t);
-                }
-            } else {
-                for (int j = 0; j < here; j++) {
-                    t = t + lane_value(p, j);
-                    sub |= reject_sub && subnormal(t);
-                }
-            }
-            if (!finite_bits(t) || sub) {
-                for (int j = 0; j < here; j++) {
-                    const T pj = lane_value(p, j);
-                    const T nxt = total + pj;
-                    const uint32_t k_add = classify_add(total, pj, nxt, policy);
-                    if (k_add != kOk)
-                        return pack_fault((cell * K + k0 + j) * 2 + 1, k_add);
-                    total = nxt;
-                }
-            }
-            total = t;
-        }
-        if (mask)
-            return pack_fault((cell * K + k0 + l_m) * 2, __shfl(kind, l_m, 64));
-        a = na;
-        b = nb;
-    }
-    return kNoFault;
-}
-
-// Lane 0's value, on every lane of the wave.
-__device__ __forceinline__ uint64_t wave_uniform_u64(uint64_t v)
-{
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
-    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-    return ((uint64_t)hi << 32) | lo;
-}
-
 // Two passes over the suspect cells, one wave per cell, each recording the earliest fault
 // it finds with atomicMin and stopping once that lies before the cells it has left. Every
 // loop is bounded, and each wave's branches are uniform, so each ballot sees its 64 lanes.
@@ -1388,161 +1287,6 @@ __global__ __launch_bounds__(1024) void k_strict_gemm_replay(
         }
     }
     }();
-    program_close_block(close);
-}
-
-// ------------------------------------------------------------ small outputs
-// Outputs of at most fused_cells<T>() cells: one launch does the whole strict MatMul, spread
-// over many CUs. Each 256-thread workgroup owns a 16 x 16 block of cells and walks k in chunks of
-// kFusedBK, staging its op(A) rows and op(B) columns in LDS (k contiguous) and folding their
-// smallest exponents as it stages them: a block sees all of k for its rows and columns, so
-// it screens its own cells. Each thread computes one cell in k order with separately rounded
-// products and sums. A cell is suspect when its result is not finite or its row and column
-// exponents allow a tiny product (as in the screened path); a block with suspects walks them
-// in cell order with the exact per-cell search, a wave per cell, stops once its earliest
-// fault lies before the cells left, and folds that fault into the node's word with
-// atomicMin, so the word ends with the MatMul's first fault.
-constexpr int kFusedBK = 128;
-// Measured against the screened path (whole calls): binary32 1.2-1.6x faster up to 256 x 256
-// outputs, even at 512 x 2048 x 512, 2.4x slower at 1024^3; binary64 2.3-2.9x faster up to
-// 512 x 512, 1.4x slower at 1024^3.
-template <typename T> constexpr uint64_t fused_cells() { return sizeof(T) == 4 ? 256 * 256 : 512 * 512; }
-
-template <typename T, bool TA, bool TB>
-__global__ __launch_bounds__(256) void k_strict_gemm_fused(
-    const T *__restrict__ A, const T *__restrict__ B, T *__restrict__ C, int M, int N, int K,
-    int thr, int risk, int policy, unsigned long long *fault, NodeGate gate, ProgramClose close)
-{
-    if (block_gate_closed(gate)) {
-        program_close_block(close);
-        return;
-    }
-    constexpr int P = 16 / (int)sizeof(T), BKP = kFusedBK + P; // row pitch: one 16-byte pad
-    __shared__ __align__(16) T As[16][BKP];
-    __shared__ __align__(16) T Bs[16][BKP];
-    __shared__ int rexp[16], cexp[16];
-    __shared__ unsigned long long best; // this block's earliest fault
-    __shared__ int n_cand, wave_cnt[4];
-    __shared__ short cand[256];
-    const int tid = threadIdx.x, ty = tid >> 4, tx = tid & 15;
-    const int tiles_n = (N + 15) / 16;
-    const int m0 = (int)(blockIdx.x / tiles_n) * 16, n0 = (int)(blockIdx.x % tiles_n) * 16;
-    if (tid < 16) {
-        rexp[tid] = kExpNone;
-        cexp[tid] = kExpNone;
-    }
-    if (tid == 0)
-        best = kNoFault;
-    // Thread t stages one row of op(A) and one column of op(B), every 16th k of the chunk,
-    // in an order that keeps each global access coalesced.
-    const int ra = TA ? tx : ty, ka = TA ? ty : tx; // op(A) row, first k
-    const int cb = TB ? ty : tx, kb = TB ? tx : ty; // op(B) column, first k
-    T acc = (T)0;
-    for (int k0 = 0; k0 < K; k0 += kFusedBK) {
-        const int kc = K - k0 < kFusedBK ? K - k0 : kFusedBK;
-        __syncthreads(); // the previous chunk is consumed
-        // All of the thread's loads of the chunk are issued before any is used, so the chunk
-        // arrives in one round trip.
-        constexpr int L = kFusedBK / 16;
-        T va[L], vb[L];
-        const int row = m0 + ra, col = n0 + cb;
-#pragma unroll
-        for (int j = 0; j < L; j++) {
-            const int k = ka + 16 * j;
-            va[j] = (T)0;
-            if (k < kc && row < M)
-                va[j] = TA ? A[(size_t)(k0 + k) * M + row] : A[(size_t)row * K + k0 + k];
-        }
-#pragma unroll
-        for (int j = 0; j < L; j++) {
-            const int k = kb + 16 * j;
-            vb[j] = (T)0;
-            if (k < kc && col < N)
-                vb[j] = TB ? B[(size_t)col * K + k0 + k] : B[(size_t)(k0 + k) * N + col];
-        }
-        int ea = kExpNone, eb = kExpNone;
-#pragma unroll
-        for (int j = 0; j < L; j++) {
-            const int k = ka + 16 * j;
-            if (k < kc) {
-                As[ra][k] = va[j];
-                const int e = ilog2_abs(va[j]);
-                ea = e < ea ? e : ea;
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < L; j++) {
-            const int k = kb + 16 * j;
-            if (k < kc) {
-                Bs[cb][k] = vb[j];
-                const int e = ilog2_abs(vb[j]);
-                eb = e < eb ? e : eb;
-            }
-        }
-        if (ea < kExpNone)
-            atomicMin(&rexp[ra], ea);
-        if (eb < kExpNone)
-            atomicMin(&cexp[cb], eb);
-        __syncthreads();
-        int k = 0;
-        for (; k + P <= kc; k += P) {
-            const uint4 av = *reinterpret_cast<const uint4 *>(&As[ty][k]);
-            const uint4 bv = *reinterpret_cast<const uint4 *>(&Bs[tx][k]);
-            const T *a = reinterpret_cast<const T *>(&av);
-            const T *b = reinterpret_cast<const T *>(&bv);
-#pragma unroll
-            for (int j = 0; j < P; j++) {
-                const T p = a[j] * b[j];
-                acc = acc + p;
-            }
-        }
-        for (; k < kc; k++) {
-            const T p = As[ty][k] * Bs[tx][k];
-            acc = acc + p;
-        }
-    }
-    __syncthreads(); // every exponent folded
-    const int row = m0 + ty, col = n0 + tx;
-    bool sus = false;
-    if (row < M && col < N) {
-        C[(size_t)row * N + col] = acc;
-        sus = !finite_bits(acc) || (risk && rexp[ty] + cexp[tx] < thr);
-    }
-    // The block's suspect cells in cell order (tile index ty * 16 + tx grows with it).
-    const int lane = tid & 63, wave = tid >> 6;
-    const uint64_t mask = __ballot(sus);
-    if (lane == 0)
-        wave_cnt[wave] = __popcll(mask);
-    __syncthreads();
-    int before = 0;
-    for (int w = 0; w < wave; w++)
-        before += wave_cnt[w];
-    if (sus)
-        cand[before + __popcll(mask & ((1ull << lane) - 1))] = (short)tid;
-    if (tid == 0)
-        n_cand = wave_cnt[0] + wave_cnt[1] + wave_cnt[2] + wave_cnt[3];
-    __syncthreads();
-    const int nc = n_cand;
-    if (nc == 0) {
-        program_close_block(close);
-        return;
-    }
-    for (int j = wave; j < nc; j += 4) {
-        const int i = cand[j];
-        const uint64_t cell = (uint64_t)(m0 + (i >> 4)) * N + n0 + (i & 15);
-        const uint64_t bw = wave_uniform_u64(__atomic_load_n(&best, __ATOMIC_RELAXED));
-        if (bw != kNoFault && ((bw >> 3) / 2) / (uint64_t)K < cell)
-            break; // cells only grow along the list
-        const uint64_t w = cell_first_fault(A, B, (uint64_t)M, (uint64_t)N, (uint64_t)K, (int)TA,
-                                            (int)TB, cell, policy, true);
-        if (w != kNoFault && lane == 0)
-            atomicMin(&best, (unsigned long long)w);
-    }
-    __syncthreads();
-    if (tid == 0 && best != kNoFault) {
-        atomicMin(fault, best);
-        gate_record(gate);
-    }
     program_close_block(close);
 }
 
@@ -1702,7 +1446,7 @@ bool matmul_bt_wanted(int dtype, uint64_t rows, uint64_t inner, uint64_t cols, b
     // faster (4563 against 4523), its op(A) read-ahead path already hides the staging.
     if (dtype != 0 && tl)
         return false;
-    if (engine == kEngineAuto && rows * cols <= fused_cells<float>())
+    if (engine == kEngineAuto && gemm_small_wanted(dtype, rows, inner, cols))
         return false; // the fused small-output launch reads B in place
     // Whole 128 x 128 tiles filling at least one workgroup a CU: the copy measured 2-2.5%
     // faster there (NT 4096^3 1973 against 2021 us, 4096 x 1024 x 4096 510 against 521, TT
@@ -1815,29 +1559,21 @@ static hipError_t strict_matmul_t(hipStream_t s, uint64_t M, uint64_t K, uint64_
     SumCheck sck = sum_check ? SumCheck{sc.sum_flag, sc.gen, sc.flag_cols, sub_thr} : SumCheck{};
     if (ev)
         (void)hipEventRecord(ev[0], s);
-    if (engine == kEngineAuto && K > 0 && M * N <= fused_cells<T>()) {
+    if (engine == kEngineAuto && K > 0 && gemm_small_wanted(f32 ? 0 : 1, M, K, N)) {
         // A program's first node opens the program before any block can record a fault.
         if (open.words)
             hipLaunchKernelGGL(k_matmul_open, dim3(1), dim3(256), 0, s, sc.suspect, open);
         if (ev)
             (void)hipEventRecord(ev[1], s);
-        const dim3 grid((unsigned)(((M + 15) / 16) * ((N + 15) / 16)));
-        if (grid.x > kCloseMaxBlocks)
-            close = ProgramClose{}; // the publication launch ends the program
-        if (closed)
-            *closed = close.words != nullptr;
-        const int m = (int)M, n = (int)N, k = (int)K;
-        // The fused kernel walks every cell its exponents mark (no partial-sum check).
-        const int fthr = reject ? sub_thr : tiny_thr;
-        if (!ta && !tb) hipLaunchKernelGGL((k_strict_gemm_fused<T, false, false>), grid, dim3(256), 0, s, A, B, C, m, n, k, fthr, risk, policy, fault, gate, close);
-        else if (!ta && tb) hipLaunchKernelGGL((k_strict_gemm_fused<T, false, true>), grid, dim3(256), 0, s, A, B, C, m, n, k, fthr, risk, policy, fault, gate, close);
-        else if (ta && !tb) hipLaunchKernelGGL((k_strict_gemm_fused<T, true, false>), grid, dim3(256), 0, s, A, B, C, m, n, k, fthr, risk, policy, fault, gate, close);
-        else hipLaunchKernelGGL((k_strict_gemm_fused<T, true, true>), grid, dim3(256), 0, s, A, B, C, m, n, k, fthr, risk, policy, fault, gate, close);
+        // The small kernel walks every cell its exponents mark (no partial-sum check).
+        const hipError_t e = launch_gemm_small(s, f32 ? 0 : 1, (int)M, (int)N, (int)K, ta, tb, A, B, C,
+                                               reject ? sub_thr : tiny_thr, risk, policy, fault, gate,
+                                               close, closed);
         if (ev) {
             (void)hipEventRecord(ev[2], s);
             (void)hipEventRecord(ev[3], s);
         }
-        return hipGetLastError();
+        return e;
     }
     // The superslab tables let the tiny scan read only the runs of k where a product below
     // 2^tiny_thr is possible; the screen fills them wherever the scan may run (IEEE, and

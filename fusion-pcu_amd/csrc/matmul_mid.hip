@@ -524,7 +524,7 @@ static void mid_layout(hipStream_t s, MidTile tile, int M, int N, int K, const f
 // above: no single bound on the number of tiles does (a 2050 x 2050 output takes 541 us on
 // 289 128 x 128 tiles, two rounds for one, and 329 on 4225 of 32 x 32; 8190 x 8190 takes 1119
 // and 1303).
-MidTile mid_tile_f32(uint64_t M, uint64_t N, uint64_t K, bool whole)
+static MidTile mid_choose(uint64_t M, uint64_t N, uint64_t K, bool whole, double &us)
 {
     const auto per_cu = [&](uint64_t t) {
         const uint64_t tiles = ((M + t - 1) / t) * ((N + t - 1) / t);
@@ -534,9 +534,25 @@ MidTile mid_tile_f32(uint64_t M, uint64_t N, uint64_t K, bool whole)
     const double t32 = c32 <= 3 ? (9.5 + 6.5 * c32) * k + 3 : c32 * (9.3 * k + 0.5);
     const double t64 = c64 <= 1 ? 36 * k + 4 : c64 * (32.5 * k + 2);
     const double t128 = c128 * ((whole ? 118 : c128 <= 1 ? 140 : 131) * k + 4);
-    if (t128 <= t32 && t128 <= t64)
+    us = t32 < t64 ? t32 : t64;
+    if (t128 <= us) {
+        us = t128;
         return MidTile::k128;
+    }
     return t32 < t64 ? MidTile::k32 : MidTile::k64;
+}
+
+MidTile mid_tile_f32(uint64_t M, uint64_t N, uint64_t K, bool whole)
+{
+    double us;
+    return mid_choose(M, N, K, whole, us);
+}
+
+double mid_time_f32(uint64_t M, uint64_t N, uint64_t K)
+{
+    double us;
+    (void)mid_choose(M, N, K, M % 128 == 0 && N % 128 == 0 && K % 16 == 0, us);
+    return us;
 }
 
 // A lane's byte offset from its operand's tile must fit 32 bits: 64 rows of the stored matrix

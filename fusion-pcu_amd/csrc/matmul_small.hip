@@ -1,0 +1,373 @@
+// Strict F32/F64 MatMul of few cells: one launch does the whole MatMul, one cell a lane.
+//
+// Each 256-thread workgroup owns 16 x 16 cells (wave w rows 4 w .. 4 w + 3, lane row r of 16
+// lanes one of them) and walks k in chunks of 4 KiB a row, staged in LDS with k contiguous. A
+// block sees all of k for its rows and columns, so it folds their smallest exponents as it
+// stages them and screens its own cells; suspect cells (a non-finite result, or exponents that
+// allow a tiny product) are walked in cell order with the exact search, a wave per cell,
+// stopping once the block's earliest fault lies before the cells left, and that fault is
+// folded into the node's word with atomicMin, so the word ends with the MatMul's first fault.
+//
+// What bounds it: the chain of sums. A wave's add that depends on the one two instructions
+// before it issues 14 cycles after it with one or two waves a SIMD, so a cell cannot take less
+// than about 14 cycles a k, whatever feeds it. op(A) is read from LDS once per 64 k (binary64:
+// 32), each lane row of 16 holding its own row's k, and reaches the product as a broadcast
+// within the lane row (row_newbcast) that costs no instruction for binary32; op(B) takes one
+// 16-byte read per 4 k (2). The next chunk's loads are in flight while a chunk is computed.
+#include "pcu_device.hpp"
+#include "pcu_gemm_search.hpp"
+#include "pcu_kernels.hpp"
+
+#include <utility>
+
+#pragma clang fp contract(off)
+
+namespace pcu {
+
+// Lane L's v, on every lane of L's row of 16 lanes.
+template <int L> __device__ __forceinline__ int row_lane(int v)
+{
+    return __builtin_amdgcn_update_dpp(0, v, 0x150 + L, 0xf, 0xf, true); // row_newbcast:L
+}
+template <int L> __device__ __forceinline__ float row_lane(float v)
+{
+    return __int_as_float(row_lane<L>(__float_as_int(v)));
+}
+template <int L> __device__ __forceinline__ double row_lane(double v)
+{
+    const int2 w = __builtin_bit_cast(int2, v);
+    return __builtin_bit_cast(double, make_int2(row_lane<L>(w.x), row_lane<L>(w.y)));
+}
+
+// Order keys of the screen: a smaller nonzero |v| has a smaller key, zero the largest, and a
+// non-finite value one above every finite one. Two instructions an element (binary64: on the
+// high word, with a nonzero low word of the tiniest subnormals standing as its last bit).
+__device__ __forceinline__ uint32_t exp_key(float v) { return (bits_of(v) << 1) - 1u; }
+__device__ __forceinline__ uint32_t exp_key(double v)
+{
+    const uint64_t b = bits_of(v);
+    const uint32_t lo = (uint32_t)b;
+    return ((((uint32_t)(b >> 32)) | (lo < 1u ? lo : 1u)) << 1) - 1u;
+}
+// floor(log2 |v|) of the key's value (binary64 subnormals: a lower bound), kExpNone for zero and
+// non-finite.
+template <typename T> __device__ __forceinline__ int key_exp(uint32_t key)
+{
+    const uint32_t b = (key + 1u) >> 1;
+    if constexpr (sizeof(T) == 4) {
+        return ilog2_abs(__uint_as_float(b));
+    } else {
+        const uint32_t e = b >> 20;
+        return b == 0 || e == 0x7ff ? kExpNone : (e ? (int)e - 1023 : -1074);
+    }
+}
+
+// f(0) .. f(N - 1), each with its number as a constant.
+template <class F, int... J>
+__device__ __forceinline__ void each_of(F &&f, std::integer_sequence<int, J...>)
+{
+    (f(std::integral_constant<int, J>{}), ...);
+}
+template <int N, class F> __device__ __forceinline__ void each(F &&f)
+{
+    each_of(f, std::make_integer_sequence<int, N>{});
+}
+
+// VA, VB: every row of the stored matrix is 16-byte aligned.
+template <typename T, bool TA, bool TB, bool VA, bool VB>
+__global__ __launch_bounds__(256, 2) void k_strict_gemm_small(
+    const T *__restrict__ A, const T *__restrict__ B, T *__restrict__ C, int M, int N, int K,
+    int thr, int risk, int policy, unsigned long long *fault, NodeGate gate, ProgramClose close)
+{
+    if (block_gate_closed(gate)) {
+        program_close_block(close);
+        return;
+    }
+    constexpr int P = 16 / (int)sizeof(T);     // elements of 16 bytes
+    constexpr int BK = 1024 / (int)sizeof(T);  // k of a chunk
+    constexpr int BKP = BK + P;                // row pitch: one 16-byte pad
+    constexpr int L = BK / (16 * P);           // 16-byte runs of each operand a thread stages
+    __shared__ __align__(16) T As[2][16][BKP];
+    __shared__ __align__(16) T Bs[2][16][BKP];
+    __shared__ uint32_t rkey[16], ckey[16];
+    __shared__ unsigned long long best; // this block's earliest fault
+    __shared__ int n_cand, wave_cnt[4];
+    __shared__ short cand[256];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int ty = tid >> 4, tx = tid & 15; // the thread's cell
+    const int tiles_n = (N + 15) / 16;
+    const int m0 = (int)(blockIdx.x / tiles_n) * 16, n0 = (int)(blockIdx.x % tiles_n) * 16;
+    if (tid < 16) {
+        rkey[tid] = 0xffffffffu;
+        ckey[tid] = 0xffffffffu;
+    }
+    if (tid == 0)
+        best = kNoFault;
+    // A thread stages runs of P k of one row of op(A) and one column of op(B), 16 P k apart, in
+    // an order that keeps each global access coalesced: 16 threads along k where k is
+    // contiguous, else 16 threads along the rows (columns).
+    const int xa = TA ? tx : ty, ka = P * (TA ? ty : tx);
+    const int xb = TB ? ty : tx, kb = P * (TB ? tx : ty);
+    const int row = m0 + xa, col = n0 + xb;
+    const T *pa = TA ? A + (row < M ? row : M - 1) : A + (size_t)(row < M ? row : M - 1) * K;
+    const T *pb = TB ? B + (size_t)(col < N ? col : N - 1) * K : B + (col < N ? col : N - 1);
+    T va[L][P], vb[L][P];
+    // One operand's runs of the chunk at k0. FULL: the chunk lies inside K, no bound checks;
+    // else elements past K are +0.
+    auto fetch = [&](const T *p, size_t ld, auto kc_c, auto vec_c, auto full_c, int kt, int k0,
+                     T (&v)[L][P]) __attribute__((always_inline)) {
+        constexpr bool KC = decltype(kc_c)::value, VEC = decltype(vec_c)::value;
+        constexpr bool FULL = decltype(full_c)::value;
+#pragma unroll
+        for (int j = 0; j < L; j++) {
+            const int k = k0 + kt + 16 * P * j;
+            if (KC && VEC && (FULL || k + P <= K)) {
+                const uint4 q = *reinterpret_cast<const uint4 *>(p + k);
+                const T *e = reinterpret_cast<const T *>(&q);
+#pragma unroll
+                for (int c = 0; c < P; c++)
+                    v[j][c] = e[c];
+            } else {
+                const T *pk = KC ? p + k : p + (size_t)k * ld;
+#pragma unroll
+                for (int c = 0; c < P; c++)
+                    v[j][c] = FULL || k + c < K ? pk[KC ? (size_t)c : c * ld] : (T)0;
+            }
+        }
+    };
+    auto fetch_chunk = [&](int k0) __attribute__((always_inline)) {
+        const std::integral_constant<bool, !TA> kca;
+        const std::integral_constant<bool, TB> kcb;
+        const std::integral_constant<bool, VA> veca;
+        const std::integral_constant<bool, VB> vecb;
+        if (k0 + BK <= K) {
+            fetch(pa, (size_t)M, kca, veca, std::true_type{}, ka, k0, va);
+            fetch(pb, (size_t)N, kcb, vecb, std::true_type{}, kb, k0, vb);
+        } else {
+            fetch(pa, (size_t)M, kca, veca, std::false_type{}, ka, k0, va);
+            fetch(pb, (size_t)N, kcb, vecb, std::false_type{}, kb, k0, vb);
+        }
+    };
+    uint32_t amin = 0xffffffffu, bmin = 0xffffffffu;
+    auto stash_chunk = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < L; j++) {
+            uint4 qa, qb;
+            T *ea = reinterpret_cast<T *>(&qa), *eb = reinterpret_cast<T *>(&qb);
+#pragma unroll
+            for (int c = 0; c < P; c++) {
+                ea[c] = va[j][c];
+                eb[c] = vb[j][c];
+                const uint32_t x = exp_key(va[j][c]), y = exp_key(vb[j][c]);
+                amin = x < amin ? x : amin;
+                bmin = y < bmin ? y : bmin;
+            }
+            *reinterpret_cast<uint4 *>(&As[buf][xa][ka + 16 * P * j]) = qa;
+            *reinterpret_cast<uint4 *>(&Bs[buf][xb][kb + 16 * P * j]) = qb;
+        }
+    };
+    T acc = (T)0;
+    // 16 P k of the stage are a block: lane tx of a lane row holds its row's k = P tx ..
+    // P tx + P - 1 of it, and group j of P k takes lane j's.
+    constexpr int BL = 16 * P;
+    auto load16 = [](const T *p, T (&v)[P]) __attribute__((always_inline)) {
+        const uint4 q = *reinterpret_cast<const uint4 *>(p);
+        const T *e = reinterpret_cast<const T *>(&q);
+#pragma unroll
+        for (int c = 0; c < P; c++)
+            v[c] = e[c];
+    };
+    auto products = [](auto j_c, const T (&a)[P], const T (&b)[P], T (&p)[P]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int c = 0; c < P; c++)
+            p[c] = row_lane<decltype(j_c)::value>(a[c]) * b[c];
+    };
+    // `blocks` whole blocks, four k at a time. While four products are summed the next four
+    // are formed, and op(B) is read 16 k ahead (an LDS read takes longer than 12); the last
+    // block's reads ahead repeat its own first groups.
+    constexpr int G = 4 / P, NQ = 16 / G; // groups of four k; fours a block
+    auto whole_blocks = [&](const T *as, const T *bs, int blocks) __attribute__((always_inline)) {
+        T a[P], an[P], b[4][G][P], p[2][G][P];
+        load16(as + P * tx, a);
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+#pragma unroll
+            for (int g = 0; g < G; g++)
+                load16(bs + 4 * q + P * g, b[q][g]);
+        products(std::integral_constant<int, 0>{}, a, b[0][0], p[0][0]);
+        products(std::integral_constant<int, G - 1>{}, a, b[0][G - 1], p[0][G - 1]);
+        for (int i = 0; i < blocks; i++) {
+            const int ahead = i + 1 < blocks ? BL : 0;
+            as += ahead;
+            load16(as + P * tx, an);
+            each<NQ>([&](auto q_c) __attribute__((always_inline)) {
+                constexpr int q = decltype(q_c)::value, n = (q + 1) % NQ; // n: the next four
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int g = 0; g < G; g++)
+                    load16(bs + (q < NQ - 4 ? 4 * (q + 4) : ahead + 4 * (q + 4 - NQ)) + P * g, b[q & 3][g]);
+                const T(&x)[P] = q + 1 < NQ ? a : an;
+                products(std::integral_constant<int, G * n>{}, x, b[n & 3][0], p[n & 1][0]);
+                if constexpr (G == 2)
+                    products(std::integral_constant<int, G * n + G - 1>{}, x, b[n & 3][G - 1], p[n & 1][G - 1]);
+#pragma unroll
+                for (int g = 0; g < G; g++)
+#pragma unroll
+                    for (int c = 0; c < P; c++)
+                        acc = acc + p[q & 1][g][c];
+            });
+            __builtin_amdgcn_sched_barrier(0);
+            bs += ahead;
+#pragma unroll
+            for (int c = 0; c < P; c++)
+                a[c] = an[c];
+        }
+    };
+    // The last, partial block: whole groups only (zeros pad the last).
+    auto part_block = [&](const T *as, const T *bs, int left) __attribute__((always_inline)) {
+        T a[P];
+        load16(as + P * tx, a);
+        each<16>([&](auto j_c) __attribute__((always_inline)) {
+            constexpr int j = decltype(j_c)::value;
+            if (j * P < left) {
+                T b[P], p[P];
+                load16(bs + P * j, b);
+                products(j_c, a, b, p);
+#pragma unroll
+                for (int c = 0; c < P; c++)
+                    acc = acc + p[c];
+            }
+        });
+    };
+    fetch_chunk(0);
+    stash_chunk(0);
+    __syncthreads();
+    for (int k0 = 0, buf = 0; k0 < K; k0 += BK, buf ^= 1) {
+        const int kc = K - k0 < BK ? K - k0 : BK;
+        const bool next = k0 + BK < K;
+        if (next)
+            fetch_chunk(k0 + BK);
+        if (kc >= BL)
+            whole_blocks(&As[buf][ty][0], &Bs[buf][tx][0], kc / BL);
+        if (kc % BL != 0)
+            part_block(&As[buf][ty][kc / BL * BL], &Bs[buf][tx][kc / BL * BL], kc % BL);
+        if (next) {
+            stash_chunk(buf ^ 1);
+            __syncthreads();
+        }
+    }
+    if (amin != 0xffffffffu)
+        atomicMin(&rkey[xa], amin);
+    if (bmin != 0xffffffffu)
+        atomicMin(&ckey[xb], bmin);
+    __syncthreads(); // every exponent folded
+    const int crow = m0 + ty, ccol = n0 + tx;
+    bool sus = false;
+    if (crow < M && ccol < N) {
+        C[(size_t)crow * N + ccol] = acc;
+        sus = !finite_bits(acc) || (risk && key_exp<T>(rkey[ty]) + key_exp<T>(ckey[tx]) < thr);
+    }
+    // The block's suspect cells in cell order (tile index ty * 16 + tx grows with it).
+    const uint64_t mask = __ballot(sus);
+    if (lane == 0)
+        wave_cnt[wave] = __popcll(mask);
+    __syncthreads();
+    int before = 0;
+    for (int w = 0; w < wave; w++)
+        before += wave_cnt[w];
+    if (sus)
+        cand[before + __popcll(mask & ((1ull << lane) - 1))] = (short)tid;
+    if (tid == 0)
+        n_cand = wave_cnt[0] + wave_cnt[1] + wave_cnt[2] + wave_cnt[3];
+    __syncthreads();
+    const int nc = n_cand;
+    if (nc == 0) {
+        program_close_block(close);
+        return;
+    }
+    for (int j = wave; j < nc; j += 4) {
+        const int i = cand[j];
+        const uint64_t cell = (uint64_t)(m0 + (i >> 4)) * N + n0 + (i & 15);
+        const uint64_t bw = wave_uniform_u64(__atomic_load_n(&best, __ATOMIC_RELAXED));
+        if (bw != kNoFault && ((bw >> 3) / 2) / (uint64_t)K < cell)
+            break; // cells only grow along the list
+        const uint64_t w = cell_first_fault(A, B, (uint64_t)M, (uint64_t)N, (uint64_t)K, (int)TA,
+                                            (int)TB, cell, policy, true);
+        if (w != kNoFault && lane == 0)
+            atomicMin(&best, (unsigned long long)w);
+    }
+    __syncthreads();
+    if (tid == 0 && best != kNoFault) {
+        atomicMin(fault, best);
+        gate_record(gate);
+    }
+    program_close_block(close);
+}
+
+static inline bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
+
+template <typename T, bool TA, bool TB>
+static void small_launch(hipStream_t s, dim3 grid, const T *A, const T *B, T *C, int M, int N, int K,
+                         int thr, int risk, int policy, unsigned long long *fault, NodeGate gate,
+                         ProgramClose close)
+{
+    constexpr int P = 16 / (int)sizeof(T);
+    const bool va = !TA && K % P == 0 && aligned16(A), vb = TB && K % P == 0 && aligned16(B);
+    if ((TA || va) && (!TB || vb))
+        hipLaunchKernelGGL((k_strict_gemm_small<T, TA, TB, !TA, TB>), grid, dim3(256), 0, s, A, B, C, M, N, K, thr, risk, policy, fault, gate, close);
+    else
+        hipLaunchKernelGGL((k_strict_gemm_small<T, TA, TB, false, false>), grid, dim3(256), 0, s, A, B, C, M, N, K, thr, risk, policy, fault, gate, close);
+}
+
+template <typename T>
+static void small_layout(hipStream_t s, dim3 grid, bool ta, bool tb, const T *A, const T *B, T *C,
+                         int M, int N, int K, int thr, int risk, int policy,
+                         unsigned long long *fault, NodeGate gate, ProgramClose close)
+{
+    if (!ta && !tb)
+        small_launch<T, false, false>(s, grid, A, B, C, M, N, K, thr, risk, policy, fault, gate, close);
+    else if (!ta && tb)
+        small_launch<T, false, true>(s, grid, A, B, C, M, N, K, thr, risk, policy, fault, gate, close);
+    else if (ta && !tb)
+        small_launch<T, true, false>(s, grid, A, B, C, M, N, K, thr, risk, policy, fault, gate, close);
+    else
+        small_launch<T, true, true>(s, grid, A, B, C, M, N, K, thr, risk, policy, fault, gate, close);
+}
+
+// Estimated microseconds of this kernel and of the screened tile kernels, from measurements on
+// MI355X per 1024 k: up to two workgroups a CU run beside each other (binary32 12, 15; binary64
+// 22, 30), more take turns (6.1 and 13.2 each). The screened path adds a screen, a scan and a
+// replay launch (15 us). Binary64 tiles there take 205 us alone on their CU and 109 each when
+// several share it. Whole calls at the lines: binary32 256 x 1024 x 1024 (1024 workgroups) 27 us
+// against 20 + 15, 256 x 4096 x 1024 95 against 69 + 15.
+bool gemm_small_wanted(int dtype, uint64_t rows, uint64_t inner, uint64_t cols)
+{
+    const auto per_cu = [&](uint64_t tm, uint64_t tn) {
+        const uint64_t tiles = ((rows + tm - 1) / tm) * ((cols + tn - 1) / tn);
+        return (double)((tiles + kGfx950Cus - 1) / kGfx950Cus);
+    };
+    const double k = (double)inner / 1024.0, c = per_cu(16, 16);
+    if (dtype == 0)
+        return (c <= 2 ? 9 + 3 * c : 6.1 * c) * k + 3 < mid_time_f32(rows, cols, inner) + 15;
+    const double ct = per_cu(128, 64);
+    return (c <= 2 ? 14 + 8 * c : 13.2 * c) * k + 3 < (ct <= 1 ? 205 : 109 * ct) * k + 18;
+}
+
+hipError_t launch_gemm_small(hipStream_t s, int dtype, int M, int N, int K, bool ta, bool tb,
+                             const void *A, const void *B, void *C, int thr, int risk, int policy,
+                             unsigned long long *fault, NodeGate gate, ProgramClose close,
+                             bool *closed)
+{
+    const dim3 grid((unsigned)((((uint64_t)M + 15) / 16) * (((uint64_t)N + 15) / 16)));
+    if (grid.x > kCloseMaxBlocks)
+        close = ProgramClose{}; // the publication launch ends the program
+    if (closed)
+        *closed = close.words != nullptr;
+    if (dtype == 0)
+        small_layout<float>(s, grid, ta, tb, (const float *)A, (const float *)B, (float *)C, M, N, K, thr, risk, policy, fault, gate, close);
+    else
+        small_layout<double>(s, grid, ta, tb, (const double *)A, (const double *)B, (double *)C, M, N, K, thr, risk, policy, fault, gate, close);
+    return hipGetLastError();
+}
+
+} // namespace pcu

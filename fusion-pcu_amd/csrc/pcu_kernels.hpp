@@ -198,6 +198,7 @@ constexpr unsigned kGfx950Cus = 256; // compute units of a gfx950 device (MI350X
 // matmul_mid.hip. `whole`: M, N and K are multiples of the 128 x 128 tile and its slab.
 enum class MidTile { k32, k64, k128 };
 MidTile mid_tile_f32(uint64_t M, uint64_t N, uint64_t K, bool whole);
+double mid_time_f32(uint64_t M, uint64_t N, uint64_t K); // the chosen tile's estimate, in us
 // Whether matmul_mid.hip can address the operands.
 bool mid_fits_f32(uint64_t M, uint64_t N, uint64_t K, bool ta, bool tb);
 hipError_t launch_gemm_mid_f32(hipStream_t s, MidTile tile, int M, int N, int K, bool ta, bool tb,
@@ -205,6 +206,14 @@ hipError_t launch_gemm_mid_f32(hipStream_t s, MidTile tile, int M, int N, int K,
                                const unsigned long long *row_exp, const unsigned long long *col_exp,
                                int thr, int risk, unsigned long long *suspect, SumCheck sck,
                                NodeGate gate);
+
+// Strict MatMul of few cells in one launch (matmul_small.hip): screen, products, ordered sums
+// and the exact first-fault search. `wanted`: whether it is the faster route (inner > 0).
+bool gemm_small_wanted(int dtype, uint64_t rows, uint64_t inner, uint64_t cols);
+hipError_t launch_gemm_small(hipStream_t s, int dtype, int M, int N, int K, bool ta, bool tb,
+                             const void *A, const void *B, void *C, int thr, int risk, int policy,
+                             unsigned long long *fault, NodeGate gate, ProgramClose close,
+                             bool *closed);
 
 // C[rows x cols] = op(A) * op(B), k ascending, each multiply and add rounded on its own.
 // Every kernel of the op skips its work once `gate` shows that an earlier program node

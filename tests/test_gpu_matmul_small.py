@@ -1,0 +1,86 @@
+"""The one-launch strict MatMul of few cells at the sizes where it can go wrong: the edges of its
+16 x 16 blocks, of the chunks it stages (256 k for F32, 128 for F64), of the blocks it computes
+(64 and 32 k) and of the groups in them, rows that are and are not 16-byte aligned, in every
+layout, under every policy, with and without faults. Bit-exact against the oracle."""
+import numpy as np
+import pytest
+
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+DTYPES = pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+LAYOUTS = pytest.mark.parametrize("layout", [(False, False), (False, True), (True, False), (True, True)],
+                                  ids=["nn", "nt", "tn", "tt"])
+
+
+@pytest.fixture(scope="module")
+def ctx(pcu_pkg):
+    c = pcu_pkg.Context(0)
+    yield c
+    c.close()
+
+
+def _check(ctx, pcu_pkg, a, b, tl, tr, policy, offset=0):
+    """`offset`: elements between each operand's allocation and its first element."""
+    ref, rf = oracle.matmul(a, b, tl, tr, policy=policy)
+    held, args = [], []
+    for x in (a, b):
+        flat = ctx.upload(np.concatenate([np.zeros(offset, x.dtype), np.ascontiguousarray(x).reshape(-1)]))
+        held.append(flat)
+        args.append(pcu_pkg.DeviceArray(ctx, flat.ptr + offset * x.itemsize, x.shape, x.dtype))
+    try:
+        got = ctx.strict_matmul(args[0], args[1], tl, tr, policy).numpy()
+        fault = None
+    except pcu_pkg.PcuExecutionError as e:
+        f = e.tensor_fault
+        fault = (f.element_index, f.reduction_index, int(f.step), int(f.kind))
+    for h in held:
+        h.free()
+    want = None if rf is None else (rf.element_index, rf.reduction_index, rf.step, rf.kind)
+    assert fault == want, (a.shape, b.shape, tl, tr, policy, offset)
+    if want is None:
+        u = np.uint32 if a.dtype == np.float32 else np.uint64
+        np.testing.assert_array_equal(got.view(u), ref.view(u))
+
+
+def _operands(rng, m, k, n, tl, tr, dtype):
+    a = rng.uniform(-1, 1, (k, m) if tl else (m, k)).astype(dtype)
+    b = rng.uniform(-1, 1, (n, k) if tr else (k, n)).astype(dtype)
+    return a, b
+
+
+@DTYPES
+@LAYOUTS
+def test_block_chunk_and_group_edges(ctx, pcu_pkg, dtype, layout):
+    tl, tr = layout
+    rng = np.random.default_rng(5)
+    for m, n in ((1, 1), (16, 16), (17, 15), (33, 48)):
+        for k in (1, 2, 3, 4, 5, 31, 32, 33, 63, 64, 65, 127, 128, 129, 160, 255, 256, 257, 260, 511, 516):
+            a, b = _operands(rng, m, k, n, tl, tr, dtype)
+            _check(ctx, pcu_pkg, a, b, tl, tr, 0, offset=(m + k) % 3)
+
+
+@DTYPES
+@LAYOUTS
+@pytest.mark.parametrize("policy", [0, 1, 2])
+def test_first_fault_and_screen(ctx, pcu_pkg, dtype, layout, policy):
+    """Values that fault or are screened, at the first and last k, across chunks: not a number,
+    an infinity, an overflowing product, products that are tiny and inexact, exact subnormal
+    ones, and rows of zeros and subnormals whose exponents the block folds itself."""
+    tl, tr = layout
+    rng = np.random.default_rng(11 + policy)
+    info = np.finfo(dtype)
+    root = dtype(2.0 ** (info.minexp // 2))
+    for m, k, n in ((20, 70, 18), (16, 300, 33)):
+        for special in (np.nan, np.inf, info.max, root * dtype(0.7), root * dtype(0.5),
+                        info.smallest_subnormal, info.tiny * dtype(1.5), 0.0):
+            for kk in (0, k - 1):
+                a, b = _operands(rng, m, k, n, tl, tr, dtype)
+                av, bv = (a.T if tl else a), (b.T if tr else b)
+                av[m - 1, kk] = special
+                bv[kk, n - 1] = special if np.isfinite(special) else 1
+                _check(ctx, pcu_pkg, a, b, tl, tr, policy)
+                if special == info.smallest_subnormal:
+                    av[m - 1, :] = info.smallest_subnormal  # a whole row below the smallest normal
+                    _check(ctx, pcu_pkg, a, b, tl, tr, policy)
