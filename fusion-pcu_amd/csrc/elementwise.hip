@@ -12,6 +12,8 @@
 #include "pcu_device.hpp"
 #include "pcu_kernels.hpp"
 
+#include <utility>
+
 #include <limits.h>
 
 #pragma clang fp contract(off)
@@ -872,9 +874,9 @@ __device__ __forceinline__ double from_bits<double>(uint64_t b) { return __longl
 //                            of the summaries made for the running binade folds every chunk
 //                            before the first one that has no such summary or reaches the
 //                            binade's end. That chunk runs exactly: where crossings are
-//                            dense, one wave scans 64 squares at a time; elsewhere the
-//                            workgroup scans windows sized from the chunk's estimate. In
-//                            both, the first step to reach the binade's end runs as a real,
+//                            dense, one wave adds the squares one by one; elsewhere the
+//                            workgroup scans windows sized from the chunk's estimate, and
+//                            the first step of one to reach the binade's end runs as a real,
 //                            checked Add.
 // The estimate only decides how fast the walk goes, never its value.
 
@@ -990,6 +992,7 @@ template <typename T> struct WalkShared {
     uint64_t run_m;
     int run_status, run_ue;
     uint32_t run_resume;
+    typename SumBits<T>::U run_vals[SumBits<T>::kPer]; // the crossing run's squares
     uint64_t limit;
 };
 
@@ -1047,80 +1050,86 @@ __device__ __forceinline__ uint32_t window_per(double gap)
     return per;
 }
 
-// Below this expected gap (in squares) one wave walks, 64 squares per scan: a crossing
-// then costs one wave scan instead of a workgroup scan of a window. A wave walk stops at
-// the first binade whose expected gap reaches kWaveGap, or after kWaveMax squares (then a
-// window runs next, whatever the estimate says).
-constexpr double kWaveGap = 1024.0;
-constexpr uint32_t kWaveMax = 4096;
+// Below this expected gap (in squares) one wave folds the squares one by one with plain adds: a
+// window's scan and the walk of its crossing run cost about 3 us, the time of 750 such adds. The
+// fold stops at the first binade whose expected gap reaches kSerialGap, or after kSerialMax
+// squares (then a window runs next, whatever the estimate says).
+constexpr double kSerialGap = 1024.0;
+constexpr uint32_t kSerialMax = 4096;
 
-// The wave walk (wave 0 alone; every value it keeps is uniform over the wave): lane l
-// holds square off + l, a wave scan gives each lane the count before it, and the first
-// lane whose step reaches the binade's end executes that step as the contract's Add.
-// Returns false when that Add faulted (recorded).
+// f(0) .. f(15), each with its number as a constant.
+template <class F, int... J>
+__device__ __forceinline__ void each16(F &&f, std::integer_sequence<int, J...>)
+{
+    (f(std::integral_constant<int, J>{}), ...);
+}
+
+// The serial fold (wave 0 alone; every value it keeps is uniform over the wave). Each row of 16
+// lanes holds the same 16 squares and broadcasts one to its lanes per add (row_newbcast, no
+// instruction of its own for binary32), so a square costs the latency of one dependent add,
+// about 4 ns; a scan of 64 squares per wave with a step per crossing took 14 ns a square where
+// crossings are dense. The squares are finite and not negative, so a sum can only fault by
+// overflowing (the total turns, and stays, infinite) or, under RejectSubnormal, by being
+// subnormal: 64 squares are folded with plain adds and that check, and only 64 that trip it are
+// folded again with the exact add classifier. Returns false when an Add faulted (recorded).
 template <typename T>
-__device__ bool wave_walk(const typename SumBits<T>::U *vals, uint64_t base, uint32_t len,
-                          double mean, int policy, unsigned long long *fault,
-                          const NodeGate &gate, int lane, uint32_t &off, int &ue,
-                          typename SumBits<T>::C &m, typename SumBits<T>::C &mmax)
+__device__ bool serial_walk(const typename SumBits<T>::U *vals, uint64_t base, uint32_t len,
+                            double mean, int policy, unsigned long long *fault,
+                            const NodeGate &gate, int lane, uint32_t &off, int &ue,
+                            typename SumBits<T>::C &m, typename SumBits<T>::C &mmax)
 {
     using U = typename SumBits<T>::U;
-    using C = typename SumBits<T>::C;
-    const uint32_t end = off + kWaveMax < len ? off + kWaveMax : len;
+    const uint32_t end = off + kSerialMax < len ? off + kSerialMax : len;
+    const bool reject_sub = policy == kPolicyRejectSubnormal;
+    T total = from_bits<T>(sum_bits<T>(ue, m));
     while (off < end) {
-        const uint32_t i = off + (uint32_t)lane;
-        const bool in = i < end;
-        U b = 0;
-        C nn = 0;
-        uint32_t cls = kRBelow;
-        if (in) {
-            b = vals[ChunkLds<T>::slot(i)];
-            sum_elem<T>(b, ue, nn, cls);
+        const uint32_t here = end - off < 64 ? end - off : 64;
+        T v[4]; // squares past `here` read as +0, which changes no total
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+            const uint32_t i = 16 * b + (lane & 15);
+            v[b] = i < here ? from_bits<T>(vals[ChunkLds<T>::slot(off + i)]) : (T)0;
         }
-        const SumScan<T> inc = wave_scan_incl<T>(in ? scan_elem<T>(nn, cls) : scan_identity<T>());
-        SumScan<T> ex = scan_shfl_up<T>(inc, 1);
-        if (lane == 0)
-            ex = scan_identity<T>();
-        const uint32_t p0 = (uint32_t)(m & 1u);
-        const C mt = sat_add<T>(m, p0 ? ex.r1 : ex.r0);
-        const uint32_t pt = p0 ? (ex.p >> 1) & 1u : ex.p & 1u;
-        const C r = sum_step<C>(nn, cls, pt);
-        // Counts only grow along the lanes: at most one lane starts below the binade's end
-        // and reaches it.
-        const bool cross = in && mt < mmax && (cls == kRForce || mt + r >= mmax);
-        const uint64_t mask = __ballot(cross);
-        if (mask == 0) {
-            const SumScan<T> tot = scan_readlane<T>(inc, 63);
-            m = sat_add<T>(m, p0 ? tot.r1 : tot.r0);
-            off = off + 64 < end ? off + 64 : end;
-            continue;
+        T t = total;
+        bool sub = false;
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+            if (reject_sub)
+                each16([&](auto j) {
+                    t = t + row_lane<decltype(j)::value>(v[b]);
+                    sub |= subnormal(t);
+                }, std::make_integer_sequence<int, 16>{});
+            else
+                each16([&](auto j) { t = t + row_lane<decltype(j)::value>(v[b]); },
+                       std::make_integer_sequence<int, 16>{});
         }
-        const int c = __builtin_ctzll(mask);
-        U res_bits = 0;
-        uint32_t kind = kOk;
-        if (lane == c) {
-            const T acc = from_bits<T>(sum_bits<T>(ue, mt));
-            const T s_i = from_bits<T>(b);
-            const T res = acc + s_i;
-            kind = classify_add(acc, s_i, res, policy);
-            res_bits = (U)bits_of(res);
-            if (kind != kOk) {
-                atomicMin(fault, (unsigned long long)pack_fault(3 * (base + i) + 2, kind));
-                gate_record(gate);
+        if (!finite_bits(t) || sub) {
+            T acc = total;
+            for (uint32_t i = 0; i < here; i++) {
+                const T s_i = from_bits<T>(vals[ChunkLds<T>::slot(off + i)]);
+                const T nxt = acc + s_i;
+                const uint32_t kind = classify_add(acc, s_i, nxt, policy);
+                if (kind != kOk) {
+                    if (lane == 0) {
+                        atomicMin(fault, (unsigned long long)pack_fault(3 * (base + off + i) + 2, kind));
+                        gate_record(gate);
+                    }
+                    return false;
+                }
+                acc = nxt;
             }
         }
-        if (readlane_c(kind, c) != kOk)
-            return false;
-        sum_phase<T>(readlane_c(res_bits, c), ue, m, mmax);
-        off += (uint32_t)c + 1;
-        if (expected_gap((double)(mmax - m), ue, mean) >= kWaveGap)
+        total = t;
+        off += here;
+        sum_phase<T>((U)bits_of(total), ue, m, mmax);
+        if (expected_gap((double)(mmax - m), ue, mean) >= kSerialGap)
             break;
     }
     return true;
 }
 
 // Exact fold of elements [start, len) of the chunk at base from the phase (ue, m, mmax): by
-// the wave walk where crossings are dense, elsewhere window by window, where the one thread
+// the serial walk where crossings are dense, elsewhere window by window, where the one thread
 // whose run holds the window's first step to reach the binade's end executes that step as
 // the contract's Add and the next window starts after it in the new binade. Returns false
 // when an Add faulted (recorded).
@@ -1140,17 +1149,17 @@ __device__ bool exact_chunk(const typename SumBits<T>::U *__restrict__ src, uint
         sh.at[0] = sh.at[1] = kNoStep;
     __syncthreads();
     uint32_t off = start, per = 0; // per = 0: no window has run yet
-    bool wave_ok = true;
+    bool serial_ok = true;
     for (int it = 0; off < len; it++) {
         const int slot = it & 1;
         const double gap = expected_gap((double)(mmax - m), ue, mean);
-        if (wave_ok && gap < kWaveGap) {
+        if (serial_ok && gap < kSerialGap) {
             if (wave == 0) {
                 uint32_t o = off;
                 int u = ue;
                 C mm = m, mx = mmax;
-                const bool ok = wave_walk<T>(sh.vals, base, len, mean, policy, fault, gate, lane,
-                                             o, u, mm, mx);
+                const bool ok = serial_walk<T>(sh.vals, base, len, mean, policy, fault, gate, lane,
+                                               o, u, mm, mx);
                 if (lane == 0) {
                     sh.stop[slot] = !ok;
                     sh.total[slot] = sum_bits<T>(u, mm);
@@ -1166,7 +1175,7 @@ __device__ bool exact_chunk(const typename SumBits<T>::U *__restrict__ src, uint
             if (stop)
                 return false;
             sum_phase<T>(tot, ue, m, mmax);
-            wave_ok = next - off < kWaveMax;
+            serial_ok = next - off < kSerialMax;
             off = next;
             per = 0;
             continue;
@@ -1231,7 +1240,7 @@ __device__ bool exact_chunk(const typename SumBits<T>::U *__restrict__ src, uint
         sum_phase<T>(tot, ue, m, mmax);
         off = at + 1;
         per = 0;
-        wave_ok = true;
+        serial_ok = true;
     }
     return true;
 }
@@ -1285,8 +1294,35 @@ __device__ int run_prefix_chunk(const typename SumBits<T>::U *__restrict__ src,
         bool crossed = false;
         const uint32_t i0 = (uint32_t)tid * P, i1 = i0 + P < len ? i0 + P : len;
         uint32_t at = i1;
+        // The run's squares and the candidates' entries after it, in one round trip to memory
+        // ahead of the step loop, which then reads LDS.
+        U vals[P];
+        if (i0 + P <= len && ((uintptr_t)src & 15u) == 0) {
+#pragma unroll
+            for (uint32_t j = 0; j < P; j += 16 / sizeof(U)) {
+                const uint4 x = *reinterpret_cast<const uint4 *>(src + base + i0 + j);
+                const U *xs = reinterpret_cast<const U *>(&x);
+#pragma unroll
+                for (uint32_t e = 0; e < 16 / sizeof(U); e++)
+                    vals[j + e] = xs[e];
+            }
+        } else {
+#pragma unroll
+            for (uint32_t j = 0; j < P; j++)
+                vals[j] = i0 + j < len ? src[base + i0 + j] : (U)0;
+        }
+        ChunkSummary cs[kCands];
+        SumScan<T> ce[kCands];
+#pragma unroll
+        for (int y = 0; y < kCands; y++) {
+            cs[y] = summ_c[y];
+            ce[y] = tid + 1 < kSumThreads ? runs_c[(size_t)y * kSumThreads + tid + 1] : scan_identity<T>();
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < P; j++)
+            sh.run_vals[j] = vals[j];
         for (uint32_t i = i0; i < i1; i++) {
-            const U b = src[base + i];
+            const U b = sh.run_vals[i - i0];
             C nn;
             uint32_t cls;
             sum_elem<T>(b, u, nn, cls);
@@ -1318,20 +1354,22 @@ __device__ int run_prefix_chunk(const typename SumBits<T>::U *__restrict__ src,
         if (status == 1 && i1 < len) {
             // The runs after this one, from the prefixes of a candidate for the new binade.
             status = -1;
-            for (int y = 0; y < kCands; y++) {
-                if (summ_c[y].ue != u)
-                    continue;
-                const SumScan<T> Ey = runs_c[(size_t)y * kSumThreads + tid + 1];
-                const SumScan<T> Ty = scan_of_summary<T>(summ_c[y]);
-                const int q = (Ey.p & 1u) == pt ? 0 : (((Ey.p >> 1) & 1u) == pt ? 1 : -1);
-                if (q < 0)
-                    break;
+            int found = -1;
+            SumScan<T> Ey = scan_identity<T>(), Ty = scan_identity<T>();
+#pragma unroll
+            for (int y = kCands - 1; y >= 0; y--)
+                if (cs[y].ue == u) {
+                    found = y;
+                    Ey = ce[y];
+                    Ty = scan_of_summary<T>(cs[y]);
+                }
+            const int q = (Ey.p & 1u) == pt ? 0 : (((Ey.p >> 1) & 1u) == pt ? 1 : -1);
+            if (found >= 0 && q >= 0) {
                 const C tq = q ? Ty.r1 : Ty.r0, eq = q ? Ey.r1 : Ey.r0;
                 if (tq < SumBits<T>::kCap && mm + (tq - eq) < mx) {
                     mm += tq - eq;
                     status = 1;
                 }
-                break;
             }
         }
         sh.run_status = status;
@@ -1361,8 +1399,24 @@ __global__ __launch_bounds__(256) void k_mse_chunk_sums(const T *__restrict__ sq
     const uint64_t base = (uint64_t)blockIdx.x * sum_chunk_len<T>();
     const uint64_t end = base + sum_chunk_len<T>() < limit ? base + sum_chunk_len<T>() : limit;
     double acc = 0.0;
-    for (uint64_t i = base + threadIdx.x; i < end; i += 256)
-        acc += (double)sq[i];
+    if (end - base == sum_chunk_len<T>() && ((uintptr_t)sq & 15u) == 0) {
+        // A whole chunk: every 16-byte load of the thread in flight at once.
+        constexpr int P = 16 / sizeof(T), R = (int)(kSumThreads * SumBits<T>::kPer / (256 * P));
+        uint4 q[R];
+#pragma unroll
+        for (int j = 0; j < R; j++)
+            q[j] = *reinterpret_cast<const uint4 *>(sq + base + P * (256 * j + threadIdx.x));
+#pragma unroll
+        for (int j = 0; j < R; j++) {
+            const T *v = reinterpret_cast<const T *>(&q[j]);
+#pragma unroll
+            for (int e = 0; e < P; e++)
+                acc += (double)v[e];
+        }
+    } else {
+        for (uint64_t i = base + threadIdx.x; i < end; i += 256)
+            acc += (double)sq[i];
+    }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1)
         acc += __shfl_xor(acc, off, 64);
@@ -1484,26 +1538,45 @@ __global__ __launch_bounds__(kSumThreads) __attribute__((amdgpu_waves_per_eu(4))
     int ue;
     C m, mmax;
     sum_phase<T>((U)0, ue, m, mmax); // the total starts at +0
-    uint64_t c0 = 0;
-    for (int it = 0; c0 < chunks; it++) {
+    // Batches of 512 chunks: thread t keeps the candidates of chunk b0 + t in registers, read
+    // once a batch, and the batch is scanned again from the chunk after each stopping one.
+    int it = 0;
+    for (uint64_t b0 = 0; b0 < chunks; b0 += kSumThreads) {
+        const uint64_t c = b0 + tid;
+        int32_t cue[kCands];
+        SumScan<T> cscan[kCands];
+#pragma unroll
+        for (int y = 0; y < kCands; y++) {
+            cue[y] = kNoPhase;
+            cscan[y] = scan_identity<T>();
+            if (c < chunks) {
+                const ChunkSummary cs = summ[kCands * c + y];
+                cue[y] = cs.ue;
+                // Summary counts saturate at kCap, past any crossing: they fit C.
+                cscan[y] = scan_of_summary<T>(cs);
+            }
+        }
+        const uint64_t bend = b0 + kSumThreads < chunks ? b0 + kSumThreads : chunks;
+        for (uint64_t c0 = b0; c0 < bend; it++) {
         const int slot = it & 1;
-        const uint64_t c = c0 + tid;
         SumScan<T> mine = scan_identity<T>();
         int cand = -1;
-        if (c < chunks) {
+        if (c >= c0 && c < chunks) {
+            // No summary for this binade: stop here.
+            mine = SumScan<T>{kBig, kBig, 2u};
+#pragma unroll
             for (int y = kCands - 1; y >= 0; y--)
-                if (summ[kCands * c + y].ue == ue)
+                if (cue[y] == ue) {
                     cand = y;
-            // Summary counts saturate at kCap, past any crossing: they fit C. No summary for
-            // this binade: stop here.
-            mine = cand >= 0 ? scan_of_summary<T>(summ[kCands * c + cand]) : SumScan<T>{kBig, kBig, 2u};
+                    mine = cscan[y];
+                }
         }
         SumScan<T> before, total;
         block_scan<T>(mine, lane, wave, sh.wave_tot, before, total);
         const uint32_t p0 = (uint32_t)(m & 1u);
         const C mt = sat_add<T>(m, p0 ? before.r1 : before.r0);
         const uint32_t pt = p0 ? (before.p >> 1) & 1u : before.p & 1u;
-        if (c < chunks && mt < mmax && sat_add<T>(mt, pt ? mine.r1 : mine.r0) >= mmax) {
+        if (c >= c0 && c < chunks && mt < mmax && sat_add<T>(mt, pt ? mine.r1 : mine.r0) >= mmax) {
             sh.first[slot] = (uint32_t)tid;
             sh.m_first[slot] = (uint64_t)mt;
             sh.first_cand[slot] = cand;
@@ -1516,14 +1589,14 @@ __global__ __launch_bounds__(kSumThreads) __attribute__((amdgpu_waves_per_eu(4))
             sh.first[slot ^ 1] = kNoStep;
         if (first == kNoStep) {
             m = sat_add<T>(m, p0 ? total.r1 : total.r0);
-            c0 += kSumThreads;
+            c0 = bend;
             continue;
         }
         // Chunks before the stopping one fold; it runs exactly from the count before it:
         // from its run prefixes when it has a summary for this binade, and in windows from
         // wherever that leaves off.
         m = m_first;
-        const uint64_t cc = c0 + first;
+        const uint64_t cc = b0 + first;
         const uint64_t base = cc * L;
         const uint32_t len = (uint32_t)(base + L <= limit ? L : limit - base);
         uint32_t resume = 0;
@@ -1537,6 +1610,7 @@ __global__ __launch_bounds__(kSumThreads) __attribute__((amdgpu_waves_per_eu(4))
                                           fault, ue, m, mmax, sh, gate))
             return;
         c0 = cc + 1;
+        }
     }
     if (limit < n || tid != 0)
         return;

@@ -24,21 +24,6 @@
 
 namespace pcu {
 
-// Lane L's v, on every lane of L's row of 16 lanes.
-template <int L> __device__ __forceinline__ int row_lane(int v)
-{
-    return __builtin_amdgcn_update_dpp(0, v, 0x150 + L, 0xf, 0xf, true); // row_newbcast:L
-}
-template <int L> __device__ __forceinline__ float row_lane(float v)
-{
-    return __int_as_float(row_lane<L>(__float_as_int(v)));
-}
-template <int L> __device__ __forceinline__ double row_lane(double v)
-{
-    const int2 w = __builtin_bit_cast(int2, v);
-    return __builtin_bit_cast(double, make_int2(row_lane<L>(w.x), row_lane<L>(w.y)));
-}
-
 // Order keys of the screen: a smaller nonzero |v| has a smaller key, zero the largest, and a
 // non-finite value one above every finite one. Two instructions an element (binary64: on the
 // high word, with a nonzero low word of the tiniest subnormals standing as its last bit).

@@ -357,6 +357,21 @@ __device__ __forceinline__ uint32_t classify_relu_backward(T x, T up, T r, int p
     return kOk;
 }
 
+// Lane L's v, on every lane of L's row of 16 lanes.
+template <int L> __device__ __forceinline__ int row_lane(int v)
+{
+    return __builtin_amdgcn_update_dpp(0, v, 0x150 + L, 0xf, 0xf, true); // row_newbcast:L
+}
+template <int L> __device__ __forceinline__ float row_lane(float v)
+{
+    return __int_as_float(row_lane<L>(__float_as_int(v)));
+}
+template <int L> __device__ __forceinline__ double row_lane(double v)
+{
+    const int2 w = __builtin_bit_cast(int2, v);
+    return __builtin_bit_cast(double, make_int2(row_lane<L>(w.x), row_lane<L>(w.y)));
+}
+
 // ---------------------------------------------------------- wave reductions
 // Minimum of a 64-bit key over the wavefront (gfx950 waves are 64 lanes wide).
 __device__ __forceinline__ uint64_t wave_min_u64(uint64_t v)
