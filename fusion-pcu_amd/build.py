@@ -37,7 +37,8 @@ COMMON = [
     f"-I{CSRC}",
 ]
 
-SOURCES = ["elementwise.hip", "matmul.hip", "matmul_mfma.hip", "matmul_mid.hip", "matmul_small.hip", "runtime.cpp", "graph.cpp"]
+SOURCES = ["elementwise.hip", "matmul.hip", "matmul_mfma.hip", "matmul_mid.hip", "matmul_small.hip",
+           "matmul_native.hip", "matmul_valu.hip", "runtime.cpp", "graph.cpp"]
 
 
 def _compile(src: str) -> str:

@@ -12,6 +12,34 @@
 
 namespace pcu {
 
+// Direct global -> LDS load of W words a lane: lane l's words land at lds + 4 W l bytes. base
+// and lds are uniform across the wave; base stays in scalar registers (the scalar unit advances
+// it), which the compiler's form of this load does not do. Issued from inline assembly, so the
+// compiler does not track it: the caller waits for it before the barrier that publishes the
+// stage.
+template <int W> __device__ __forceinline__ void load_lds(const void *base, uint32_t off, uint32_t lds)
+{
+    static_assert(W == 1 || W == 4, "words a lane");
+    if constexpr (W == 4)
+        asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base)
+                     : "memory", "m0");
+    else
+        asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(off), "s"(base)
+                     : "memory", "m0");
+}
+// The LDS byte address of p.
+__device__ __forceinline__ uint32_t lds_address(const void *p)
+{
+    return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void *)p;
+}
+__device__ __forceinline__ void wait_lds_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+// Wait until at most N of this wave's vector memory loads are outstanding: loads complete in
+// the order they were issued, so every load before the last N has landed.
+template <int N> __device__ __forceinline__ void wait_loads_but()
+{
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
 // E consecutive elements of a row-major operand at p; `valid` of them in bounds.
 template <typename T, int E, bool VEC>
 __device__ __forceinline__ void load_run(const T *__restrict__ p, int valid, T (&v)[E])
@@ -90,6 +118,22 @@ __device__ __forceinline__ void tile_of(int bid, int tiles_m, int tiles_n, int &
     tm = first_m + (L % per_group) % gsize;
     tn = (L % per_group) / gsize;
 }
+
+// Workgroup shape: WM x WN waves, each owning SM x SN output subtiles of 32 x 32; k-slabs
+// of BK are staged through k-major LDS tiles (two or three stages).
+template <int WM_, int WN_, int SM_, int SN_, int BK_, int WAVES_PER_SIMD_> struct MfmaCfg {
+    static constexpr int WM = WM_, WN = WN_, SM = SM_, SN = SN_, BK = BK_;
+    static constexpr int kWavesPerSimd = WAVES_PER_SIMD_; // occupancy the registers allow
+    static constexpr int BM = WM * SM * 32, BN = WN * SN * 32;
+    static constexpr int kThreads = 64 * WM * WN;
+    static constexpr int LDA = BM + 4, LDB = BN + 4; // row pitch of the k-major LDS tiles
+    static constexpr int EA = BM * BK / kThreads;    // A elements one thread stages per slab
+    static constexpr int EB = BN * BK / kThreads;
+    static_assert(EA % 4 == 0 && EB % 4 == 0, "staging moves whole float4s");
+    // A thread staging several float4s of a B k-row takes them BN / (EB / 4) apart (measured
+    // 1.5-2.5% faster for the native kernel's 16 elements than one contiguous run).
+    template <bool TA> static constexpr bool kSplitRunsB = EB > 4;
+};
 
 // Cfg provides BM, BN, BK, kThreads, EA, EB, LDA, LDB and kSplitRunsB<TA>.
 template <typename T, class Cfg, bool TA, bool TB, bool VA, bool VB> struct SlabStager {

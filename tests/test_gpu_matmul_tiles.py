@@ -76,3 +76,25 @@ def test_tiles_first_fault_and_partial_sums(ctx, pcu_pkg, m, k, n, policy, layou
             av[m - 1, k - 1] = special
             bv[k - 1, n - 1] = special
         _check(ctx, pcu_pkg, a, b, tl, tr, policy)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("m,n", [(33, 65), (200, 130), (900, 1030)])
+@pytest.mark.parametrize("layout", [(False, False), (False, True), (True, False), (True, True)])
+def test_native_tile_edges(ctx, dtype, m, n, layout):
+    """Each native product within gamma_k (|A| |B|), gamma_k = k u / (1 - k u), of the exact one,
+    whatever the order of its sum."""
+    tl, tr = layout
+    rng = np.random.default_rng(m)
+    u = np.finfo(dtype).eps / 2
+    for k in (1, 3, 16, 31, 32, 33, 64, 100, 161):
+        a = rng.uniform(-1, 1, (k, m) if tl else (m, k)).astype(dtype)
+        b = rng.uniform(-1, 1, (n, k) if tr else (k, n)).astype(dtype)
+        got = ctx.native_matmul(ctx.upload(a), ctx.upload(b), tl, tr)
+        ctx.synchronize()
+        la, lb = (a.T if tl else a).astype(np.longdouble), (b.T if tr else b).astype(np.longdouble)
+        la, lb = (la, lb) if dtype == np.float64 and m < 300 else (la.astype(np.float64), lb.astype(np.float64))
+        exact, size = la @ lb, abs(la) @ abs(lb)
+        # The reference's own sum is rounded too where it is in binary64.
+        slack = (k * u / (1 - k * u) + k * 2.0 ** -52) * size
+        assert np.all(abs(got.numpy() - exact) <= slack), (k, m, n, tl, tr)
