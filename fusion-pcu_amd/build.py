@@ -38,7 +38,7 @@ COMMON = [
 ]
 
 SOURCES = ["elementwise.hip", "matmul.hip", "matmul_mfma.hip", "matmul_mid.hip", "matmul_small.hip",
-           "matmul_native.hip", "matmul_valu.hip", "runtime.cpp", "graph.cpp"]
+           "matmul_native.hip", "matmul_valu.hip", "matmul_f64.hip", "runtime.cpp", "graph.cpp"]
 
 
 def _compile(src: str) -> str:

@@ -969,7 +969,8 @@ bool matmul_bt_wanted(int dtype, uint64_t rows, uint64_t inner, uint64_t cols, b
     // against 54.6 us).
     return rows % 128 == 0 && cols % 128 == 0 && (rows / 128) * (cols / 128) >= 256 &&
            inner * cols <= kBtMaxElems &&
-           (dtype != 0 || mid_tile_f32(rows, cols, inner, true) == MidTile::k128);
+           (dtype == 0 ? mid_tile_f32(rows, cols, inner, true) == MidTile::k128
+                       : !mid_wanted_f64(rows, cols, inner, tl, tr, false));
 }
 
 // The exponent screen of op(A) rows and op(B) columns, both jobs in one launch.
@@ -1020,8 +1021,8 @@ static hipError_t strict_matmul_t(hipStream_t s, uint64_t M, uint64_t K, uint64_
     const bool reject = policy == kPolicyRejectSubnormal;
     int risk = policy != kPolicyAllowGradual;
     // Under RejectSubnormal the tile kernels check the partial sums of every tile that may
-    // meet a product below 2^sub_thr (all but the narrow binary64 tile, when the scratch has
-    // the block words); a cell is then suspect only for a non-finite result, a possibly tiny
+    // meet a product below 2^sub_thr (binary64: on grids of at least 256 tiles of 128 x 128; when
+    // the scratch has the block words); a cell is then suspect only for a non-finite result, a possibly tiny
     // product or a subnormal partial sum in its lane. Without the check every cell the
     // exponents put below sub_thr is suspect and walked in full.
     const uint64_t tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
@@ -1098,9 +1099,10 @@ static hipError_t strict_matmul_t(hipStream_t s, uint64_t M, uint64_t K, uint64_
         }
         (void)launch_gemm_mfma_f32(s, m, n, k, ta, tbt, (const float *)A, Bt, (float *)C,
                                    sc.row_exp, sc.col_exp, thr, risk, sc.suspect, sck, gate, epi, epi_done);
-    } else if (!f32 && (uint64_t)grid.x < 256) {
-        (void)launch_gemm_f64_small_grid(s, m, n, k, ta, tb, (const double *)A, (const double *)B,
-                                         (double *)C, sc.row_exp, sc.col_exp, thr, risk, sc.suspect, gate);
+    } else if (!f32 && sck.flag == nullptr && mid_wanted_f64(M, N, K, ta, tb, false)) {
+        // (The 64 x 64 tiles have no partial-sum check.)
+        (void)launch_gemm_mid_f64(s, false, m, n, k, ta, tb, (const double *)A, (const double *)B,
+                                  (double *)C, sc.row_exp, sc.col_exp, thr, risk, sc.suspect, gate);
     } else {
         // A transposed binary64 op(B) on a full grid goes to the tile kernel as its K x N
         // copy, as for the matrix-core engine above.

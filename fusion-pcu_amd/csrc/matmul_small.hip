@@ -322,20 +322,20 @@ static void small_layout(hipStream_t s, dim3 grid, bool ta, bool tb, const T *A,
 // Estimated microseconds of this kernel and of the screened tile kernels, from measurements on
 // MI355X per 1024 k: up to two workgroups a CU run beside each other (binary32 12, 15; binary64
 // 22, 30), more take turns (6.1 and 13.2 each). The screened path adds a screen, a scan and a
-// replay launch (15 us). Binary64 tiles there take 205 us alone on their CU and 109 each when
-// several share it. Whole calls at the lines: binary32 256 x 1024 x 1024 (1024 workgroups) 27 us
-// against 20 + 15, 256 x 4096 x 1024 95 against 69 + 15.
+// replay launch (15 us). Its binary64 tiles: see mid_wanted_f64. Kernels at the lines: binary32
+// 256 x 1024 x 1024 (1024 workgroups) 27 us against 20 + 15, 256 x 4096 x 1024 95 against
+// 69 + 15; binary64 512 x 1024 x 512 53 against 88 + 15.
 bool gemm_small_wanted(int dtype, uint64_t rows, uint64_t inner, uint64_t cols)
 {
-    const auto per_cu = [&](uint64_t tm, uint64_t tn) {
-        const uint64_t tiles = ((rows + tm - 1) / tm) * ((cols + tn - 1) / tn);
+    const auto per_cu = [&](uint64_t t) {
+        const uint64_t tiles = ((rows + t - 1) / t) * ((cols + t - 1) / t);
         return (double)((tiles + kGfx950Cus - 1) / kGfx950Cus);
     };
-    const double k = (double)inner / 1024.0, c = per_cu(16, 16);
+    const double k = (double)inner / 1024.0, c = per_cu(16);
     if (dtype == 0)
         return (c <= 2 ? 9 + 3 * c : 6.1 * c) * k + 3 < mid_time_f32(rows, cols, inner) + 15;
-    const double ct = per_cu(128, 64);
-    return (c <= 2 ? 14 + 8 * c : 13.2 * c) * k + 3 < (ct <= 1 ? 205 : 109 * ct) * k + 18;
+    const double c64 = per_cu(64);
+    return (c <= 2 ? 14 + 8 * c : 13.2 * c) * k + 3 < (c64 <= 2 ? 26 + 65 * c64 : 74 * c64) * k + 18;
 }
 
 hipError_t launch_gemm_small(hipStream_t s, int dtype, int M, int N, int K, bool ta, bool tb,

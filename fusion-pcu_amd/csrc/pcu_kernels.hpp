@@ -207,18 +207,19 @@ hipError_t launch_gemm_mid_f32(hipStream_t s, MidTile tile, int M, int N, int K,
                                int thr, int risk, unsigned long long *suspect, SumCheck sck,
                                NodeGate gate);
 
-// The vector-unit engine's 128 x 128 tiles (matmul_valu.hip), and the strict F64 tiles for fewer
-// of those than CUs.
+// The vector-unit engine's 128 x 128 tiles (matmul_valu.hip).
 hipError_t launch_gemm_valu(hipStream_t s, int dtype, int M, int N, int K, bool ta, bool tb,
                             const void *A, const void *B, void *C,
                             const unsigned long long *row_exp, const unsigned long long *col_exp,
                             int thr, int risk, unsigned long long *suspect, SumCheck sck,
                             NodeGate gate);
-hipError_t launch_gemm_f64_small_grid(hipStream_t s, int M, int N, int K, bool ta, bool tb,
-                                      const double *A, const double *B, double *C,
-                                      const unsigned long long *row_exp,
-                                      const unsigned long long *col_exp, int thr, int risk,
-                                      unsigned long long *suspect, NodeGate gate);
+// F64 on 64 x 64 tiles (matmul_f64.hip), strict or native, and whether those are the faster ones.
+bool mid_wanted_f64(uint64_t M, uint64_t N, uint64_t K, bool ta, bool tb, bool native);
+hipError_t launch_gemm_mid_f64(hipStream_t s, bool native, int M, int N, int K, bool ta, bool tb,
+                               const double *A, const double *B, double *C,
+                               const unsigned long long *row_exp, const unsigned long long *col_exp,
+                               int thr, int risk, unsigned long long *suspect, NodeGate gate);
+
 // Strict MatMul of few cells in one launch (matmul_small.hip): screen, products, ordered sums
 // and the exact first-fault search. `wanted`: whether it is the faster route (inner > 0).
 bool gemm_small_wanted(int dtype, uint64_t rows, uint64_t inner, uint64_t cols);

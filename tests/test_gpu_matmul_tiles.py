@@ -78,6 +78,21 @@ def test_tiles_first_fault_and_partial_sums(ctx, pcu_pkg, m, k, n, policy, layou
         _check(ctx, pcu_pkg, a, b, tl, tr, policy)
 
 
+# F64: 64 x 64 tiles of its own, slabs of 16 k.
+@pytest.mark.parametrize("m,n", [(63, 1025), (64, 1024), (65, 1026), (513, 515)])
+@pytest.mark.parametrize("layout", [(False, False), (False, True), (True, False), (True, True)])
+def test_f64_tile_edges_and_slab_remainders(ctx, m, n, layout):
+    tl, tr = layout
+    rng = np.random.default_rng(m + n)
+    for k in (1, 2, 15, 16, 17, 32, 47, 48, 50, 64, 65, 98):
+        a = rng.uniform(-1, 1, (k, m) if tl else (m, k))
+        b = rng.uniform(-1, 1, (n, k) if tr else (k, n))
+        got = ctx.strict_matmul(ctx.upload(a), ctx.upload(b), tl, tr).numpy()
+        ref, fault = oracle.matmul(a, b, tl, tr)
+        assert fault is None
+        np.testing.assert_array_equal(got.view(np.uint64), ref.view(np.uint64))
+
+
 @pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
 @pytest.mark.parametrize("m,n", [(33, 65), (200, 130), (900, 1030)])
 @pytest.mark.parametrize("layout", [(False, False), (False, True), (True, False), (True, True)])
