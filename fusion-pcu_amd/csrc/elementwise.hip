@@ -12,8 +12,6 @@
 #include "pcu_device.hpp"
 #include "pcu_kernels.hpp"
 
-#include <utility>
-
 #include <limits.h>
 
 #pragma clang fp contract(off)
@@ -601,60 +599,16 @@ __global__ __launch_bounds__(kEwThreads) void k_sgd_pair(SgdPairArgs<T> a, int p
 // (ordinal 3n). The sum is a dependent chain by contract; it stops before the first
 // element whose Subtract or Multiply faulted.
 
-template <typename T, bool VEC>
-__global__ __launch_bounds__(kEwThreads) void k_mse_squares(const T *__restrict__ p,
-                                                            const T *__restrict__ t,
-                                                            T *__restrict__ sq, uint64_t n,
-                                                            int policy,
-                                                            unsigned long long *fault, NodeGate gate)
-{
-    if (wave_gate_closed(gate))
-        return;
-    constexpr int W = Lanes<T, VEC>::W;
-    uint64_t key = kNoFault;
-    PCU_EW_LOOP(W)
-    {
-        T pv[W], tv[W], d[W], sv[W];
-        load_lanes<T, VEC>(p, base, n, pv);
-        load_lanes<T, VEC>(t, base, n, tv);
-        bool any = false;
-#pragma unroll
-        for (int j = 0; j < W; j++) {
-            d[j] = pv[j] - tv[j];
-            sv[j] = d[j] * d[j];
-            any |= base + j < n && (add_suspect(pv[j], tv[j], d[j], policy) |
-                                    mul_suspect(d[j], d[j], sv[j], policy));
-        }
-        // Ordinary stores: the ordered sum reads the squares next.
-        store_lanes<T, VEC, false>(sq, base, n, sv);
-        if (any && key == kNoFault) {
-#pragma unroll
-            for (int j = 0; j < W; j++) {
-                if (base + j >= n || key != kNoFault)
-                    continue;
-                const uint32_t ks = classify_add(pv[j], tv[j], d[j], policy);
-                if (ks != kOk) {
-                    key = pack_fault(3 * (base + j), ks);
-                } else {
-                    const uint32_t km = classify_mul(d[j], d[j], sv[j], policy);
-                    if (km != kOk)
-                        key = pack_fault(3 * (base + j) + 1, km);
-                }
-            }
-        }
-    }
-    wave_record_fault(key, fault, gate);
-}
-
 // Ordered sum of the squares, exact and parallel. Every square is +0 or positive, so the
 // running total never decreases. While the total stays inside one binade [2^E, 2^(E+1))
 // (or below the smallest normal), it is m * u for an integer m and the binade's quantum u,
 // and one rounded step total (+) s equals (m + r) * u where r is s/u rounded to the nearest
 // integer, a tie going to the r that makes m + r even. So inside a binade the chain is a
 // prefix sum of integers whose only coupling is the parity of m at each tie: a two-state
-// automaton, which composes associatively and scans in parallel. The first element whose
-// step would reach the binade's upper end (or any element a screen cannot place) is
-// executed as the real rounded hardware add, checked like every other Add, and starts the
+// automaton, which composes associatively and scans in parallel. What a run of squares adds from
+// an even and from an odd m is read off two chains of plain adds, from the binade's first two
+// values. The run holding the first element whose step would reach the binade's upper end is
+// executed as real rounded hardware adds, checked like every other Add, and its total starts the
 // next phase. Results equal the dependent chain of the contract bit for bit.
 
 template <typename T> struct SumBits;
@@ -665,7 +619,7 @@ template <> struct SumBits<float> {
     static constexpr int kQmin = -149;   // exponent of the smallest subnormal
     static constexpr uint32_t kExpAll = 0xff;
     static constexpr int kPer = 16;      // elements per thread of a full-chunk scan
-    static constexpr C kBig = 1u << 25;  // r of a step that surely leaves the binade
+    static constexpr C kBig = 1u << 25;  // count of a run that surely leaves the binade
     static constexpr C kCap = 1u << 30;  // saturation of prefix counts (past any crossing)
 };
 template <> struct SumBits<double> {
@@ -679,9 +633,9 @@ template <> struct SumBits<double> {
     static constexpr C kCap = 1ull << 62;
 };
 
+// Threads of a chunk's scan; a chunk is kPer elements for each.
 constexpr int kSumThreads = 512;
-
-enum : uint32_t { kRBelow = 0, kRAbove = 1, kRTie = 2, kRForce = 3 };
+constexpr int kQuarters = 4; // parts of a chunk that the squares kernel sums on their own
 
 template <typename T>
 __device__ __forceinline__ typename SumBits<T>::C sat_add(typename SumBits<T>::C a,
@@ -689,50 +643,6 @@ __device__ __forceinline__ typename SumBits<T>::C sat_add(typename SumBits<T>::C
 {
     const typename SumBits<T>::C c = a + b; // a, b <= kCap: no wrap
     return c < SumBits<T>::kCap ? c : SumBits<T>::kCap;
-}
-
-// Step r of one square s (bits) on the quantum 2^ue, before the tie decision.
-template <typename T>
-__device__ __forceinline__ void sum_elem(typename SumBits<T>::U b, int ue,
-                                         typename SumBits<T>::C &n, uint32_t &cls)
-{
-    using B = SumBits<T>;
-    using U = typename B::U;
-    using C = typename B::C;
-    const uint32_t e = (uint32_t)(b >> B::kFrac) & B::kExpAll;
-    const C f = (C)(b & (((U)1 << B::kFrac) - 1));
-    if ((b >> (sizeof(U) * 8 - 1)) || e == B::kExpAll) { // negative or non-finite
-        n = B::kBig;
-        cls = kRForce;
-        return;
-    }
-    const C sig = e ? (f | ((C)1 << B::kFrac)) : f;
-    const int q = e ? (int)e + B::kQmin - 1 : B::kQmin;
-    cls = kRBelow;
-    if (sig == 0) {
-        n = 0;
-        return;
-    }
-    const int sh = q - ue;
-    if (sh >= 0) {
-        // sh > 0 only for normal squares (sig >= 2^kFrac): from sh = 2 on, r >= kBig.
-        n = sh >= 2 ? B::kBig : (sig << sh);
-        return;
-    }
-    const int k = -sh;
-    if (k > B::kFrac + 1) { // sig < 2^(kFrac+1) <= half a quantum: rounds to 0
-        n = 0;
-        return;
-    }
-    n = sig >> k;
-    const C rem = sig & (((C)1 << k) - 1), half = (C)1 << (k - 1);
-    cls = rem < half ? kRBelow : (rem > half ? kRAbove : kRTie);
-}
-
-template <typename C>
-__device__ __forceinline__ C sum_step(C n, uint32_t cls, uint32_t parity)
-{
-    return n + (C)(cls == kRAbove) + (C)(cls == kRTie && ((parity ^ (uint32_t)n) & 1u));
 }
 
 // Effect of a run of steps as a function of the parity of m before it: the added count
@@ -755,14 +665,6 @@ __device__ __forceinline__ SumScan<T> scan_compose(const SumScan<T> &a, const Su
     c.r1 = sat_add<T>(a.r1, a1 ? b.r1 : b.r0);
     c.p = (a0 ? b1 : b0) | ((a1 ? b1 : b0) << 1);
     return c;
-}
-
-template <typename T>
-__device__ __forceinline__ SumScan<T> scan_elem(typename SumBits<T>::C n, uint32_t cls)
-{
-    using C = typename SumBits<T>::C;
-    const C r0 = sum_step<C>(n, cls, 0), r1 = sum_step<C>(n, cls, 1);
-    return SumScan<T>{r0, r1, (uint32_t)(r0 & 1u) | ((uint32_t)((r1 + 1) & 1u) << 1)};
 }
 
 // Cross-lane moves of a summary. DPP (a register read across lanes, no LDS): a lane
@@ -862,22 +764,58 @@ __device__ __forceinline__ float from_bits<float>(uint32_t b) { return __uint_as
 template <>
 __device__ __forceinline__ double from_bits<double>(uint64_t b) { return __longlong_as_double((long long)b); }
 
+// Whether 2^ue is the quantum of some binade.
+template <typename T> __device__ __forceinline__ bool phase_valid(int ue)
+{
+    return ue >= SumBits<T>::kQmin && ue - SumBits<T>::kQmin + 1 < (int)SumBits<T>::kExpAll;
+}
+
+// Effect of the squares v (+0: none) on the quantum 2^ue. The count a run adds depends on the
+// count before it only through its parity, so it is what two chains of rounded adds gain that
+// start at the binade's first value and at the one after it: inside a binade the bits are the
+// count (the subnormals share the quantum of the first normal binade, whose values stand in for
+// them). A chain that leaves the binade has added more than any total in it can take. Two adds a
+// square against some 40 instructions of integer steps: the summaries of 4096 x 1024 f32 squares
+// took 15.9 us with those, 7.3 so.
+template <typename T, int N>
+__device__ __forceinline__ SumScan<T> run_summary(const T (&v)[N], int ue)
+{
+    using B = SumBits<T>;
+    using U = typename B::U;
+    const U even = (U)(ue - B::kQmin + 1) << B::kFrac, odd = even + 1, end = even + ((U)1 << B::kFrac);
+    T t0 = from_bits<T>(even), t1 = from_bits<T>(odd);
+#pragma unroll
+    for (int j = 0; j < N; j++) {
+        t0 = t0 + v[j];
+        t1 = t1 + v[j];
+    }
+    const U b0 = (U)bits_of(t0), b1 = (U)bits_of(t1);
+    SumScan<T> s;
+    s.r0 = b0 < end ? b0 - even : B::kBig; // NaN and infinities lie past the end
+    s.r1 = b1 < end ? b1 - odd : B::kBig;
+    s.p = (uint32_t)(s.r0 & 1u) | ((uint32_t)((s.r1 + 1) & 1u) << 1);
+    return s;
+}
+
 // ----------------------------------------------------- ordered sum: pipeline
 // The squares are cut into chunks of 512*P elements (P = 16 for binary32, 8 for binary64).
-//  A  k_mse_chunk_sums       per-chunk sum in binary64 (an estimate: order does not matter);
-//  B  k_mse_chunk_prefix     the exclusive prefix of those sums: about where the running
-//                            total stands at each chunk start;
+//  A  k_mse_squares          the squares, and each quarter chunk's sum in binary64 (an
+//                            estimate: order does not matter);
+//  B  k_mse_chunk_prefix     the chunks' sums and their exclusive prefix: about where the
+//                            running total stands at each chunk start;
 //  C  k_mse_chunk_summaries  per chunk, in parallel, the summary (count added for an even
 //                            and an odd start) of the whole chunk inside one binade, for
 //                            the one or two binades the estimate allows;
 //  D  k_mse_ordered_walk     one workgroup walks the chunks in order, 512 at a time: a scan
 //                            of the summaries made for the running binade folds every chunk
 //                            before the first one that has no such summary or reaches the
-//                            binade's end. That chunk runs exactly: where crossings are
-//                            dense, one wave adds the squares one by one; elsewhere the
-//                            workgroup scans windows sized from the chunk's estimate, and
-//                            the first step of one to reach the binade's end runs as a real,
-//                            checked Add.
+//                            binade's end. That chunk runs exactly: the run of 16 (8)
+//                            squares holding the crossing is added square by square, checked
+//                            like every other Add, and the runs after it fold from the
+//                            prefixes made for the next binade; where several crossings
+//                            share a chunk, one wave adds the squares one by one while they
+//                            are dense, and elsewhere the workgroup scans windows sized from
+//                            the chunk's estimate.
 // The estimate only decides how fast the walk goes, never its value.
 
 struct ChunkSummary {
@@ -983,16 +921,16 @@ template <typename T> struct WalkShared {
     SumScan<T> wave_tot[kSumThreads / 64];
     uint64_t m_first[2];             // count standing before the stopping chunk
     uint32_t first[2];               // stopping chunk of a batch (offset), kNoStep: none
-    uint32_t at[2];                  // crossing element of a window, or the element after a
-                                     // wave walk (offset); kNoStep: no crossing
-    typename SumBits<T>::U total[2]; // total after the crossing Add or the wave walk
+    uint32_t at[2];                  // element after a window's crossing run, or after a
+                                     // serial walk (offset); kNoStep: no crossing
+    typename SumBits<T>::U total[2]; // total before that element
     int stop[2];                     // an Add faulted
     int first_cand[2];               // candidate summary the stopping chunk matched, or -1
+    double mean[2];                  // the stopping chunk's mean square (an estimate)
     // Result of a chunk's run-prefix fold (written by the one thread holding the crossing).
     uint64_t run_m;
     int run_status, run_ue;
     uint32_t run_resume;
-    typename SumBits<T>::U run_vals[SumBits<T>::kPer]; // the crossing run's squares
     uint64_t limit;
 };
 
@@ -1001,17 +939,11 @@ template <typename T, int PER>
 __device__ __forceinline__ SumScan<T> run_scan(const typename SumBits<T>::U *vals, uint32_t i0,
                                                uint32_t i1, int ue)
 {
-    SumScan<T> s = scan_identity<T>();
+    T v[PER];
 #pragma unroll
-    for (int j = 0; j < PER; j++) {
-        if (i0 + j < i1) {
-            typename SumBits<T>::C nn;
-            uint32_t cls;
-            sum_elem<T>(vals[ChunkLds<T>::slot(i0 + j)], ue, nn, cls);
-            s = scan_compose<T>(s, scan_elem<T>(nn, cls));
-        }
-    }
-    return s;
+    for (int j = 0; j < PER; j++)
+        v[j] = i0 + j < i1 ? from_bits<T>(vals[ChunkLds<T>::slot(i0 + j)]) : (T)0;
+    return run_summary<T, PER>(v, ue);
 }
 
 template <typename T>
@@ -1051,27 +983,92 @@ __device__ __forceinline__ uint32_t window_per(double gap)
 }
 
 // Below this expected gap (in squares) one wave folds the squares one by one with plain adds: a
-// window's scan and the walk of its crossing run cost about 3 us, the time of 750 such adds. The
-// fold stops at the first binade whose expected gap reaches kSerialGap, or after kSerialMax
-// squares (then a window runs next, whatever the estimate says).
-constexpr double kSerialGap = 1024.0;
+// window costs 2.2 to 2.9 us, the time of about 500 such adds. The fold stops at the first binade whose
+// expected gap reaches kSerialGap, or after kSerialMax squares (then a window runs next, whatever
+// the estimate says).
+constexpr double kSerialGap = 512.0;
 constexpr uint32_t kSerialMax = 4096;
 
-// f(0) .. f(15), each with its number as a constant.
-template <class F, int... J>
-__device__ __forceinline__ void each16(F &&f, std::integer_sequence<int, J...>)
+// `count` squares from global element `at` on, given by read(0 .. count - 1), added to `total` one
+// by one with the exact add classifier: false when an Add faulted (recorded).
+template <typename T, class F>
+__device__ __forceinline__ bool fold_exact(T total, uint32_t count, uint64_t at, int policy,
+                                                     unsigned long long *fault, const NodeGate &gate,
+                                                     F read)
 {
-    (f(std::integral_constant<int, J>{}), ...);
+    for (uint32_t i = 0; i < count; i++) {
+        const T s_i = read(i);
+        const T nxt = total + s_i;
+        const uint32_t kind = classify_add(total, s_i, nxt, policy);
+        if (kind != kOk) {
+            atomicMin(fault, (unsigned long long)pack_fault(3 * (at + i) + 2, kind));
+            gate_record(gate);
+            return false;
+        }
+        total = nxt;
+    }
+    return true;
 }
 
-// The serial fold (wave 0 alone; every value it keeps is uniform over the wave). Each row of 16
-// lanes holds the same 16 squares and broadcasts one to its lanes per add (row_newbcast, no
-// instruction of its own for binary32), so a square costs the latency of one dependent add,
-// about 4 ns; a scan of 64 squares per wave with a step per crossing took 14 ns a square where
-// crossings are dense. The squares are finite and not negative, so a sum can only fault by
-// overflowing (the total turns, and stays, infinite) or, under RejectSubnormal, by being
-// subnormal: 64 squares are folded with plain adds and that check, and only 64 that trip it are
-// folded again with the exact add classifier. Returns false when an Add faulted (recorded).
+// One thread's run of squares (those past its end +0, which change no total) added to `total`.
+// The squares are finite and not negative, so a sum can only fault by overflowing (the total
+// turns, and stays, infinite) or, under RejectSubnormal, by being subnormal: plain adds and that
+// check, and only a run that trips it goes through the exact classifier. Returns false when an
+// Add faulted (recorded).
+template <typename T, class F>
+__device__ __forceinline__ bool fold_run(const T (&v)[SumBits<T>::kPer], T &total, uint32_t count,
+                                         uint64_t at, int policy, unsigned long long *fault,
+                                         const NodeGate &gate, F read)
+{
+    T t = total;
+    bool sub = false;
+#pragma unroll
+    for (int j = 0; j < SumBits<T>::kPer; j++) {
+        t = t + v[j];
+        sub |= subnormal(t);
+    }
+    if (!finite_bits(t) || (sub && policy == kPolicyRejectSubnormal))
+        if (!fold_exact<T>(total, count, at, policy, fault, gate, read))
+            return false;
+    total = t;
+    return true;
+}
+
+// t = t + (lane j's v) for j = 0 .. 63 in order. Each lane value goes through a scalar register,
+// read four adds ahead (the ties keep that order: a read right before its add would be waited
+// for). f sees every partial sum.
+__device__ __forceinline__ void tie_scalar(uint32_t &x) { asm volatile("" : "+s"(x)); }
+__device__ __forceinline__ void tie_scalar(uint64_t &x) { asm volatile("" : "+s"(x)); }
+
+template <typename T, class F>
+__device__ __forceinline__ T fold_lanes(T t, typename SumBits<T>::U v, F &&f)
+{
+    typename SumBits<T>::U q[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        q[j] = readlane_c(v, j);
+        tie_scalar(q[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < 64; j++) {
+        t = t + from_bits<T>(q[j & 3]);
+        asm volatile("" : "+v"(t));
+        f(t);
+        if (j + 4 < 64) {
+            q[j & 3] = readlane_c(v, j + 4);
+            tie_scalar(q[j & 3]);
+        }
+    }
+    return t;
+}
+
+// The serial fold (wave 0 alone; every value it keeps is uniform over the wave). Lane l holds
+// square off + l, and each add takes its square from that lane through a scalar register, read
+// while the add before it is in flight, so a square costs the latency of one dependent add, about
+// 4.6 ns. The squares are finite and not negative, so a sum can only fault by overflowing (the
+// total turns, and stays, infinite) or, under RejectSubnormal, by being subnormal: 64 squares are
+// folded with plain adds and that check, and only 64 that trip it are folded again with the exact
+// add classifier. Returns false when an Add faulted (recorded).
 template <typename T>
 __device__ bool serial_walk(const typename SumBits<T>::U *vals, uint64_t base, uint32_t len,
                             double mean, int policy, unsigned long long *fault,
@@ -1082,60 +1079,48 @@ __device__ bool serial_walk(const typename SumBits<T>::U *vals, uint64_t base, u
     const uint32_t end = off + kSerialMax < len ? off + kSerialMax : len;
     const bool reject_sub = policy == kPolicyRejectSubnormal;
     T total = from_bits<T>(sum_bits<T>(ue, m));
+    auto load = [&](uint32_t o) { // squares past `end` read as +0, which changes no total
+        const uint32_t i = o + lane < end ? o + lane : end - 1;
+        const U x = vals[ChunkLds<T>::slot(i)];
+        return o + lane < end ? x : (U)0;
+    };
+    U v = load(off);
     while (off < end) {
         const uint32_t here = end - off < 64 ? end - off : 64;
-        T v[4]; // squares past `here` read as +0, which changes no total
-#pragma unroll
-        for (int b = 0; b < 4; b++) {
-            const uint32_t i = 16 * b + (lane & 15);
-            v[b] = i < here ? from_bits<T>(vals[ChunkLds<T>::slot(off + i)]) : (T)0;
-        }
+        const U nx = load(off + here);
         T t = total;
         bool sub = false;
-#pragma unroll
-        for (int b = 0; b < 4; b++) {
-            if (reject_sub)
-                each16([&](auto j) {
-                    t = t + row_lane<decltype(j)::value>(v[b]);
-                    sub |= subnormal(t);
-                }, std::make_integer_sequence<int, 16>{});
-            else
-                each16([&](auto j) { t = t + row_lane<decltype(j)::value>(v[b]); },
-                       std::make_integer_sequence<int, 16>{});
-        }
+        if (reject_sub)
+            t = fold_lanes<T>(total, v, [&](T x) { sub |= subnormal(x); });
+        else
+            t = fold_lanes<T>(total, v, [](T) {});
         if (!finite_bits(t) || sub) {
-            T acc = total;
-            for (uint32_t i = 0; i < here; i++) {
-                const T s_i = from_bits<T>(vals[ChunkLds<T>::slot(off + i)]);
-                const T nxt = acc + s_i;
-                const uint32_t kind = classify_add(acc, s_i, nxt, policy);
-                if (kind != kOk) {
-                    if (lane == 0) {
-                        atomicMin(fault, (unsigned long long)pack_fault(3 * (base + off + i) + 2, kind));
-                        gate_record(gate);
-                    }
-                    return false;
-                }
-                acc = nxt;
-            }
+            bool ok = true;
+            if (lane == 0)
+                ok = fold_exact<T>(total, here, base + off, policy, fault, gate, [&](uint32_t i) {
+                    return from_bits<T>(vals[ChunkLds<T>::slot(off + i)]);
+                });
+            if (__ballot(!ok))
+                return false;
         }
         total = t;
         off += here;
+        const int was = ue;
         sum_phase<T>((U)bits_of(total), ue, m, mmax);
-        if (expected_gap((double)(mmax - m), ue, mean) >= kSerialGap)
+        if (ue != was && expected_gap((double)(mmax - m), ue, mean) >= kSerialGap)
             break;
+        v = nx;
     }
     return true;
 }
 
-// Exact fold of elements [start, len) of the chunk at base from the phase (ue, m, mmax): by
-// the serial walk where crossings are dense, elsewhere window by window, where the one thread
-// whose run holds the window's first step to reach the binade's end executes that step as
-// the contract's Add and the next window starts after it in the new binade. Returns false
-// when an Add faulted (recorded).
+// Exact fold of elements [start, len) of the chunk at base, staged in sh.vals (its barrier is
+// here), from the phase (ue, m, mmax): by the serial walk where crossings are dense, elsewhere
+// window by window, where the one thread whose run holds the window's first step to reach the
+// binade's end adds its run square by square and the next window starts after it, in the new
+// binade. Returns false when an Add faulted (recorded).
 template <typename T>
-__device__ bool exact_chunk(const typename SumBits<T>::U *__restrict__ src, uint64_t base,
-                            uint32_t len, uint32_t start, double mean, int policy,
+__device__ bool exact_chunk(uint64_t base, uint32_t len, uint32_t start, double mean, int policy,
                             unsigned long long *fault, int &ue, typename SumBits<T>::C &m,
                             typename SumBits<T>::C &mmax, WalkShared<T> &sh, const NodeGate &gate)
 {
@@ -1143,8 +1128,6 @@ __device__ bool exact_chunk(const typename SumBits<T>::U *__restrict__ src, uint
     using C = typename SumBits<T>::C;
     constexpr uint32_t P = SumBits<T>::kPer;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    for (uint32_t i = tid; i < len; i += kSumThreads)
-        sh.vals[ChunkLds<T>::slot(i)] = src[base + i];
     if (tid == 0)
         sh.at[0] = sh.at[1] = kNoStep;
     __syncthreads();
@@ -1195,34 +1178,16 @@ __device__ bool exact_chunk(const typename SumBits<T>::U *__restrict__ src, uint
         // Counts only grow along the window, so exactly one run can start below the
         // binade's end and reach it.
         if (mt < mmax && sat_add<T>(mt, pt ? mine.r1 : mine.r0) >= mmax) {
-            C mm = mt;
-            uint32_t pp = pt;
-            for (uint32_t i = i0; i < i1; i++) {
-                const U b = sh.vals[ChunkLds<T>::slot(i)];
-                C nn;
-                uint32_t cls;
-                sum_elem<T>(b, ue, nn, cls);
-                const C r = sum_step<C>(nn, cls, pp);
-                if (cls == kRForce || mm + r >= mmax) {
-                    // The crossing step, executed and checked as the contract's Add.
-                    const T acc = from_bits<T>(sum_bits<T>(ue, mm));
-                    const T s_i = from_bits<T>(b);
-                    const T res = acc + s_i;
-                    const uint32_t kind = classify_add(acc, s_i, res, policy);
-                    if (kind != kOk) {
-                        atomicMin(fault, (unsigned long long)pack_fault(3 * (base + i) + 2, kind));
-                        gate_record(gate);
-                        sh.stop[slot] = 1;
-                    } else {
-                        sh.stop[slot] = 0;
-                        sh.total[slot] = (U)bits_of(res);
-                    }
-                    sh.at[slot] = i;
-                    break;
-                }
-                mm += r;
-                pp = (pp + (uint32_t)r) & 1u;
-            }
+            T v[P], tot_run = from_bits<T>(sum_bits<T>(ue, mt));
+#pragma unroll
+            for (uint32_t j = 0; j < P; j++)
+                v[j] = i0 + j < i1 ? from_bits<T>(sh.vals[ChunkLds<T>::slot(i0 + j)]) : (T)0;
+            const bool ok = fold_run<T>(v, tot_run, i1 - i0, base + i0, policy, fault, gate, [&](uint32_t i) {
+                return from_bits<T>(sh.vals[ChunkLds<T>::slot(i0 + i)]);
+            });
+            sh.stop[slot] = !ok;
+            sh.total[slot] = (U)bits_of(tot_run);
+            sh.at[slot] = i1;
         }
         __syncthreads();
         const uint32_t at = sh.at[slot];
@@ -1238,7 +1203,7 @@ __device__ bool exact_chunk(const typename SumBits<T>::U *__restrict__ src, uint
         if (stop)
             return false;
         sum_phase<T>(tot, ue, m, mmax);
-        off = at + 1;
+        off = at;
         per = 0;
         serial_ok = true;
     }
@@ -1261,12 +1226,14 @@ __device__ __forceinline__ SumScan<T> scan_of_summary(const ChunkSummary &c)
 // Run-prefix fold of the chunk at base whose summary `cand` (made for the running binade)
 // reaches the binade's end. runs_c holds, per candidate, each thread run's exclusive prefix
 // (run t = elements [P*t, P*t + P)). The run where the count reaches the end is the one
-// whose prefixes straddle it; its thread walks the run with the automaton, executes the
-// crossing step as the contract's Add, and walks the rest of the run in the new binade.
+// whose prefixes straddle it; its thread adds the run's squares one by one (16 dependent adds,
+// 0.1 us; stepping the automaton through them took about 3) and so lands in the new binade.
 // The runs after it fold at once from the prefixes of a candidate made for the new binade:
 // from parity q at the chunk start a candidate's prefix adds E(q) before run t and T(q) over
 // the whole chunk, so the runs from t on add T(q) - E(q), for the q whose parity after E is
-// the parity actually standing there. Returns 1 when the chunk is folded, 0 when the Add
+// the parity actually standing there. Every thread loads its squares and its prefixes of every
+// candidate at once: one round trip to memory, which is most of the time (in a second one after
+// the crossing is known, another). Returns 1 when the chunk is folded, 0 when an Add
 // faulted (recorded), -1 when a second crossing (or a missing candidate) leaves elements
 // [*resume, len) to the windowed path, with (ue, m, mmax) standing before element *resume.
 template <typename T>
@@ -1281,90 +1248,56 @@ __device__ int run_prefix_chunk(const typename SumBits<T>::U *__restrict__ src,
     using C = typename SumBits<T>::C;
     constexpr uint32_t P = SumBits<T>::kPer;
     const int tid = threadIdx.x;
-    const SumScan<T> *ry = runs_c + (size_t)cand * kSumThreads;
-    const SumScan<T> E = ry[tid];
-    const SumScan<T> E1 = tid + 1 < kSumThreads ? ry[tid + 1] : scan_of_summary<T>(summ_c[cand]);
+    U vals[P];
+    load_chunk<T>(src, ((uintptr_t)src & 15u) == 0, base, base + len, tid, vals);
+    ChunkSummary cs[kCands];
+    SumScan<T> e0[kCands], e1[kCands];
+    const int next = tid + 1 < kSumThreads ? tid + 1 : tid;
+#pragma unroll
+    for (int y = 0; y < kCands; y++) {
+        cs[y] = summ_c[y];
+        e0[y] = runs_c[(size_t)y * kSumThreads + tid];
+        e1[y] = runs_c[(size_t)y * kSumThreads + next];
+    }
+    SumScan<T> E = e0[0], E1 = e1[0];
+#pragma unroll
+    for (int y = 0; y < kCands; y++) {
+        if (next == tid)
+            e1[y] = scan_of_summary<T>(cs[y]);
+        if (y == cand) {
+            E = e0[y];
+            E1 = e1[y];
+        }
+    }
     const uint32_t p0 = (uint32_t)(m & 1u);
     const C mt = sat_add<T>(m, p0 ? E.r1 : E.r0), mt1 = sat_add<T>(m, p0 ? E1.r1 : E1.r0);
     // Counts only grow along the chunk: exactly one run starts below the end and reaches it.
     if (mt < mmax && mt1 >= mmax) {
-        uint32_t pt = p0 ? (E.p >> 1) & 1u : E.p & 1u;
-        C mm = mt, mx = mmax;
-        int u = ue, status = 1;
-        bool crossed = false;
         const uint32_t i0 = (uint32_t)tid * P, i1 = i0 + P < len ? i0 + P : len;
-        uint32_t at = i1;
-        // The run's squares and the candidates' entries after it, in one round trip to memory
-        // ahead of the step loop, which then reads LDS.
-        U vals[P];
-        if (i0 + P <= len && ((uintptr_t)src & 15u) == 0) {
-#pragma unroll
-            for (uint32_t j = 0; j < P; j += 16 / sizeof(U)) {
-                const uint4 x = *reinterpret_cast<const uint4 *>(src + base + i0 + j);
-                const U *xs = reinterpret_cast<const U *>(&x);
-#pragma unroll
-                for (uint32_t e = 0; e < 16 / sizeof(U); e++)
-                    vals[j + e] = xs[e];
-            }
-        } else {
-#pragma unroll
-            for (uint32_t j = 0; j < P; j++)
-                vals[j] = i0 + j < len ? src[base + i0 + j] : (U)0;
-        }
-        ChunkSummary cs[kCands];
-        SumScan<T> ce[kCands];
-#pragma unroll
-        for (int y = 0; y < kCands; y++) {
-            cs[y] = summ_c[y];
-            ce[y] = tid + 1 < kSumThreads ? runs_c[(size_t)y * kSumThreads + tid + 1] : scan_identity<T>();
-        }
+        T v[P], total = from_bits<T>(sum_bits<T>(ue, mt));
 #pragma unroll
         for (uint32_t j = 0; j < P; j++)
-            sh.run_vals[j] = vals[j];
-        for (uint32_t i = i0; i < i1; i++) {
-            const U b = sh.run_vals[i - i0];
-            C nn;
-            uint32_t cls;
-            sum_elem<T>(b, u, nn, cls);
-            const C r = sum_step<C>(nn, cls, pt);
-            if (cls == kRForce || mm + r >= mx) {
-                if (crossed) { // a second crossing inside the run
-                    status = -1;
-                    at = i;
-                    break;
-                }
-                const T acc = from_bits<T>(sum_bits<T>(u, mm));
-                const T s_i = from_bits<T>(b);
-                const T res = acc + s_i;
-                const uint32_t kind = classify_add(acc, s_i, res, policy);
-                if (kind != kOk) {
-                    atomicMin(fault, (unsigned long long)pack_fault(3 * (base + i) + 2, kind));
-                    gate_record(gate);
-                    status = 0;
-                    break;
-                }
-                sum_phase<T>((U)bits_of(res), u, mm, mx);
-                pt = (uint32_t)(mm & 1u);
-                crossed = true;
-                continue;
-            }
-            mm += r;
-            pt = (pt + (uint32_t)r) & 1u;
-        }
-        if (status == 1 && i1 < len) {
+            v[j] = from_bits<T>(vals[j]);
+        const bool ok = fold_run<T>(v, total, i1 - i0, base + i0, policy, fault, gate,
+                                    [&](uint32_t i) { return from_bits<T>(src[base + i0 + i]); });
+        C mm, mx;
+        int u, status = ok ? 1 : 0;
+        sum_phase<T>((U)bits_of(total), u, mm, mx);
+        if (ok && i1 < len) {
             // The runs after this one, from the prefixes of a candidate for the new binade.
             status = -1;
-            int found = -1;
+            const uint32_t pt = (uint32_t)(mm & 1u);
+            bool found = false;
             SumScan<T> Ey = scan_identity<T>(), Ty = scan_identity<T>();
 #pragma unroll
             for (int y = kCands - 1; y >= 0; y--)
                 if (cs[y].ue == u) {
-                    found = y;
-                    Ey = ce[y];
+                    found = true;
+                    Ey = e1[y];
                     Ty = scan_of_summary<T>(cs[y]);
                 }
             const int q = (Ey.p & 1u) == pt ? 0 : (((Ey.p >> 1) & 1u) == pt ? 1 : -1);
-            if (found >= 0 && q >= 0) {
+            if (found && q >= 0) {
                 const C tq = q ? Ty.r1 : Ty.r0, eq = q ? Ey.r1 : Ey.r0;
                 if (tq < SumBits<T>::kCap && mm + (tq - eq) < mx) {
                     mm += tq - eq;
@@ -1375,7 +1308,7 @@ __device__ int run_prefix_chunk(const typename SumBits<T>::U *__restrict__ src,
         sh.run_status = status;
         sh.run_ue = u;
         sh.run_m = (uint64_t)mm;
-        sh.run_resume = at;
+        sh.run_resume = i1;
     }
     __syncthreads();
     const int status = sh.run_status;
@@ -1386,36 +1319,71 @@ __device__ int run_prefix_chunk(const typename SumBits<T>::U *__restrict__ src,
     return status;
 }
 
-// A: chunk sums in binary64 (order inside a chunk does not matter: only an estimate).
-template <typename T>
-__global__ __launch_bounds__(256) void k_mse_chunk_sums(const T *__restrict__ sq, uint64_t n,
-                                                        const unsigned long long *fault,
-                                                        double *__restrict__ chunk_sum, NodeGate gate)
+// A: the squares, with the first faulting Subtract or Multiply, and beside them each quarter
+// chunk's sum in binary64 (order does not matter: only an estimate, so what is not finite, at or
+// after a fault, is left out). One quarter a workgroup, all of a thread's loads in flight at
+// once; 12 bytes an element (f32) over memory bound it. A pass of its own over the squares for
+// the sums took 4.6 us beside 14 at 4096 x 1024 f32.
+template <typename T, bool VEC>
+__global__ __launch_bounds__(kEwThreads) void k_mse_squares(const T *__restrict__ p,
+                                                            const T *__restrict__ t,
+                                                            T *__restrict__ sq, uint64_t n,
+                                                            int policy,
+                                                            double *__restrict__ quarter_sum,
+                                                            unsigned long long *fault, NodeGate gate)
 {
     if (block_gate_closed(gate))
         return;
-    __shared__ double part[4];
-    const uint64_t limit = sum_limit(fault, n);
-    const uint64_t base = (uint64_t)blockIdx.x * sum_chunk_len<T>();
-    const uint64_t end = base + sum_chunk_len<T>() < limit ? base + sum_chunk_len<T>() : limit;
+    constexpr int W = Lanes<T, VEC>::W;
+    constexpr int kQuarter = kSumThreads * SumBits<T>::kPer / kQuarters;
+    constexpr int R = kQuarter / (kEwThreads * W);
+    __shared__ double part[kEwThreads / 64];
+    const uint64_t first = (uint64_t)blockIdx.x * kQuarter + threadIdx.x * W;
+    uint64_t key = kNoFault;
     double acc = 0.0;
-    if (end - base == sum_chunk_len<T>() && ((uintptr_t)sq & 15u) == 0) {
-        // A whole chunk: every 16-byte load of the thread in flight at once.
-        constexpr int P = 16 / sizeof(T), R = (int)(kSumThreads * SumBits<T>::kPer / (256 * P));
-        uint4 q[R];
+    T pv[R][W], tv[R][W];
 #pragma unroll
-        for (int j = 0; j < R; j++)
-            q[j] = *reinterpret_cast<const uint4 *>(sq + base + P * (256 * j + threadIdx.x));
-#pragma unroll
-        for (int j = 0; j < R; j++) {
-            const T *v = reinterpret_cast<const T *>(&q[j]);
-#pragma unroll
-            for (int e = 0; e < P; e++)
-                acc += (double)v[e];
+    for (int r = 0; r < R; r++) {
+        const uint64_t base = first + (uint64_t)r * kEwThreads * W;
+        if (base < n) {
+            load_lanes<T, VEC>(p, base, n, pv[r]);
+            load_lanes<T, VEC>(t, base, n, tv[r]);
         }
-    } else {
-        for (uint64_t i = base + threadIdx.x; i < end; i += 256)
-            acc += (double)sq[i];
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const uint64_t base = first + (uint64_t)r * kEwThreads * W;
+        if (base >= n)
+            break;
+        T d[W], sv[W];
+        bool any = false;
+#pragma unroll
+        for (int j = 0; j < W; j++) {
+            d[j] = pv[r][j] - tv[r][j];
+            sv[j] = d[j] * d[j];
+            if (base + j < n) {
+                any |= add_suspect(pv[r][j], tv[r][j], d[j], policy) |
+                       mul_suspect(d[j], d[j], sv[j], policy);
+                acc += finite_bits(sv[j]) ? (double)sv[j] : 0.0;
+            }
+        }
+        // Ordinary stores: the ordered sum reads the squares next.
+        store_lanes<T, VEC, false>(sq, base, n, sv);
+        if (any && key == kNoFault) {
+#pragma unroll
+            for (int j = 0; j < W; j++) {
+                if (base + j >= n || key != kNoFault)
+                    continue;
+                const uint32_t ks = classify_add(pv[r][j], tv[r][j], d[j], policy);
+                if (ks != kOk) {
+                    key = pack_fault(3 * (base + j), ks);
+                } else {
+                    const uint32_t km = classify_mul(d[j], d[j], sv[j], policy);
+                    if (km != kOk)
+                        key = pack_fault(3 * (base + j) + 1, km);
+                }
+            }
+        }
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1)
@@ -1424,13 +1392,15 @@ __global__ __launch_bounds__(256) void k_mse_chunk_sums(const T *__restrict__ sq
         part[threadIdx.x >> 6] = acc;
     __syncthreads();
     if (threadIdx.x == 0)
-        chunk_sum[blockIdx.x] = (part[0] + part[1]) + (part[2] + part[3]);
+        quarter_sum[blockIdx.x] = (part[0] + part[1]) + (part[2] + part[3]);
+    wave_record_fault(key, fault, gate);
 }
 
-// B: exclusive prefix of the chunk sums (one workgroup; each thread a contiguous run).
+// B: chunk sums and their exclusive prefix (one workgroup; each thread a contiguous run).
 constexpr int kPrefixThreads = 1024;
-__global__ __launch_bounds__(kPrefixThreads) void k_mse_chunk_prefix(const double *__restrict__ chunk_sum,
+__global__ __launch_bounds__(kPrefixThreads) void k_mse_chunk_prefix(const double *__restrict__ quarter_sum,
                                                                      uint64_t chunks,
+                                                                     double *__restrict__ chunk_sum,
                                                                      double *__restrict__ pre,
                                                                      NodeGate gate)
 {
@@ -1442,8 +1412,12 @@ __global__ __launch_bounds__(kPrefixThreads) void k_mse_chunk_prefix(const doubl
     const uint64_t i0 = (uint64_t)tid * per;
     const uint64_t i1 = i0 + per < chunks ? i0 + per : chunks;
     double own = 0.0;
-    for (uint64_t i = i0; i < i1; i++)
-        own += chunk_sum[i];
+    for (uint64_t i = i0; i < i1; i++) {
+        const double *q = quarter_sum + kQuarters * i;
+        const double sum = (q[0] + q[1]) + (q[2] + q[3]);
+        chunk_sum[i] = sum;
+        own += sum;
+    }
     double inc = own;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
@@ -1484,26 +1458,21 @@ __global__ __launch_bounds__(kSumThreads) void k_mse_chunk_summaries(
     const int32_t lo = phase_ue_of<T>(pre * (1.0 - 1.0 / 512)), hi = phase_ue_of<T>(pre * (1.0 + 1.0 / 512));
     const int32_t end = phase_ue_of<T>((pre + chunk_sum[c]) * (1.0 + 1.0 / 512));
     ChunkSummary *out = summ + kCands * c + blockIdx.y;
-    if ((blockIdx.y == 1 && hi == lo) || (blockIdx.y == 2 && end <= lo)) {
+    const int ue = blockIdx.y == 0 ? lo : (blockIdx.y == 1 ? hi : hi + 1);
+    if ((blockIdx.y == 1 && hi == lo) || (blockIdx.y == 2 && end <= lo) || !phase_valid<T>(ue)) {
         if (tid == 0)
             *out = ChunkSummary{0, 0, kNoPhase, 0};
         return;
     }
-    const int ue = blockIdx.y == 0 ? lo : (blockIdx.y == 1 ? hi : hi + 1);
     const U *src = reinterpret_cast<const U *>(sq);
     U cur[P];
     const uint64_t base = c * sum_chunk_len<T>();
     load_chunk<T>(src, ((uintptr_t)sq & 15u) == 0, base, limit, tid, cur);
-    const uint64_t first = base + (uint64_t)tid * P;
-    SumScan<T> mine = scan_identity<T>();
+    T v[P];
 #pragma unroll
-    for (int j = 0; j < P; j++) {
-        typename SumBits<T>::C nn;
-        uint32_t cls;
-        sum_elem<T>(cur[j], ue, nn, cls);
-        if (first + j < limit)
-            mine = scan_compose<T>(mine, scan_elem<T>(nn, cls));
-    }
+    for (int j = 0; j < P; j++)
+        v[j] = from_bits<T>(cur[j]);
+    const SumScan<T> mine = run_summary<T, P>(v, ue);
     SumScan<T> excl, total;
     block_scan<T>(mine, lane, wave, wave_tot, excl, total);
     runs[(kCands * c + blockIdx.y) * kSumThreads + tid] = excl;
@@ -1545,6 +1514,7 @@ __global__ __launch_bounds__(kSumThreads) __attribute__((amdgpu_waves_per_eu(4))
         const uint64_t c = b0 + tid;
         int32_t cue[kCands];
         SumScan<T> cscan[kCands];
+        const double csum = c < chunks ? chunk_sum[c] : 0.0;
 #pragma unroll
         for (int y = 0; y < kCands; y++) {
             cue[y] = kNoPhase;
@@ -1580,11 +1550,13 @@ __global__ __launch_bounds__(kSumThreads) __attribute__((amdgpu_waves_per_eu(4))
             sh.first[slot] = (uint32_t)tid;
             sh.m_first[slot] = (uint64_t)mt;
             sh.first_cand[slot] = cand;
+            sh.mean[slot] = csum / (double)(c + 1 < chunks ? L : limit - c * L);
         }
         __syncthreads();
         const uint32_t first = sh.first[slot];
         const C m_first = (C)sh.m_first[slot];
         const int first_cand = sh.first_cand[slot];
+        const double mean = sh.mean[slot];
         if (tid == 0)
             sh.first[slot ^ 1] = kNoStep;
         if (first == kNoStep) {
@@ -1592,23 +1564,32 @@ __global__ __launch_bounds__(kSumThreads) __attribute__((amdgpu_waves_per_eu(4))
             c0 = bend;
             continue;
         }
-        // Chunks before the stopping one fold; it runs exactly from the count before it:
-        // from its run prefixes when it has a summary for this binade, and in windows from
+        // Chunks before the stopping one fold; it runs exactly from the count before it: from
+        // its run prefixes when it has a summary for this binade and the next binade is not
+        // expected to end in the chunk's dense part too, and with the staged squares from
         // wherever that leaves off.
         m = m_first;
         const uint64_t cc = b0 + first;
         const uint64_t base = cc * L;
         const uint32_t len = (uint32_t)(base + L <= limit ? L : limit - base);
         uint32_t resume = 0;
-        const int folded = first_cand < 0 ? -1
-                                          : run_prefix_chunk<T>(src, runs + kCands * cc * kSumThreads,
-                                                                summ + kCands * cc, first_cand, base, len,
-                                                                policy, fault, ue, m, mmax, resume, sh, gate);
+        const bool dense = expected_gap((double)((C)1 << SumBits<T>::kFrac), ue + 1, mean) < kSerialGap;
+        const int folded = first_cand < 0 || dense
+                               ? -1
+                               : run_prefix_chunk<T>(src, runs + kCands * cc * kSumThreads,
+                                                     summ + kCands * cc, first_cand, base, len,
+                                                     policy, fault, ue, m, mmax, resume, sh, gate);
         if (folded == 0)
             return;
-        if (folded < 0 && !exact_chunk<T>(src, base, len, resume, chunk_sum[cc] / (double)len, policy,
-                                          fault, ue, m, mmax, sh, gate))
-            return;
+        if (folded < 0) {
+            U vals[SumBits<T>::kPer];
+            load_chunk<T>(src, ((uintptr_t)src & 15u) == 0, base, base + len, tid, vals);
+#pragma unroll
+            for (uint32_t j = 0; j < (uint32_t)SumBits<T>::kPer; j++)
+                sh.vals[ChunkLds<T>::slot(tid * SumBits<T>::kPer + j)] = vals[j];
+            if (!exact_chunk<T>(base, len, resume, mean, policy, fault, ue, m, mmax, sh, gate))
+                return;
+        }
         c0 = cc + 1;
         }
     }
@@ -1625,36 +1606,33 @@ __global__ __launch_bounds__(kSumThreads) __attribute__((amdgpu_waves_per_eu(4))
     }
 }
 
-// Small inputs (n <= kMseSerialMax), one workgroup. Its four waves form every difference and
-// square in parallel into LDS (each thread issues all of its loads before it computes, so
-// the inputs arrive in one round trip) and find the first faulting Subtract or Multiply; then
-// one wave folds the squares before that element into the total in order, a chunk of 60
-// (binary64 30) at a time, each lane holding the chunk's squares in registers and the next
-// chunk's loads in flight. The
-// squares folded are finite, so a sum can only fault by overflowing (the total turns, and
-// stays, infinite) or, under RejectSubnormal, by being subnormal: a chunk is folded with
-// plain adds (under RejectSubnormal each partial total is kept and checked after), and folded
-// again with the exact add classifier only when that trips. The same results and first fault
-// as the pipeline above, in one launch and no scratch.
-template <typename T, bool REJECT_SUB>
-__global__ __launch_bounds__(256) void k_mse_serial(const T *__restrict__ p, const T *__restrict__ t,
-                                                    uint64_t n, T count, int policy,
-                                                    T *__restrict__ out, unsigned long long *fault,
-                                                    NodeGate gate)
+// Inputs of one chunk, one workgroup. Its waves form every difference and square in parallel into
+// LDS (each thread issues all of its loads before it computes, so the inputs arrive in one round
+// trip), find the first faulting Subtract or Multiply and estimate the mean; then the squares
+// before that element fold as a chunk of the pipeline above does, from +0. The same results and
+// first fault, in one launch and no scratch. What bounds it is the chain of phases: 512 or so
+// dependent adds, then a window for each doubling of the total: 17 us at 4096 f32, where one wave
+// adding all of the squares took 22.7.
+template <typename T>
+__global__ __launch_bounds__(kSumThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_mse_one(
+    const T *__restrict__ p, const T *__restrict__ t, uint64_t n, T count, int policy,
+    T *__restrict__ out, unsigned long long *fault, NodeGate gate)
 {
     if (block_gate_closed(gate))
         return;
-    constexpr int P = 16 / sizeof(T);           // squares per 16-byte LDS read
-    constexpr int R = (int)(kMseSerialMax / 256); // elements a thread
-    __shared__ __align__(16) T sq[kMseSerialMax];
+    using U = typename SumBits<T>::U;
+    using C = typename SumBits<T>::C;
+    constexpr int P = SumBits<T>::kPer;
+    __shared__ WalkShared<T> sh;
     __shared__ unsigned long long first_sm; // earliest Subtract or Multiply fault word
+    __shared__ double part[kSumThreads / 64];
     const int tid = threadIdx.x;
     if (tid == 0)
         first_sm = kNoFault;
-    T pv[R], tv[R];
+    T pv[P], tv[P];
 #pragma unroll
-    for (int j = 0; j < R; j++) {
-        const uint64_t i = (uint64_t)tid + 256u * (uint64_t)j;
+    for (int j = 0; j < P; j++) {
+        const uint64_t i = (uint64_t)tid + (uint64_t)(kSumThreads * j);
         if (i < n) {
             pv[j] = p[i];
             tv[j] = t[i];
@@ -1662,13 +1640,15 @@ __global__ __launch_bounds__(256) void k_mse_serial(const T *__restrict__ p, con
     }
     __syncthreads();
     uint64_t key = kNoFault;
+    double acc = 0.0;
 #pragma unroll
-    for (int j = 0; j < R; j++) {
-        const uint64_t i = (uint64_t)tid + 256u * (uint64_t)j;
+    for (int j = 0; j < P; j++) {
+        const uint64_t i = (uint64_t)tid + (uint64_t)(kSumThreads * j);
         if (i < n) {
             const T d = pv[j] - tv[j];
             const T s = d * d;
-            sq[i] = s;
+            sh.vals[ChunkLds<T>::slot((uint32_t)i)] = (U)bits_of(s);
+            acc += finite_bits(s) ? (double)s : 0.0;
             if (key == kNoFault) {
                 const uint32_t ks = classify_add(pv[j], tv[j], d, policy);
                 if (ks != kOk) {
@@ -1683,105 +1663,34 @@ __global__ __launch_bounds__(256) void k_mse_serial(const T *__restrict__ p, con
     }
     if (key != kNoFault)
         atomicMin(&first_sm, (unsigned long long)key);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1)
+        acc += __shfl_xor(acc, off, 64);
+    if ((tid & 63) == 0)
+        part[tid >> 6] = acc;
     __syncthreads();
-    if (tid >= 64)
-        return;
     const unsigned long long fsm = first_sm;
     const uint64_t limit = fsm == kNoFault ? n : ((fsm >> 3) / 3); // elements summed
-    auto record = [&](uint64_t w) {
-        if (tid == 0) {
-            atomicMin(fault, (unsigned long long)w);
-            gate_record(gate);
-        }
-    };
-    T total = (T)0;
-    // The exact pass over squares i0 .. i0 + here - 1 from `total`: false when an add faults
-    // (recorded).
-    auto exact = [&](uint64_t i0, int here) {
-        T tot = total;
-        for (int j = 0; j < here; j++) {
-            const T sj = sq[i0 + j];
-            const T nxt = tot + sj;
-            const uint32_t k_add = classify_add(tot, sj, nxt, policy);
-            if (k_add != kOk) {
-                record(pack_fault(3 * (i0 + j) + 2, k_add));
-                return false;
-            }
-            tot = nxt;
-        }
-        return true;
-    };
-    // A chunk is 15 LDS reads: with the next chunk's 15 reads issued before its adds, the
-    // wait for this chunk (in-order LDS counter, at most 15 outstanding) leaves all of them in
-    // flight.
-    constexpr int CH = 15 * P;
-    auto load = [&](T (&v)[CH], uint64_t i0) {
+    double sum = 0.0;
 #pragma unroll
-        for (int q = 0; q < CH / P; q++)
-            *reinterpret_cast<uint4 *>(&v[P * q]) = *reinterpret_cast<const uint4 *>(&sq[i0 + P * q]);
-    };
-    // Folds a whole chunk held in v; false when an add faults (recorded).
-    auto fold = [&](T (&v)[CH], uint64_t i0) __attribute__((always_inline)) {
-        T sum = total;
-        bool trip = false;
-        if constexpr (!REJECT_SUB) {
-#pragma unroll
-            for (int j = 0; j < CH; j++)
-                sum = sum + v[j];
-        } else {
-#pragma unroll
-            for (int j = 0; j < CH; j++) {
-                sum = sum + v[j];
-                v[j] = sum;
-            }
-#pragma unroll
-            for (int j = 0; j < CH; j++)
-                trip |= subnormal(v[j]);
-        }
-        if ((!finite_bits(sum) || trip) && !exact(i0, CH))
-            return false;
-        total = sum;
-        return true;
-    };
-    const uint64_t full = limit / CH * CH;
-    T va[CH], vb[CH];
-    if (full > 0)
-        load(va, 0);
-    for (uint64_t i0 = 0; i0 < full; i0 += 2 * CH) {
-        const bool second = i0 + CH < full;
-        if (second)
-            load(vb, i0 + CH);
-        if (!fold(va, i0))
-            return;
-        if (!second)
-            break;
-        if (i0 + 2 * CH < full)
-            load(va, i0 + 2 * CH);
-        if (!fold(vb, i0 + CH))
-            return;
-    }
-    if (limit > full) {
-        const int here = (int)(limit - full);
-        T sum = total;
-        bool trip = false;
-        for (int j = 0; j < here; j++) {
-            sum = sum + sq[full + j];
-            trip |= REJECT_SUB && subnormal(sum);
-        }
-        if ((!finite_bits(sum) || trip) && !exact(full, here))
-            return;
-        total = sum;
-    }
-    if (fsm != kNoFault) {
-        record(fsm);
+    for (int w = 0; w < kSumThreads / 64; w++)
+        sum += part[w];
+    int ue;
+    C m, mmax;
+    sum_phase<T>((U)0, ue, m, mmax); // the total starts at +0
+    if (!exact_chunk<T>(0, (uint32_t)limit, 0, sum / (double)n, policy, fault, ue, m, mmax, sh, gate))
         return;
-    }
+    if (tid != 0)
+        return;
+    const T total = from_bits<T>(sum_bits<T>(ue, m));
     const T r = total / count;
-    const uint32_t kind = classify_div(total, count, r, policy);
-    if (kind != kOk)
-        record(pack_fault(3 * n, kind));
-    else if (tid == 0)
+    const uint32_t kind = fsm != kNoFault ? kOk : classify_div(total, count, r, policy);
+    if (fsm != kNoFault || kind != kOk) {
+        atomicMin(fault, fsm != kNoFault ? fsm : (unsigned long long)pack_fault(3 * n, kind));
+        gate_record(gate);
+    } else {
         *out = r;
+    }
 }
 
 // ------------------------------------------------------------- native compounds
@@ -2140,7 +2049,7 @@ hipError_t launch_sgd_pair(hipStream_t s, int dtype, const SgdJob &j0, const Sgd
                       : sgd_pair_t<double>(s, j0, j1, policy, close, closed);
 }
 
-// Scratch of one MSE call: the squares, then the chunk sums and the chunk summaries.
+// Scratch of one MSE call: the squares, then the quarter and chunk sums and the summaries.
 static inline size_t round256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 template <typename T>
@@ -2155,14 +2064,15 @@ size_t mse_scratch_bytes(int dtype, uint64_t n)
     const size_t es = dtype == 0 ? 4 : 8;
     const size_t chunks = dtype == 0 ? mse_chunks<float>(n) : mse_chunks<double>(n);
     const size_t run_bytes = dtype == 0 ? sizeof(SumScan<float>) : sizeof(SumScan<double>);
-    return round256(n * es) + 2 * round256(chunks * sizeof(double)) +
+    return round256(n * es) + round256(kQuarters * chunks * sizeof(double)) +
+           2 * round256(chunks * sizeof(double)) +
            round256(kCands * chunks * sizeof(ChunkSummary)) +
            round256(kCands * chunks * kSumThreads * run_bytes);
 }
 
 template <typename T> struct MseScratch {
     T *squares;
-    double *chunk_sum, *chunk_pre;
+    double *quarter_sum, *chunk_sum, *chunk_pre;
     ChunkSummary *summ;
     SumScan<T> *runs;
     size_t chunks;
@@ -2171,7 +2081,8 @@ template <typename T> struct MseScratch {
         char *base = (char *)scratch;
         chunks = mse_chunks<T>(n);
         squares = (T *)base;
-        chunk_sum = (double *)(base + round256(n * sizeof(T)));
+        quarter_sum = (double *)(base + round256(n * sizeof(T)));
+        chunk_sum = (double *)((char *)quarter_sum + round256(kQuarters * chunks * sizeof(double)));
         chunk_pre = (double *)((char *)chunk_sum + round256(chunks * sizeof(double)));
         summ = (ChunkSummary *)((char *)chunk_pre + round256(chunks * sizeof(double)));
         runs = (SumScan<T> *)((char *)summ + round256(kCands * chunks * sizeof(ChunkSummary)));
@@ -2182,16 +2093,14 @@ template <typename T>
 static hipError_t mse_prepare_t(hipStream_t s, uint64_t n, const void *p, const void *t,
                                 void *scratch, int policy, unsigned long long *fault, NodeGate gate)
 {
-    constexpr int Wd = Vec<T>::width;
     const MseScratch<T> m(scratch, n);
     const bool vec = aligned16(p) && aligned16(t) && aligned16(m.squares);
-    const unsigned grid = grid_for(vec ? (n + Wd - 1) / Wd : n);
+    const unsigned grid = (unsigned)(kQuarters * m.chunks);
     if (vec)
-        hipLaunchKernelGGL((k_mse_squares<T, true>), dim3(grid), dim3(kEwThreads), 0, s, (const T *)p, (const T *)t, m.squares, n, policy, fault, gate);
+        hipLaunchKernelGGL((k_mse_squares<T, true>), dim3(grid), dim3(kEwThreads), 0, s, (const T *)p, (const T *)t, m.squares, n, policy, m.quarter_sum, fault, gate);
     else
-        hipLaunchKernelGGL((k_mse_squares<T, false>), dim3(grid), dim3(kEwThreads), 0, s, (const T *)p, (const T *)t, m.squares, n, policy, fault, gate);
-    hipLaunchKernelGGL((k_mse_chunk_sums<T>), dim3((unsigned)m.chunks), dim3(256), 0, s, (const T *)m.squares, n, (const unsigned long long *)fault, m.chunk_sum, gate);
-    hipLaunchKernelGGL(k_mse_chunk_prefix, dim3(1), dim3(kPrefixThreads), 0, s, (const double *)m.chunk_sum, (uint64_t)m.chunks, m.chunk_pre, gate);
+        hipLaunchKernelGGL((k_mse_squares<T, false>), dim3(grid), dim3(kEwThreads), 0, s, (const T *)p, (const T *)t, m.squares, n, policy, m.quarter_sum, fault, gate);
+    hipLaunchKernelGGL(k_mse_chunk_prefix, dim3(1), dim3(kPrefixThreads), 0, s, (const double *)m.quarter_sum, (uint64_t)m.chunks, m.chunk_sum, m.chunk_pre, gate);
     hipLaunchKernelGGL((k_mse_chunk_summaries<T>), dim3((unsigned)m.chunks, kCands), dim3(kSumThreads), 0, s, (const T *)m.squares, n, (const unsigned long long *)fault, (const double *)m.chunk_sum, (const double *)m.chunk_pre, m.summ, m.runs, gate);
     return hipGetLastError();
 }
@@ -2223,21 +2132,20 @@ hipError_t launch_mse_walk(hipStream_t s, int dtype, uint64_t n, void *scratch, 
                       : mse_walk_t<double>(s, n, scratch, count, out, policy, fault, gate);
 }
 
-hipError_t launch_mse_serial(hipStream_t s, int dtype, uint64_t n, const void *p, const void *t,
-                             double count, void *out, int policy, unsigned long long *fault,
-                             NodeGate gate)
+uint64_t mse_one_max(int dtype)
 {
-    if (n == 0 || n > kMseSerialMax)
+    return (uint64_t)kSumThreads * (dtype == 0 ? SumBits<float>::kPer : SumBits<double>::kPer);
+}
+
+hipError_t launch_mse_one(hipStream_t s, int dtype, uint64_t n, const void *p, const void *t,
+                          double count, void *out, int policy, unsigned long long *fault, NodeGate gate)
+{
+    if (n == 0 || n > mse_one_max(dtype))
         return hipErrorInvalidValue;
-    const bool rs = policy == kPolicyRejectSubnormal;
-    if (dtype == 0 && rs)
-        hipLaunchKernelGGL((k_mse_serial<float, true>), dim3(1), dim3(256), 0, s, (const float *)p, (const float *)t, n, (float)count, policy, (float *)out, fault, gate);
-    else if (dtype == 0)
-        hipLaunchKernelGGL((k_mse_serial<float, false>), dim3(1), dim3(256), 0, s, (const float *)p, (const float *)t, n, (float)count, policy, (float *)out, fault, gate);
-    else if (rs)
-        hipLaunchKernelGGL((k_mse_serial<double, true>), dim3(1), dim3(256), 0, s, (const double *)p, (const double *)t, n, count, policy, (double *)out, fault, gate);
+    if (dtype == 0)
+        hipLaunchKernelGGL((k_mse_one<float>), dim3(1), dim3(kSumThreads), 0, s, (const float *)p, (const float *)t, n, (float)count, policy, (float *)out, fault, gate);
     else
-        hipLaunchKernelGGL((k_mse_serial<double, false>), dim3(1), dim3(256), 0, s, (const double *)p, (const double *)t, n, count, policy, (double *)out, fault, gate);
+        hipLaunchKernelGGL((k_mse_one<double>), dim3(1), dim3(kSumThreads), 0, s, (const double *)p, (const double *)t, n, count, policy, (double *)out, fault, gate);
     return hipGetLastError();
 }
 

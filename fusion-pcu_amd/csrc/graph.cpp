@@ -896,7 +896,7 @@ pcu_status Prepared::build(Ctx *c, const Graph &g, const std::vector<uint32_t> &
     // more than the overlap saves.
     for (uint32_t i : order)
         if (graph.nodes[i].op == Op::MeanSquaredError && uses[i] == 0 && route[i] == Route::Strict &&
-            graph.elements(graph.nodes[i].a) > kMseSerialMax)
+            graph.elements(graph.nodes[i].a) > mse_one_max(graph.nodes[graph.nodes[i].a].dtype))
             mse_side[i] = 1;
     // Device storage: one buffer per computed node; outputs get two banks so a faulting
     // execution never overwrites the published results. A Constant is uploaded once here

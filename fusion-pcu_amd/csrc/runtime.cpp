@@ -1164,8 +1164,8 @@ pcu_status Ctx::op_mse(int dtype, uint64_t n, const void *p, const void *t, void
     pcu_status st = add_node(NodeInfo{Prim::Mse, n, 0}, &word);
     if (st)
         return st;
-    if (n <= kMseSerialMax) {
-        // One wave folds a small input in order; it overlaps the following work on the side
+    if (n <= mse_one_max(dtype)) {
+        // One workgroup folds a small input in order; it overlaps the following work on the side
         // stream as the walk does.
         if ((st = open_words()))
             return st;
@@ -1179,8 +1179,8 @@ pcu_status Ctx::op_mse(int dtype, uint64_t n, const void *p, const void *t, void
             side_pending = true;
         }
         hipEvent_t t1 = timer_start(s);
-        if ((st = hip(launch_mse_serial(s, dtype, n, p, t, count_as(dtype, n), out, policy, word,
-                                        gate_for(word)), "strict_mse launch")))
+        if ((st = hip(launch_mse_one(s, dtype, n, p, t, count_as(dtype, n), out, policy, word,
+                                     gate_for(word)), "strict_mse launch")))
             return st;
         timer_stop(PCU_KERNEL_MSE, t1, s);
         return PCU_OK;

@@ -34,12 +34,14 @@ def _check(ctx, pcu_pkg, p, policy):
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
 @pytest.mark.parametrize("policy", [0, 1, 2])
-def test_first_squares(ctx, pcu_pkg, dtype, policy):
+@pytest.mark.parametrize("n", [4 * 8192 + 77, 8192, 4096])
+def test_first_squares(ctx, pcu_pkg, dtype, policy, n):
     rng = np.random.default_rng(3)
     info = np.finfo(dtype)
-    n = 4 * 8192 + 77
     base = rng.uniform(-1, 1, n).astype(dtype)
-    for first in (0, 1, 63, 64, 65, 1000, 4095, 4096, 5000):
+    for first in (0, 1, 63, 64, 65, 1000, 4000, 4095, 4096, 5000):
+        if first + 3 > n:
+            continue
         p = base.copy()
         p[:first] = 0  # the total leaves +0 at square `first`
         _check(ctx, pcu_pkg, p, policy)
@@ -59,9 +61,15 @@ def test_first_squares(ctx, pcu_pkg, dtype, policy):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
-def test_lengths_past_the_one_workgroup_kernel(ctx, pcu_pkg, dtype):
+def test_lengths_about_the_one_workgroup_kernel(ctx, pcu_pkg, dtype):
     rng = np.random.default_rng(9)
-    for n in (4097, 4160, 4161, 8191, 8192, 8193, 8192 + 63, 12289, 16385, 40960 + 15):
+    for n in (1, 63, 65, 512, 513, 4095, 4096, 4097, 4160, 4161, 8191, 8192, 8193, 8192 + 63, 12289,
+              16385, 40960 + 15):
         _check(ctx, pcu_pkg, rng.normal(0, 1, n).astype(dtype), 0)
         # Whole counts: a crossing at every power of two, at run and chunk edges.
         _check(ctx, pcu_pkg, np.ones(n, dtype), 0)
+        # A first Subtract fault late in each quarter of the last chunk.
+        for at in {n - 1, n - n // 4 - 1, n // 2}:
+            p = rng.normal(0, 1, n).astype(dtype)
+            p[at] = np.inf
+            _check(ctx, pcu_pkg, p, 0)
