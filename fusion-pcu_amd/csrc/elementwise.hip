@@ -802,7 +802,8 @@ __device__ __forceinline__ SumScan<T> run_summary(const T (&v)[N], int ue)
 //  A  k_mse_squares          the squares, and each quarter chunk's sum in binary64 (an
 //                            estimate: order does not matter);
 //  B  k_mse_chunk_prefix     the chunks' sums and their exclusive prefix: about where the
-//                            running total stands at each chunk start;
+//                            running total stands at each chunk start (C's own work for
+//                            up to 512 chunks);
 //  C  k_mse_chunk_summaries  per chunk, in parallel, the summary (count added for an even
 //                            and an odd start) of the whole chunk inside one binade, for
 //                            the one or two binades the estimate allows;
@@ -1440,11 +1441,15 @@ __global__ __launch_bounds__(kPrefixThreads) void k_mse_chunk_prefix(const doubl
 // C: summary of chunk blockIdx.x for candidate blockIdx.y (0: the binade of the estimate
 // less 1/512 of it; 1: plus 1/512, skipped when both agree; 2: the binade after candidate 1,
 // only when the estimate says the chunk crosses), with every thread run's exclusive prefix.
+// Up to kSumThreads chunks (chunk_pre null) each block sums the quarters before its chunk itself,
+// four loads a thread at most, and the first block of a chunk stores its sum: 9.2 us at 512 chunks
+// against 7.3 with a launch of 3.9 before it. With more chunks each block would read more.
 template <typename T>
 __global__ __launch_bounds__(kSumThreads) void k_mse_chunk_summaries(
     const T *__restrict__ sq, uint64_t n, const unsigned long long *fault,
-    const double *__restrict__ chunk_sum, const double *__restrict__ chunk_pre,
-    ChunkSummary *__restrict__ summ, SumScan<T> *__restrict__ runs, NodeGate gate)
+    const double *__restrict__ quarter_sum, double *__restrict__ chunk_sum,
+    const double *__restrict__ chunk_pre, ChunkSummary *__restrict__ summ,
+    SumScan<T> *__restrict__ runs, NodeGate gate)
 {
     if (block_gate_closed(gate))
         return;
@@ -1454,9 +1459,36 @@ __global__ __launch_bounds__(kSumThreads) void k_mse_chunk_summaries(
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint64_t c = blockIdx.x;
     const uint64_t limit = sum_limit(fault, n);
-    const double pre = chunk_pre[c];
+    double pre, own;
+    if (chunk_pre != nullptr) {
+        pre = chunk_pre[c];
+        own = chunk_sum[c];
+    } else {
+        __shared__ double part[kSumThreads / 64];
+        double q[kQuarters];
+#pragma unroll
+        for (int j = 0; j < kQuarters; j++) {
+            const uint64_t i = (uint64_t)(kSumThreads * j + tid);
+            q[j] = i < kQuarters * c ? quarter_sum[i] : 0.0;
+        }
+        const double *mine = quarter_sum + kQuarters * c;
+        own = (mine[0] + mine[1]) + (mine[2] + mine[3]);
+        if (blockIdx.y == 0 && tid == 0)
+            chunk_sum[c] = own;
+        double acc = (q[0] + q[1]) + (q[2] + q[3]);
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1)
+            acc += __shfl_xor(acc, off, 64);
+        if (lane == 0)
+            part[wave] = acc;
+        __syncthreads();
+        pre = 0.0;
+#pragma unroll
+        for (int w = 0; w < kSumThreads / 64; w++)
+            pre += part[w];
+    }
     const int32_t lo = phase_ue_of<T>(pre * (1.0 - 1.0 / 512)), hi = phase_ue_of<T>(pre * (1.0 + 1.0 / 512));
-    const int32_t end = phase_ue_of<T>((pre + chunk_sum[c]) * (1.0 + 1.0 / 512));
+    const int32_t end = phase_ue_of<T>((pre + own) * (1.0 + 1.0 / 512));
     ChunkSummary *out = summ + kCands * c + blockIdx.y;
     const int ue = blockIdx.y == 0 ? lo : (blockIdx.y == 1 ? hi : hi + 1);
     if ((blockIdx.y == 1 && hi == lo) || (blockIdx.y == 2 && end <= lo) || !phase_valid<T>(ue)) {
@@ -1482,10 +1514,11 @@ __global__ __launch_bounds__(kSumThreads) void k_mse_chunk_summaries(
 
 // D: the ordered walk (one workgroup), then total (/) count.
 template <typename T>
-__global__ __launch_bounds__(kSumThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_mse_ordered_walk(
-    const T *__restrict__ sq, uint64_t n, T count, int policy, T *__restrict__ out,
-    unsigned long long *fault, const double *__restrict__ chunk_sum,
-    const ChunkSummary *__restrict__ summ, const SumScan<T> *__restrict__ runs, NodeGate gate)
+__device__ __forceinline__ void ordered_walk(const T *__restrict__ sq, uint64_t n, T count, int policy,
+                                             T *__restrict__ out, unsigned long long *fault,
+                                             const double *__restrict__ chunk_sum,
+                                             const ChunkSummary *__restrict__ summ,
+                                             const SumScan<T> *__restrict__ runs, const NodeGate &gate)
 {
     if (block_gate_closed(gate))
         return;
@@ -1606,6 +1639,18 @@ __global__ __launch_bounds__(kSumThreads) __attribute__((amdgpu_waves_per_eu(4))
     }
 }
 
+// A call of its own ends its program in this kernel (close).
+template <typename T>
+__global__ __launch_bounds__(kSumThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_mse_ordered_walk(
+    const T *__restrict__ sq, uint64_t n, T count, int policy, T *__restrict__ out,
+    unsigned long long *fault, const double *__restrict__ chunk_sum,
+    const ChunkSummary *__restrict__ summ, const SumScan<T> *__restrict__ runs, NodeGate gate,
+    ProgramClose close)
+{
+    ordered_walk<T>(sq, n, count, policy, out, fault, chunk_sum, summ, runs, gate);
+    program_close_block(close);
+}
+
 // Inputs of one chunk, one workgroup. Its waves form every difference and square in parallel into
 // LDS (each thread issues all of its loads before it computes, so the inputs arrive in one round
 // trip), find the first faulting Subtract or Multiply and estimate the mean; then the squares
@@ -1614,9 +1659,9 @@ __global__ __launch_bounds__(kSumThreads) __attribute__((amdgpu_waves_per_eu(4))
 // dependent adds, then a window for each doubling of the total: 17 us at 4096 f32, where one wave
 // adding all of the squares took 22.7.
 template <typename T>
-__global__ __launch_bounds__(kSumThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_mse_one(
-    const T *__restrict__ p, const T *__restrict__ t, uint64_t n, T count, int policy,
-    T *__restrict__ out, unsigned long long *fault, NodeGate gate)
+__device__ __forceinline__ void mse_one(const T *__restrict__ p, const T *__restrict__ t, uint64_t n,
+                                        T count, int policy, T *__restrict__ out,
+                                        unsigned long long *fault, const NodeGate &gate)
 {
     if (block_gate_closed(gate))
         return;
@@ -1691,6 +1736,15 @@ __global__ __launch_bounds__(kSumThreads) __attribute__((amdgpu_waves_per_eu(4))
     } else {
         *out = r;
     }
+}
+
+template <typename T>
+__global__ __launch_bounds__(kSumThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_mse_one(
+    const T *__restrict__ p, const T *__restrict__ t, uint64_t n, T count, int policy,
+    T *__restrict__ out, unsigned long long *fault, NodeGate gate, ProgramClose close)
+{
+    mse_one<T>(p, t, n, count, policy, out, fault, gate);
+    program_close_block(close);
 }
 
 // ------------------------------------------------------------- native compounds
@@ -2100,17 +2154,19 @@ static hipError_t mse_prepare_t(hipStream_t s, uint64_t n, const void *p, const 
         hipLaunchKernelGGL((k_mse_squares<T, true>), dim3(grid), dim3(kEwThreads), 0, s, (const T *)p, (const T *)t, m.squares, n, policy, m.quarter_sum, fault, gate);
     else
         hipLaunchKernelGGL((k_mse_squares<T, false>), dim3(grid), dim3(kEwThreads), 0, s, (const T *)p, (const T *)t, m.squares, n, policy, m.quarter_sum, fault, gate);
-    hipLaunchKernelGGL(k_mse_chunk_prefix, dim3(1), dim3(kPrefixThreads), 0, s, (const double *)m.quarter_sum, (uint64_t)m.chunks, m.chunk_sum, m.chunk_pre, gate);
-    hipLaunchKernelGGL((k_mse_chunk_summaries<T>), dim3((unsigned)m.chunks, kCands), dim3(kSumThreads), 0, s, (const T *)m.squares, n, (const unsigned long long *)fault, (const double *)m.chunk_sum, (const double *)m.chunk_pre, m.summ, m.runs, gate);
+    const bool prefix = m.chunks > kSumThreads;
+    if (prefix)
+        hipLaunchKernelGGL(k_mse_chunk_prefix, dim3(1), dim3(kPrefixThreads), 0, s, (const double *)m.quarter_sum, (uint64_t)m.chunks, m.chunk_sum, m.chunk_pre, gate);
+    hipLaunchKernelGGL((k_mse_chunk_summaries<T>), dim3((unsigned)m.chunks, kCands), dim3(kSumThreads), 0, s, (const T *)m.squares, n, (const unsigned long long *)fault, (const double *)m.quarter_sum, m.chunk_sum, prefix ? (const double *)m.chunk_pre : nullptr, m.summ, m.runs, gate);
     return hipGetLastError();
 }
 
 template <typename T>
 static hipError_t mse_walk_t(hipStream_t s, uint64_t n, void *scratch, T count, void *out,
-                             int policy, unsigned long long *fault, NodeGate gate)
+                             int policy, unsigned long long *fault, NodeGate gate, ProgramClose close)
 {
     const MseScratch<T> m(scratch, n);
-    hipLaunchKernelGGL((k_mse_ordered_walk<T>), dim3(1), dim3(kSumThreads), 0, s, (const T *)m.squares, n, count, policy, (T *)out, fault, (const double *)m.chunk_sum, (const ChunkSummary *)m.summ, (const SumScan<T> *)m.runs, gate);
+    hipLaunchKernelGGL((k_mse_ordered_walk<T>), dim3(1), dim3(kSumThreads), 0, s, (const T *)m.squares, n, count, policy, (T *)out, fault, (const double *)m.chunk_sum, (const ChunkSummary *)m.summ, (const SumScan<T> *)m.runs, gate, close);
     return hipGetLastError();
 }
 
@@ -2124,12 +2180,13 @@ hipError_t launch_mse_prepare(hipStream_t s, int dtype, uint64_t n, const void *
 }
 
 hipError_t launch_mse_walk(hipStream_t s, int dtype, uint64_t n, void *scratch, double count,
-                           void *out, int policy, unsigned long long *fault, NodeGate gate)
+                           void *out, int policy, unsigned long long *fault, NodeGate gate,
+                           ProgramClose close)
 {
     if (n == 0)
         return hipErrorInvalidValue;
-    return dtype == 0 ? mse_walk_t<float>(s, n, scratch, (float)count, out, policy, fault, gate)
-                      : mse_walk_t<double>(s, n, scratch, count, out, policy, fault, gate);
+    return dtype == 0 ? mse_walk_t<float>(s, n, scratch, (float)count, out, policy, fault, gate, close)
+                      : mse_walk_t<double>(s, n, scratch, count, out, policy, fault, gate, close);
 }
 
 uint64_t mse_one_max(int dtype)
@@ -2138,14 +2195,15 @@ uint64_t mse_one_max(int dtype)
 }
 
 hipError_t launch_mse_one(hipStream_t s, int dtype, uint64_t n, const void *p, const void *t,
-                          double count, void *out, int policy, unsigned long long *fault, NodeGate gate)
+                          double count, void *out, int policy, unsigned long long *fault, NodeGate gate,
+                          ProgramClose close)
 {
     if (n == 0 || n > mse_one_max(dtype))
         return hipErrorInvalidValue;
     if (dtype == 0)
-        hipLaunchKernelGGL((k_mse_one<float>), dim3(1), dim3(kSumThreads), 0, s, (const float *)p, (const float *)t, n, (float)count, policy, (float *)out, fault, gate);
+        hipLaunchKernelGGL((k_mse_one<float>), dim3(1), dim3(kSumThreads), 0, s, (const float *)p, (const float *)t, n, (float)count, policy, (float *)out, fault, gate, close);
     else
-        hipLaunchKernelGGL((k_mse_one<double>), dim3(1), dim3(kSumThreads), 0, s, (const double *)p, (const double *)t, n, count, policy, (double *)out, fault, gate);
+        hipLaunchKernelGGL((k_mse_one<double>), dim3(1), dim3(kSumThreads), 0, s, (const double *)p, (const double *)t, n, count, policy, (double *)out, fault, gate, close);
     return hipGetLastError();
 }
 

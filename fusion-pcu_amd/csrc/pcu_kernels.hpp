@@ -16,10 +16,9 @@ struct NodeGate {
 
 enum : int { kOpAdd = 0, kOpSub = 1, kOpMul = 2, kOpDiv = 3 };
 
-// The end of a program done by the launch of its last op (a MatMul that is the program's
+// The end of a program done by the launch of its last op (a MatMul or MSE that is the program's
 // only node, or a final SGD update) instead of a publication launch of its own: the n fault
-// words go to the coherent pinned
-// mirror host_words and are reset to `value`, the stage gate is opened, and then the
+// words go to the coherent pinned mirror host_words and are reset to `value`, the stage gate is opened, and then the
 // sequence number `seq` is stored to host_seq (the host waits on it). `ticket` (zero between
 // launches) counts the workgroups or waves that have finished when the last of them must do
 // it. words == nullptr: no.
@@ -117,12 +116,13 @@ size_t mse_scratch_bytes(int dtype, uint64_t n);
 hipError_t launch_mse_prepare(hipStream_t s, int dtype, uint64_t n, const void *p, const void *t,
                               void *scratch, int policy, unsigned long long *fault, NodeGate gate);
 hipError_t launch_mse_walk(hipStream_t s, int dtype, uint64_t n, void *scratch, double count,
-                           void *out, int policy, unsigned long long *fault, NodeGate gate);
+                           void *out, int policy, unsigned long long *fault, NodeGate gate,
+                           ProgramClose close = {});
 // Strict MSE of at most mse_one_max(dtype) elements in one launch of one workgroup, no scratch.
 uint64_t mse_one_max(int dtype);
 hipError_t launch_mse_one(hipStream_t s, int dtype, uint64_t n, const void *p, const void *t,
                           double count, void *out, int policy, unsigned long long *fault,
-                          NodeGate gate);
+                          NodeGate gate, ProgramClose close = {});
 
 // Strict MatMul scratch. Exponent words (generation << 32 | bias - minimum exponent) of
 // op(A) rows and op(B) columns; per output row, the first column whose cell has a product

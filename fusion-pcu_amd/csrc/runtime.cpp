@@ -456,8 +456,8 @@ pcu_status Ctx::read_words(size_t *used)
         // the next program (which then needs no opening launch), and stores this program's
         // sequence number last; the host spins on that word. Against a D2H copy and a stream
         // synchronization this saves the copy command and the runtime's wake-up. A program
-        // whose only node is a MatMul or a strict SGD update, or whose last launch is a
-        // strict SGD update on a small grid, had one of its own kernels do the same
+        // whose only node is a MatMul, a strict MSE or a strict SGD update, or whose last launch is
+        // a strict SGD update on a small grid, had one of its own kernels do the same
         // (closed_seq): a MatMul's tiny scan when no cell is suspect, else its replay.
         seq = ++pub_seq;
         if ((st = hip(launch_program_publish(stream, fault_words, *used, kNoFaultWord,
@@ -1164,6 +1164,11 @@ pcu_status Ctx::op_mse(int dtype, uint64_t n, const void *p, const void *t, void
     pcu_status st = add_node(NodeInfo{Prim::Mse, n, 0}, &word);
     if (st)
         return st;
+    if (implicit_program && nodes.size() == 1)
+        close_next = true; // a single pcu_strict_mse call: its last kernel ends the program
+    ProgramClose close;
+    if ((st = take_close(&close)))
+        return st;
     if (n <= mse_one_max(dtype)) {
         // One workgroup folds a small input in order; it overlaps the following work on the side
         // stream as the walk does.
@@ -1180,9 +1185,11 @@ pcu_status Ctx::op_mse(int dtype, uint64_t n, const void *p, const void *t, void
         }
         hipEvent_t t1 = timer_start(s);
         if ((st = hip(launch_mse_one(s, dtype, n, p, t, count_as(dtype, n), out, policy, word,
-                                     gate_for(word)), "strict_mse launch")))
+                                     gate_for(word), close), "strict_mse launch")))
             return st;
         timer_stop(PCU_KERNEL_MSE, t1, s);
+        if (close.words)
+            closed_seq = ++pub_seq;
         return PCU_OK;
     }
     void *sq = nullptr;
@@ -1207,10 +1214,12 @@ pcu_status Ctx::op_mse(int dtype, uint64_t n, const void *p, const void *t, void
         side_pending = true;
     }
     hipEvent_t t1 = timer_start(s);
-    if ((st = hip(launch_mse_walk(s, dtype, n, sq, count_as(dtype, n), out, policy, word, gate_for(word)),
+    if ((st = hip(launch_mse_walk(s, dtype, n, sq, count_as(dtype, n), out, policy, word, gate_for(word), close),
                   "strict_mse launch")))
         return st;
     timer_stop(PCU_KERNEL_MSE, t1, s);
+    if (close.words)
+        closed_seq = ++pub_seq;
     return PCU_OK;
 }
 
