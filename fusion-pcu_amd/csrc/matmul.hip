@@ -8,12 +8,14 @@
 // Four launches:
 //  1. prefilter   per-row minimum exponent of op(A) and per-column minimum exponent of
 //                 op(B) over finite nonzero entries (bandwidth-bound, ~2 reads of A and B).
-//  2. main        LDS-staged 128x128 output tile per 256-thread workgroup, 8x8 register
-//                 block per thread, k in order with separate v_mul/v_add. The epilogue
-//                 marks a cell suspect when its result is non-finite (the only trace an
-//                 invalid operand or an overflow leaves) or when the two exponents allow a
-//                 product small enough to be tiny (the only way an underflow can arise),
-//                 and keeps the first suspect cell with one atomicMin per wave.
+//  2. main        a tile kernel, k in order, products and sums rounded on their own: F32 on
+//                 128x128 tiles (matmul_mfma.hip) or 32x32 and 64x64 ones (matmul_mid.hip),
+//                 F64 on 64x64 (matmul_f64.hip) or 128x128 (matmul_valu.hip), whichever
+//                 the grid and K make the fastest. The epilogue marks a cell suspect when
+//                 its result is non-finite (the only trace an invalid operand or an
+//                 overflow leaves) or when the two exponents allow a product small enough
+//                 to be tiny (the only way an underflow can arise), and keeps the first
+//                 suspect cell with one atomicMin per wave.
 //  3. tiny scan   (IEEE policy, only when a cell is marked) a tiled pass over the tiles
 //                 the screen marks, finding the cells that can have a tiny product from the
 //                 smallest exponent sum over k (16-bit exponents, packed); see
@@ -23,7 +25,7 @@
 //                 flagged have their K products classified in parallel by a wave. Both stop
 //                 once the earliest fault found lies before the cells still to visit. The
 //                 fault-free path returns at once.
-// Small outputs (engine auto) take one fused launch instead (matmul_small.hip).
+// Few cells (engine auto) take one launch instead (matmul_small.hip).
 #include "pcu_device.hpp"
 #include "pcu_gemm_search.hpp"
 #include "pcu_gemm_stage.hpp"
@@ -34,7 +36,6 @@
 #pragma clang fp contract(off)
 
 namespace pcu {
-
 
 __device__ __forceinline__ int wave_min_i32(int v)
 {
@@ -962,11 +963,13 @@ bool matmul_bt_wanted(int dtype, uint64_t rows, uint64_t inner, uint64_t cols, b
     if (dtype != 0 && tl)
         return false;
     if (engine == kEngineAuto && gemm_small_wanted(dtype, rows, inner, cols))
-        return false; // the fused small-output launch reads B in place
+        return false; // the launch for few cells reads B in place
     // Whole 128 x 128 tiles filling at least one workgroup a CU: the copy measured 2-2.5%
     // faster there (NT 4096^3 1973 against 2021 us, 4096 x 1024 x 4096 510 against 521, TT
     // 4096^3 -2%), and 4.5-7% slower on the 64 x 64 tiles of smaller grids (1024^3 NT 57.1
-    // against 54.6 us).
+    // against 54.6 us). Where binary64 goes to 64 x 64 tiles there is no copy, also for the
+    // 128 x 128 tiles that check their sums there: RejectSubnormal NT 2048^3 took 784 us a call
+    // with it, 699 without.
     return rows % 128 == 0 && cols % 128 == 0 && (rows / 128) * (cols / 128) >= 256 &&
            inner * cols <= kBtMaxElems &&
            (dtype == 0 ? mid_tile_f32(rows, cols, inner, true) == MidTile::k128
@@ -1021,10 +1024,10 @@ static hipError_t strict_matmul_t(hipStream_t s, uint64_t M, uint64_t K, uint64_
     const bool reject = policy == kPolicyRejectSubnormal;
     int risk = policy != kPolicyAllowGradual;
     // Under RejectSubnormal the tile kernels check the partial sums of every tile that may
-    // meet a product below 2^sub_thr (binary64: on grids of at least 256 tiles of 128 x 128; when
-    // the scratch has the block words); a cell is then suspect only for a non-finite result, a possibly tiny
-    // product or a subnormal partial sum in its lane. Without the check every cell the
-    // exponents put below sub_thr is suspect and walked in full.
+    // meet a product below 2^sub_thr (binary64: on grids of at least 256 tiles of 128 x 128), when
+    // the scratch has the block words; a cell is then suspect only for a non-finite result, a
+    // possibly tiny product or a subnormal partial sum in its lane. Without the check every cell
+    // the exponents put below sub_thr is suspect and walked in full.
     const uint64_t tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
     const bool sum_check = reject && K > 0 && sc.sum_flag != nullptr && (f32 || tiles >= 256);
     int thr = reject && !sum_check ? sub_thr : tiny_thr;
