@@ -953,27 +953,21 @@ __global__ __launch_bounds__(256) void k_transpose(const T *__restrict__ X, T *_
 // Largest op(B) copied out (2^28 elements); larger ones are read in place.
 constexpr uint64_t kBtMaxElems = 1ull << 28;
 
-bool matmul_bt_wanted(int dtype, uint64_t rows, uint64_t inner, uint64_t cols, bool tl,
-                      bool tr, int engine)
+bool matmul_bt_wanted(int dtype, uint64_t rows, uint64_t inner, uint64_t cols, bool tr, int engine)
 {
-    if (!tr || (dtype == 0 && engine == kEngineValu) || inner == 0 || inner % 16 != 0)
-        return false;
-    // Binary64: NT 4096^3 4507 against 4692 us, 2048^3 610 against 674; TT measured no
-    // faster (4563 against 4523), its op(A) read-ahead path already hides the staging.
-    if (dtype != 0 && tl)
+    // Binary64 reads it in place: with the copy NT 4096^3 took 4727 to 4847 us a call against 4547
+    // to 4739, 4096 x 1024 x 4096 1306 against 1279, 4096 x 512 x 4096 717 against 702, and
+    // RejectSubnormal NT 2048^3 784 against 699.
+    if (dtype != 0 || !tr || engine == kEngineValu || inner == 0 || inner % 16 != 0)
         return false;
     if (engine == kEngineAuto && gemm_small_wanted(dtype, rows, inner, cols))
         return false; // the launch for few cells reads B in place
     // Whole 128 x 128 tiles filling at least one workgroup a CU: the copy measured 2-2.5%
     // faster there (NT 4096^3 1973 against 2021 us, 4096 x 1024 x 4096 510 against 521, TT
     // 4096^3 -2%), and 4.5-7% slower on the 64 x 64 tiles of smaller grids (1024^3 NT 57.1
-    // against 54.6 us). Where binary64 goes to 64 x 64 tiles there is no copy, also for the
-    // 128 x 128 tiles that check their sums there: RejectSubnormal NT 2048^3 took 784 us a call
-    // with it, 699 without.
+    // against 54.6 us).
     return rows % 128 == 0 && cols % 128 == 0 && (rows / 128) * (cols / 128) >= 256 &&
-           inner * cols <= kBtMaxElems &&
-           (dtype == 0 ? mid_tile_f32(rows, cols, inner, true) == MidTile::k128
-                       : !mid_wanted_f64(rows, cols, inner, tl, tr, false));
+           inner * cols <= kBtMaxElems && mid_tile_f32(rows, cols, inner, true) == MidTile::k128;
 }
 
 // The exponent screen of op(A) rows and op(B) columns, both jobs in one launch.
@@ -1107,17 +1101,7 @@ static hipError_t strict_matmul_t(hipStream_t s, uint64_t M, uint64_t K, uint64_
         (void)launch_gemm_mid_f64(s, false, m, n, k, ta, tb, (const double *)A, (const double *)B,
                                   (double *)C, sc.row_exp, sc.col_exp, thr, risk, sc.suspect, gate);
     } else {
-        // A transposed binary64 op(B) on a full grid goes to the tile kernel as its K x N
-        // copy, as for the matrix-core engine above.
-        const T *Bk = B;
-        bool tbk = tb;
-        if (!f32 && tb && sc.bt && aligned16(B)) {
-            const unsigned tiles = (unsigned)(((N + 63) / 64) * ((K + 63) / 64));
-            hipLaunchKernelGGL(k_transpose<T>, dim3(tiles), dim3(256), 0, s, B, (T *)sc.bt, n, k, gate);
-            Bk = (const T *)sc.bt;
-            tbk = false;
-        }
-        (void)launch_gemm_valu(s, f32 ? 0 : 1, m, n, k, ta, tbk, A, Bk, C, sc.row_exp, sc.col_exp, thr,
+        (void)launch_gemm_valu(s, f32 ? 0 : 1, m, n, k, ta, tb, A, B, C, sc.row_exp, sc.col_exp, thr,
                                risk, sc.suspect, sck, gate);
     }
     hipError_t e = hipGetLastError();

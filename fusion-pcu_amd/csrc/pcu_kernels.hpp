@@ -166,12 +166,11 @@ struct SumCheck {
     const short *tbl_a = nullptr, *tbl_b = nullptr;
     int a_xmajor = 0, b_xmajor = 0;
 };
-// Whether a strict MatMul (F32 on the matrix-core engine, or F64) runs its tile kernel on a
-// copy of a transposed op(B) stored K x N (grids of whole 128 x 128 tiles, K a multiple of
-// 16): the tile kernels load an untransposed op(B) straight into LDS but stage a transposed
-// one through registers.
-bool matmul_bt_wanted(int dtype, uint64_t rows, uint64_t inner, uint64_t cols, bool tl,
-                      bool tr, int engine);
+// Whether a strict MatMul (F32 on the matrix-core engine) runs its tile kernel on a copy of a
+// transposed op(B) stored K x N (grids of whole 128 x 128 tiles, K a multiple of 16): the tile
+// kernel loads an untransposed op(B) straight into LDS but stages a transposed one through
+// registers.
+bool matmul_bt_wanted(int dtype, uint64_t rows, uint64_t inner, uint64_t cols, bool tr, int engine);
 // `sum_flags`: the scratch also carries the partial-sum block words. The superslab tables
 // take a buffer of their own of slab_table_bytes() bytes (0: too large, none), or none.
 size_t matmul_scratch_bytes(uint64_t rows, uint64_t cols, bool sum_flags);
