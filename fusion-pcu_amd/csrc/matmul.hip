@@ -998,6 +998,30 @@ static void tiny_scan_dispatch(hipStream_t s, dim3 grid, const T *A, const T *B,
         hipLaunchKernelGGL((k_gemm_tiny_scan<T, TA, TB, false, false>), grid, dim3(256), 0, s, A, B, M, N, K, sc.row_exp, sc.col_exp, thr, sc.suspect, sc.row_flag, sc.flag_first, sc.gen, tb, gate, close);
 }
 
+// Whether the tile kernels of a RejectSubnormal MatMul check the partial sums of every tile that
+// may meet a product below 2^sub_thr: F32, and F64 on grids of at least 256 tiles of 128 x 128.
+static bool sum_check_wanted(int dtype, uint64_t M, uint64_t K, uint64_t N, int policy, bool sum_flags)
+{
+    return policy == kPolicyRejectSubnormal && K > 0 && sum_flags &&
+           (dtype == 0 || ((M + BM - 1) / BM) * ((N + BN - 1) / BN) >= 256);
+}
+
+int strict_matmul_tile(int dtype, uint64_t rows, uint64_t inner, uint64_t cols, bool ta, bool tb,
+                       int policy, int engine, bool sum_flags)
+{
+    if (engine == kEngineAuto && inner > 0 && gemm_small_wanted(dtype, rows, inner, cols))
+        return 16;
+    if (dtype == 0 && engine != kEngineValu) {
+        const MidTile t = mfma_tile_f32(rows, cols, inner, ta, tb);
+        return t == MidTile::k32 ? 32 : (t == MidTile::k64 ? 64 : 128);
+    }
+    // (The binary64 64 x 64 tiles have no partial-sum check.)
+    return dtype != 0 && !sum_check_wanted(dtype, rows, inner, cols, policy, sum_flags) &&
+                   mid_wanted_f64(rows, cols, inner, ta, tb, false)
+               ? 64
+               : 128;
+}
+
 template <typename T>
 static hipError_t strict_matmul_t(hipStream_t s, uint64_t M, uint64_t K, uint64_t N, bool ta,
                                   bool tb, const T *A, const T *B, T *C, int policy,
@@ -1017,18 +1041,16 @@ static hipError_t strict_matmul_t(hipStream_t s, uint64_t M, uint64_t K, uint64_
     const int tiny_thr = f32 ? -126 : -1022, sub_thr = f32 ? -103 : -970;
     const bool reject = policy == kPolicyRejectSubnormal;
     int risk = policy != kPolicyAllowGradual;
-    // Under RejectSubnormal the tile kernels check the partial sums of every tile that may
-    // meet a product below 2^sub_thr (binary64: on grids of at least 256 tiles of 128 x 128), when
-    // the scratch has the block words; a cell is then suspect only for a non-finite result, a
-    // possibly tiny product or a subnormal partial sum in its lane. Without the check every cell
-    // the exponents put below sub_thr is suspect and walked in full.
-    const uint64_t tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-    const bool sum_check = reject && K > 0 && sc.sum_flag != nullptr && (f32 || tiles >= 256);
+    // With the tile kernels' partial-sum check a cell is suspect only for a non-finite result, a
+    // possibly tiny product or a subnormal partial sum in its lane. Without it every cell the
+    // exponents put below sub_thr is suspect and walked in full.
+    const bool sum_check = sum_check_wanted(f32 ? 0 : 1, M, K, N, policy, sc.sum_flag != nullptr);
     int thr = reject && !sum_check ? sub_thr : tiny_thr;
     SumCheck sck = sum_check ? SumCheck{sc.sum_flag, sc.gen, sc.flag_cols, sub_thr} : SumCheck{};
     if (ev)
         (void)hipEventRecord(ev[0], s);
-    if (engine == kEngineAuto && K > 0 && gemm_small_wanted(f32 ? 0 : 1, M, K, N)) {
+    const int tile = strict_matmul_tile(f32 ? 0 : 1, M, K, N, ta, tb, policy, engine, sc.sum_flag != nullptr);
+    if (tile == 16) {
         // A program's first node opens the program before any block can record a fault.
         if (open.words)
             hipLaunchKernelGGL(k_matmul_open, dim3(1), dim3(256), 0, s, sc.suspect, open);
@@ -1096,8 +1118,7 @@ static hipError_t strict_matmul_t(hipStream_t s, uint64_t M, uint64_t K, uint64_
         }
         (void)launch_gemm_mfma_f32(s, m, n, k, ta, tbt, (const float *)A, Bt, (float *)C,
                                    sc.row_exp, sc.col_exp, thr, risk, sc.suspect, sck, gate, epi, epi_done);
-    } else if (!f32 && sck.flag == nullptr && mid_wanted_f64(M, N, K, ta, tb, false)) {
-        // (The 64 x 64 tiles have no partial-sum check.)
+    } else if (!f32 && tile == 64) {
         (void)launch_gemm_mid_f64(s, false, m, n, k, ta, tb, (const double *)A, (const double *)B,
                                   (double *)C, sc.row_exp, sc.col_exp, thr, risk, sc.suspect, gate);
     } else {
@@ -1134,6 +1155,13 @@ static hipError_t strict_matmul_t(hipStream_t s, uint64_t M, uint64_t K, uint64_
     if (ev)
         (void)hipEventRecord(ev[3], s);
     return hipGetLastError();
+}
+
+// strict_matmul_tile of a call that has all of its scratch, for tests of the choice.
+extern "C" int pcu_internal_strict_matmul_tile(int dtype, uint64_t rows, uint64_t inner,
+                                               uint64_t cols, int ta, int tb, int policy, int engine)
+{
+    return strict_matmul_tile(dtype, rows, inner, cols, ta != 0, tb != 0, policy, engine, true);
 }
 
 hipError_t launch_strict_matmul(hipStream_t s, int dtype, uint64_t rows, uint64_t inner,

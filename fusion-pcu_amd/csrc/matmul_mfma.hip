@@ -649,6 +649,13 @@ static void mfma_launch(hipStream_t s, int M, int N, int K, bool ta, bool tb, co
 // 32 x 32, a 256 x 128 tile, 4-wave tiles of 128 x 64 and 64 x 64, and BK = 32 (which
 // spills with the pinned slab).
 using GemmCfg = MfmaCfg<4, 2, 1, 2, 16, 4>;
+
+MidTile mfma_tile_f32(uint64_t M, uint64_t N, uint64_t K, bool ta, bool tb)
+{
+    const bool whole = M % GemmCfg::BM == 0 && N % GemmCfg::BN == 0 && K % GemmCfg::BK == 0;
+    return mid_fits_f32(M, N, K, ta, tb) ? mid_tile_f32(M, N, K, whole) : MidTile::k128;
+}
+
 hipError_t launch_gemm_mfma_f32(hipStream_t s, int M, int N, int K, bool ta, bool tb,
                                 const float *A, const float *B, float *C,
                                 const unsigned long long *row_exp,
@@ -656,9 +663,8 @@ hipError_t launch_gemm_mfma_f32(hipStream_t s, int M, int N, int K, bool ta, boo
                                 unsigned long long *suspect, SumCheck sck, NodeGate gate,
                                 const GemmEpilogue *epi, bool *epi_done)
 {
-    const bool whole = M % GemmCfg::BM == 0 && N % GemmCfg::BN == 0 && K % GemmCfg::BK == 0;
-    const MidTile tile = mid_tile_f32((uint64_t)M, (uint64_t)N, (uint64_t)K, whole);
-    if (tile != MidTile::k128 && mid_fits_f32((uint64_t)M, (uint64_t)N, (uint64_t)K, ta, tb))
+    const MidTile tile = mfma_tile_f32((uint64_t)M, (uint64_t)N, (uint64_t)K, ta, tb);
+    if (tile != MidTile::k128)
         return launch_gemm_mid_f32(s, tile, M, N, K, ta, tb, A, B, C, row_exp, col_exp, thr, risk, suspect, sck, gate);
     mfma_launch<GemmCfg>(s, M, N, K, ta, tb, A, B, C, row_exp, col_exp, thr, risk, suspect, sck, gate, epi, epi_done);
     return hipGetLastError();

@@ -200,6 +200,8 @@ MidTile mid_tile_f32(uint64_t M, uint64_t N, uint64_t K, bool whole);
 double mid_time_f32(uint64_t M, uint64_t N, uint64_t K); // the chosen tile's estimate, in us
 // Whether matmul_mid.hip can address the operands.
 bool mid_fits_f32(uint64_t M, uint64_t N, uint64_t K, bool ta, bool tb);
+// The tile that launch_gemm_mfma_f32 takes.
+MidTile mfma_tile_f32(uint64_t M, uint64_t N, uint64_t K, bool ta, bool tb);
 hipError_t launch_gemm_mid_f32(hipStream_t s, MidTile tile, int M, int N, int K, bool ta, bool tb,
                                const float *A, const float *B, float *C,
                                const unsigned long long *row_exp, const unsigned long long *col_exp,
@@ -226,6 +228,11 @@ hipError_t launch_gemm_small(hipStream_t s, int dtype, int M, int N, int K, bool
                              const void *A, const void *B, void *C, int thr, int risk, int policy,
                              unsigned long long *fault, NodeGate gate, ProgramClose close,
                              bool *closed);
+
+// The kernel that a strict MatMul takes, by the side of its output tile: 16 (the one launch of
+// matmul_small.hip), 32, 64 or 128. `sum_flags`: the scratch carries the partial-sum block words.
+int strict_matmul_tile(int dtype, uint64_t rows, uint64_t inner, uint64_t cols, bool ta, bool tb,
+                       int policy, int engine, bool sum_flags);
 
 // C[rows x cols] = op(A) * op(B), k ascending, each multiply and add rounded on its own.
 // Every kernel of the op skips its work once `gate` shows that an earlier program node

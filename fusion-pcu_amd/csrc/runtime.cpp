@@ -1591,12 +1591,12 @@ pcu_status pcu_ctx_set_matmul_engine(pcu_ctx *ctx, pcu_matmul_engine engine)
         return bad_ctx();
     if (engine < PCU_MATMUL_AUTO || engine > PCU_MATMUL_MFMA_PRODUCTS)
         return PCU_ERR_ARGUMENT;
-    Ctx *c = reinterpret_cast<Ctx *>(ctx);
-    if (engine == PCU_MATMUL_MFMA_PRODUCTS)
-        engine = PCU_MATMUL_AUTO; // F64 has no K=1 matrix form: AUTO is the same choice
-    c->matmul_engine = (int)engine;
+    reinterpret_cast<Ctx *>(ctx)->matmul_engine = (int)engine;
     return PCU_OK;
 }
+
+// The engine a context's MatMuls run with, for tests.
+int pcu_internal_matmul_engine(const pcu_ctx *ctx) { return reinterpret_cast<const Ctx *>(ctx)->matmul_engine; }
 
 pcu_status pcu_profile_enable(pcu_ctx *ctx, int on)
 {

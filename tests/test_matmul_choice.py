@@ -1,0 +1,39 @@
+"""Which kernel a strict MatMul takes, by the side of its output tile (16: the one launch of few
+cells). The choice is made on the host, so it is checked without a GPU."""
+import ctypes
+
+import pytest
+
+AUTO, VALU, MFMA = 0, 1, 2
+IEEE, REJECT, GRADUAL = 0, 1, 2
+
+
+@pytest.fixture(scope="module")
+def tile(pcu_pkg):
+    f = pcu_pkg.lib().pcu_internal_strict_matmul_tile
+    f.argtypes = [ctypes.c_int] + 3 * [ctypes.c_uint64] + 4 * [ctypes.c_int]
+    f.restype = ctypes.c_int
+
+    def call(dtype, m, k, n, tl=False, tr=False, policy=IEEE, engine=AUTO):
+        return f({"f32": 0, "f64": 1}[dtype], m, k, n, int(tl), int(tr), policy, engine)
+
+    return call
+
+
+@pytest.mark.parametrize("engine", [VALU, MFMA])
+def test_a_chosen_engine_always_takes_the_tile_kernels(tile, engine):
+    for dtype in ("f32", "f64"):
+        for m in (1, 16, 64, 256, 1000, 4096):
+            for k in (1, 8, 64, 256, 4096):
+                for n in (1, 64, 512, 4096):
+                    assert tile(dtype, m, k, n, engine=engine) in (32, 64, 128)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,engine", [("auto", AUTO), ("valu", VALU), ("mfma_products", MFMA)])
+def test_a_context_runs_with_the_engine_it_was_given(pcu_pkg, name, engine):
+    f = pcu_pkg.lib().pcu_internal_matmul_engine
+    f.argtypes, f.restype = [ctypes.c_void_p], ctypes.c_int
+    with pcu_pkg.Context(0) as ctx:
+        ctx.set_matmul_engine(name)
+        assert f(ctx.handle) == engine
