@@ -96,11 +96,12 @@ double mid_time_f32(uint64_t M, uint64_t N, uint64_t K)
 }
 
 // A lane's byte offset from its operand's tile must fit 32 bits: 64 rows of the stored matrix
-// and one slab.
+// and one slab. And a launch holds fewer than 2^32 threads: 32 x 32 tiles take 256 each (an
+// output of 2^34 cells reaches that; 128 x 128 tiles take an eighth of the threads).
 bool mid_fits_f32(uint64_t M, uint64_t N, uint64_t K, bool ta, bool tb)
 {
     const uint64_t lda = ta ? M : K, ldb = tb ? K : N;
-    return lda < (1u << 24) && ldb < (1u << 24);
+    return lda < (1u << 24) && ldb < (1u << 24) && ((M + 31) / 32) * ((N + 31) / 32) <= UINT32_MAX / 256;
 }
 
 hipError_t launch_gemm_mid_f32(hipStream_t s, MidTile tile, int M, int N, int K, bool ta, bool tb,

@@ -332,6 +332,9 @@ bool gemm_small_wanted(int dtype, uint64_t rows, uint64_t inner, uint64_t cols)
         return (double)((tiles + kGfx950Cus - 1) / kGfx950Cus);
     };
     const double k = (double)inner / 1024.0, c = per_cu(16);
+    // A launch holds fewer than 2^32 threads: one a cell.
+    if (((rows + 15) / 16) * ((cols + 15) / 16) > UINT32_MAX / 256)
+        return false;
     if (dtype == 0)
         return (c <= 2 ? 9 + 3 * c : 6.1 * c) * k + 3 < mid_time_f32(rows, cols, inner) + 15;
     const double c64 = per_cu(64);

@@ -29,6 +29,18 @@ def test_a_chosen_engine_always_takes_the_tile_kernels(tile, engine):
                     assert tile(dtype, m, k, n, engine=engine) in (32, 64, 128)
 
 
+def test_no_choice_launches_more_threads_than_a_grid_holds(tile):
+    """A launch holds fewer than 2^32 threads. The one-launch kernel takes one thread a cell, the
+    32 x 32 and 64 x 64 binary32 tiles one for each 4 and 8 cells; outputs of that size fit the
+    device's memory and run on 128 x 128 tiles."""
+    threads = {16: 1 / 1, 32: 1 / 4, 64: 1 / 8, 128: 1 / 32}
+    for m, k, n in ((65536, 8, 65536), (65537, 15, 70001), (1 << 20, 1, 1 << 14), (131073, 5000, 131073),
+                    (185400, 5000, 185400), (1 << 18, 16, 1 << 16)):
+        for policy in (IEEE, REJECT, GRADUAL):
+            for dtype in ("f32", "f64"):
+                assert m * n * threads[tile(dtype, m, k, n, policy=policy)] < 2 ** 32, (dtype, m, k, n)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("name,engine", [("auto", AUTO), ("valu", VALU), ("mfma_products", MFMA)])
 def test_a_context_runs_with_the_engine_it_was_given(pcu_pkg, name, engine):
