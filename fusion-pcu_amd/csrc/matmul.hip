@@ -1056,7 +1056,7 @@ static hipError_t strict_matmul_t(hipStream_t s, uint64_t M, uint64_t K, uint64_
             hipLaunchKernelGGL(k_matmul_open, dim3(1), dim3(256), 0, s, sc.suspect, open);
         if (ev)
             (void)hipEventRecord(ev[1], s);
-        // The small kernel walks every cell its exponents mark (no partial-sum check).
+        // The small kernel searches every cell its exponents mark (no partial-sum check).
         const hipError_t e = launch_gemm_small(s, f32 ? 0 : 1, (int)M, (int)N, (int)K, ta, tb, A, B, C,
                                                reject ? sub_thr : tiny_thr, risk, policy, fault, gate,
                                                close, closed);

@@ -3,10 +3,10 @@
 // Each 256-thread workgroup owns 16 x 16 cells (wave w rows 4 w .. 4 w + 3, lane row r of 16
 // lanes one of them) and walks k in chunks of 4 KiB a row, staged in LDS with k contiguous. A
 // block sees all of k for its rows and columns, so it folds their smallest exponents as it
-// stages them and screens its own cells; suspect cells (a non-finite result, or exponents that
-// allow a tiny product) are walked in cell order with the exact search, a wave per cell,
-// stopping once the block's earliest fault lies before the cells left, and that fault is
-// folded into the node's word with atomicMin, so the word ends with the MatMul's first fault.
+// stages them and screens its own cells; the suspect cells (a non-finite result, or exponents that
+// allow a tiny product) are searched, each by its own lane, until the block's earliest fault lies
+// before the cells left, and that fault is folded into the node's word with atomicMin, so the word
+// ends with the MatMul's first fault.
 //
 // What bounds it: the chain of sums. A wave's add that depends on the one two instructions
 // before it issues 14 cycles after it with one or two waves a SIMD, so a cell cannot take less
@@ -18,6 +18,7 @@
 #include "pcu_gemm_search.hpp"
 #include "pcu_kernels.hpp"
 
+#include <limits.h>
 #include <utility>
 
 #pragma clang fp contract(off)
@@ -58,6 +59,63 @@ template <int N, class F> __device__ __forceinline__ void each(F &&f)
     each_of(f, std::make_integer_sequence<int, N>{});
 }
 
+// Stands for a zero operand in the search's stages where only tiny products are looked for: its
+// product with any operand is far above the smallest normal.
+template <typename T> constexpr T kZeroStand = sizeof(T) == 4 ? (T)0x1p100 : (T)0x1p1000;
+
+// The first fault of one cell in the kc k of a staged chunk (as: its row, bs: its column, zeros or
+// their stands up to the next 16 k), kNoFault when there is none or `on` is false. `step`: the
+// first k's Multiply. ADDS: t carries the cell's sum from chunk to chunk, and every product and
+// sum is checked; else only for a tiny product, with zeros staged as kZeroStand. Sixteen k at a
+// time, whose smallest product (and sum, where subnormal ones are rejected) says whether they go
+// through the exact classifiers: a compare for each k would have cost three times the products.
+template <typename T, bool ADDS>
+__device__ __forceinline__ uint64_t chunk_first_fault(const T *as, const T *bs, int kc, T &t, bool on,
+                                                      uint64_t step, int policy)
+{
+    constexpr int P = 16 / (int)sizeof(T), U = 16;
+    const bool reject_sub = policy == kPolicyRejectSubnormal;
+    for (int k = 0; k < kc; k += U) {
+        uint4 qa[U / P], qb[U / P];
+#pragma unroll
+        for (int g = 0; g < U / P; g++) {
+            qa[g] = *reinterpret_cast<const uint4 *>(as + k + P * g);
+            qb[g] = *reinterpret_cast<const uint4 *>(bs + k + P * g);
+        }
+        const T *a = reinterpret_cast<const T *>(qa), *b = reinterpret_cast<const T *>(qb);
+        T n = t, least = (T)1;
+#pragma unroll
+        for (int c = 0; c < U; c++) {
+            const T p = a[c] * b[c];
+            least = __builtin_elementwise_min(least, __builtin_elementwise_abs(p));
+            if (ADDS) {
+                n = n + p;
+                if (reject_sub)
+                    least = __builtin_elementwise_min(least, __builtin_elementwise_abs(n));
+            }
+        }
+        // (A non-finite sum stays so, and a NaN is no minimum.)
+        const bool look = (policy != kPolicyAllowGradual && at_most_min_normal(least)) || (ADDS && !finite_bits(n));
+        if (on && look) {
+#pragma unroll 1
+            for (int c = 0; c < U; c++) {
+                const T x = as[k + c], y = bs[k + c], p = x * y;
+                uint32_t kind = classify_mul(x, y, p, policy);
+                if (kind != kOk && (ADDS || kind == kUnderflow))
+                    return pack_fault(step + 2 * (uint64_t)(k + c), kind);
+                if (ADDS) {
+                    kind = classify_add(t, p, t + p, policy);
+                    if (kind != kOk)
+                        return pack_fault(step + 2 * (uint64_t)(k + c) + 1, kind);
+                    t = t + p;
+                }
+            }
+        }
+        t = n;
+    }
+    return kNoFault;
+}
+
 // VA, VB: every row of the stored matrix is 16-byte aligned.
 template <typename T, bool TA, bool TB, bool VA, bool VB>
 __global__ __launch_bounds__(256, 2) void k_strict_gemm_small(
@@ -76,9 +134,8 @@ __global__ __launch_bounds__(256, 2) void k_strict_gemm_small(
     __shared__ __align__(16) T Bs[2][16][BKP];
     __shared__ uint32_t rkey[16], ckey[16];
     __shared__ unsigned long long best; // this block's earliest fault
-    __shared__ int n_cand, wave_cnt[4];
-    __shared__ short cand[256];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    __shared__ int first_sus;           // its first suspect cell, and whether that is finite
+    const int tid = threadIdx.x;
     const int ty = tid >> 4, tx = tid & 15; // the thread's cell
     const int tiles_n = (N + 15) / 16;
     const int m0 = (int)(blockIdx.x / tiles_n) * 16, n0 = (int)(blockIdx.x % tiles_n) * 16;
@@ -86,8 +143,10 @@ __global__ __launch_bounds__(256, 2) void k_strict_gemm_small(
         rkey[tid] = 0xffffffffu;
         ckey[tid] = 0xffffffffu;
     }
-    if (tid == 0)
+    if (tid == 0) {
         best = kNoFault;
+        first_sus = INT_MAX;
+    }
     // A thread stages runs of P k of one row of op(A) and one column of op(B), 16 P k apart, in
     // an order that keeps each global access coalesced: 16 threads along k where k is
     // contiguous, else 16 threads along the rows (columns).
@@ -134,15 +193,17 @@ __global__ __launch_bounds__(256, 2) void k_strict_gemm_small(
         }
     };
     uint32_t amin = 0xffffffffu, bmin = 0xffffffffu;
-    auto stash_chunk = [&](int buf) __attribute__((always_inline)) {
+    // STAND: zeros are staged as kZeroStand.
+    auto stash_chunk = [&](int buf, auto stand_c) __attribute__((always_inline)) {
+        constexpr bool STAND = decltype(stand_c)::value;
 #pragma unroll
         for (int j = 0; j < L; j++) {
             uint4 qa, qb;
             T *ea = reinterpret_cast<T *>(&qa), *eb = reinterpret_cast<T *>(&qb);
 #pragma unroll
             for (int c = 0; c < P; c++) {
-                ea[c] = va[j][c];
-                eb[c] = vb[j][c];
+                ea[c] = STAND && is_zero(va[j][c]) ? kZeroStand<T> : va[j][c];
+                eb[c] = STAND && is_zero(vb[j][c]) ? kZeroStand<T> : vb[j][c];
                 const uint32_t x = exp_key(va[j][c]), y = exp_key(vb[j][c]);
                 amin = x < amin ? x : amin;
                 bmin = y < bmin ? y : bmin;
@@ -225,7 +286,7 @@ __global__ __launch_bounds__(256, 2) void k_strict_gemm_small(
         });
     };
     fetch_chunk(0);
-    stash_chunk(0);
+    stash_chunk(0, std::false_type{});
     __syncthreads();
     for (int k0 = 0, buf = 0; k0 < K; k0 += BK, buf ^= 1) {
         const int kc = K - k0 < BK ? K - k0 : BK;
@@ -237,7 +298,7 @@ __global__ __launch_bounds__(256, 2) void k_strict_gemm_small(
         if (kc % BL != 0)
             part_block(&As[buf][ty][kc / BL * BL], &Bs[buf][tx][kc / BL * BL], kc % BL);
         if (next) {
-            stash_chunk(buf ^ 1);
+            stash_chunk(buf ^ 1, std::false_type{});
             __syncthreads();
         }
     }
@@ -252,36 +313,61 @@ __global__ __launch_bounds__(256, 2) void k_strict_gemm_small(
         C[(size_t)crow * N + ccol] = acc;
         sus = !finite_bits(acc) || (risk && key_exp<T>(rkey[ty]) + key_exp<T>(ckey[tx]) < thr);
     }
-    // The block's suspect cells in cell order (tile index ty * 16 + tx grows with it).
-    const uint64_t mask = __ballot(sus);
-    if (lane == 0)
-        wave_cnt[wave] = __popcll(mask);
-    __syncthreads();
-    int before = 0;
-    for (int w = 0; w < wave; w++)
-        before += wave_cnt[w];
-    if (sus)
-        cand[before + __popcll(mask & ((1ull << lane) - 1))] = (short)tid;
-    if (tid == 0)
-        n_cand = wave_cnt[0] + wave_cnt[1] + wave_cnt[2] + wave_cnt[3];
-    __syncthreads();
-    const int nc = n_cand;
-    if (nc == 0) {
+    if (!__syncthreads_or(sus)) {
         program_close_block(close);
         return;
     }
-    for (int j = wave; j < nc; j += 4) {
-        const int i = cand[j];
-        const uint64_t cell = (uint64_t)(m0 + (i >> 4)) * N + n0 + (i & 15);
-        const uint64_t bw = wave_uniform_u64(__atomic_load_n(&best, __ATOMIC_RELAXED));
-        if (bw != kNoFault && ((bw >> 3) / 2) / (uint64_t)K < cell)
-            break; // cells only grow along the list
-        const uint64_t w = cell_first_fault(A, B, (uint64_t)M, (uint64_t)N, (uint64_t)K, (int)TA,
-                                            (int)TB, cell, policy, true);
-        if (w != kNoFault && lane == 0)
-            atomicMin(&best, (unsigned long long)w);
-    }
+    // The search. A block whose first suspect cell is not finite has its first fault there (such a
+    // result comes of a fault), and a wave walks that cell alone.
+    const uint64_t mask = __ballot(sus);
+    if (mask != 0 && (tid & 63) == __ffsll((long long)mask) - 1)
+        atomicMin(&first_sus, 2 * tid + (int)finite_bits(acc));
     __syncthreads();
+    if (!(first_sus & 1)) {
+        const int i = first_sus >> 1;
+        if (tid < 64) {
+            const uint64_t w = cell_first_fault(A, B, (uint64_t)M, (uint64_t)N, (uint64_t)K, (int)TA, (int)TB,
+                                                (uint64_t)(m0 + (i >> 4)) * N + n0 + (i & 15), policy, true);
+            if (w != kNoFault && tid == 0) {
+                atomicMin(fault, (unsigned long long)w);
+                gate_record(gate);
+            }
+        }
+        program_close_block(close);
+        return;
+    }
+    // Else every suspect cell's lane walks its own k again, the chunks staged as before, until its
+    // first fault. A finite cell (and so each of its sums) can only fault in a tiny product, unless
+    // subnormal sums are rejected; a block of such cells forms no sums. One lane a cell, so a block
+    // whose every cell is suspect costs about as much again as the products did: 64 x 4096 x 1024
+    // binary32 124 us, 53 clean, where a wave for each cell, 64 k at a time, took 5000.
+    const uint64_t first_step = ((uint64_t)crow * N + ccol) * (uint64_t)K * 2; // of the lane's cell
+    const bool adds = policy == kPolicyRejectSubnormal || __syncthreads_or(sus && !finite_bits(acc));
+    T t = (T)0;
+    for (int k0 = 0; k0 < K; k0 += BK) {
+        if (!adds || K > BK) { // a single chunk still stands in its stage
+            fetch_chunk(k0);
+            if (adds)
+                stash_chunk(0, std::false_type{});
+            else
+                stash_chunk(0, std::true_type{});
+            __syncthreads();
+        }
+        uint64_t key = kNoFault;
+        if (__ballot(sus)) {
+            const int kc = K - k0 < BK ? K - k0 : BK;
+            const uint64_t step = first_step + 2 * (uint64_t)k0;
+            key = adds ? chunk_first_fault<T, true>(&As[0][ty][0], &Bs[0][tx][0], kc, t, sus, step, policy)
+                       : chunk_first_fault<T, false>(&As[0][ty][0], &Bs[0][tx][0], kc, t, sus, step, policy);
+            if (key != kNoFault)
+                atomicMin(&best, (unsigned long long)key);
+        }
+        __syncthreads();
+        // Cells after a cell with a fault need no walk.
+        sus = sus && key == kNoFault && pack_fault(first_step, 0) < best;
+        if (!__syncthreads_or(sus))
+            break;
+    }
     if (tid == 0 && best != kNoFault) {
         atomicMin(fault, best);
         gate_record(gate);

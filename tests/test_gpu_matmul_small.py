@@ -84,3 +84,78 @@ def test_first_fault_and_screen(ctx, pcu_pkg, dtype, layout, policy):
                 if special == info.smallest_subnormal:
                     av[m - 1, :] = info.smallest_subnormal  # a whole row below the smallest normal
                     _check(ctx, pcu_pkg, a, b, tl, tr, policy)
+
+
+@DTYPES
+@LAYOUTS
+@pytest.mark.parametrize("policy", [0, 1, 2])
+def test_search_of_many_suspect_cells(ctx, pcu_pkg, dtype, layout, policy):
+    """Every cell marked by the screen and clean; exact subnormal products everywhere (a fault
+    under RejectSubnormal only) with an inexact one after them; subnormal partial sums; and faults
+    of every kind in several workgroups at once, of which the lowest cell, k and step is the one."""
+    tl, tr = layout
+    rng = np.random.default_rng(23)
+    f32 = dtype == np.float32
+    low = dtype(2.0 ** (-120 if f32 else -1016))
+    info = np.finfo(dtype)
+    for m, k, n in ((33, 130, 50), (100, 40, 90), (18, 523, 34)):
+        def base():
+            a, b = _operands(rng, m, k, n, tl, tr, dtype)
+            av, bv = (a.T if tl else a), (b.T if tr else b)
+            av[:, 0], bv[0, :] = low, 1
+            av[:, 1], bv[1, :] = 1, dtype(2.0 ** -20)
+            return a, b, av, bv
+        a, b, av, bv = base()
+        _check(ctx, pcu_pkg, a, b, tl, tr, policy)
+        av[:, 1], bv[1, :] = low, dtype(2.0 ** -9)
+        _check(ctx, pcu_pkg, a, b, tl, tr, policy)
+        av[m - 2, k - 1], bv[k - 1, n - 3] = low * dtype(1.3), dtype(1.3 * 2.0 ** -30)
+        _check(ctx, pcu_pkg, a, b, tl, tr, policy)
+        a, b, av, bv = base()
+        # A sum that cancels to a subnormal at k 3 of one cell, its products normal.
+        av[m - 1, :4], bv[:4, n - 1] = 0, 1
+        av[m - 1, 2], av[m - 1, 3] = info.tiny * dtype(1.5), -info.tiny
+        _check(ctx, pcu_pkg, a, b, tl, tr, policy)
+        for _ in range(6):
+            a, b, av, bv = base()
+            for special in rng.choice(6, 4, replace=False):
+                i, j, kk = rng.integers(m), rng.integers(n), rng.integers(2, k - 2)
+                if special == 0:
+                    av[i, kk] = np.nan
+                elif special == 1:
+                    bv[kk, j] = -np.inf
+                elif special == 2:
+                    av[i, kk], bv[kk, j] = info.max, 2
+                elif special == 3:  # the Add overflows, not the Multiply
+                    av[i, kk:kk + 2], bv[kk:kk + 2, j] = info.max, dtype(0.75)
+                elif special == 4:
+                    av[i, kk], bv[kk, j] = low * dtype(1.3), dtype(1.7 * 2.0 ** -30)
+                else:
+                    av[i, kk], bv[kk, j] = info.smallest_subnormal, dtype(0.5)
+            _check(ctx, pcu_pkg, a, b, tl, tr, policy)
+
+
+@DTYPES
+@pytest.mark.parametrize("policy", [0, 1])
+def test_marked_cells_cost_a_bounded_multiple_of_the_call(ctx, pcu_pkg, dtype, policy):
+    """A call whose every cell the screen marks, without a fault, takes no more than 8 times the
+    clean call's time (a wave for each marked cell took 40 to 90 times as long)."""
+    import time
+
+    rng = np.random.default_rng(2)
+    m, k, n = 64, 2048, 64
+    a, b = _operands(rng, m, k, n, False, False, dtype)
+    clean = ctx.upload(a), ctx.upload(b)
+    a[:, 0], b[0, :] = dtype(2.0 ** (-120 if dtype == np.float32 else -1016)), 1
+    a[:, 1], b[1, :] = 1, dtype(2.0 ** -20)
+    marked = ctx.upload(a), ctx.upload(b)
+    out = ctx.empty((m, n), dtype)
+    best = []
+    for ops in (clean, marked):
+        times = []
+        for _ in range(12):
+            t = time.perf_counter()
+            ctx.strict_matmul(ops[0], ops[1], False, False, policy, out=out)
+            times.append(time.perf_counter() - t)
+        best.append(min(times[2:]))
+    assert best[1] < 8 * best[0], best
