@@ -1,7 +1,7 @@
 // Strict F32/F64 MatMul of few cells: one launch does the whole MatMul, one cell a lane.
 //
 // Each 256-thread workgroup owns 16 x 16 cells (wave w rows 4 w .. 4 w + 3, lane row r of 16
-// lanes one of them) and walks k in chunks of 4 KiB a row, staged in LDS with k contiguous. A
+// lanes one of them) and walks k in chunks of 1 KiB a row, staged in LDS with k contiguous. A
 // block sees all of k for its rows and columns, so it folds their smallest exponents as it
 // stages them and screens its own cells; the suspect cells (a non-finite result, or exponents that
 // allow a tiny product) are searched, each by its own lane, until the block's earliest fault lies
@@ -14,6 +14,11 @@
 // 32), each lane row of 16 holding its own row's k, and reaches the product as a broadcast
 // within the lane row (row_newbcast) that costs no instruction for binary32; op(B) takes one
 // 16-byte read per 4 k (2). The next chunk's loads are in flight while a chunk is computed.
+// Short sums are bound by what a workgroup costs apart from them: loads, four barriers and the
+// LDS it holds. Sums that fit a chunk have one stage (four workgroups a CU against the two
+// stages' two), those of 256 bytes a row a stage of that size (six). Whole calls with one form
+// of two stages for every K, and with these: binary32 512 x 8 x 512 20.3 -> 16.4 us, 512 x 64 x
+// 512 21.1 -> 17.5, 512 x 256 x 512 23.2 -> 21.5, binary64 512 x 8 x 512 20.3 -> 17.0.
 #include "pcu_device.hpp"
 #include "pcu_gemm_search.hpp"
 #include "pcu_kernels.hpp"
@@ -63,17 +68,21 @@ template <int N, class F> __device__ __forceinline__ void each(F &&f)
 // product with any operand is far above the smallest normal.
 template <typename T> constexpr T kZeroStand = sizeof(T) == 4 ? (T)0x1p100 : (T)0x1p1000;
 
+// Waves a SIMD that the registers must leave room for: the LDS of the shortest form lets eight
+// workgroups run on a CU, of the longer one-chunk form four, of the two-stage form two.
+template <int L, bool ONE> constexpr int kSmallWaves = ONE ? (L == 1 ? 6 : 4) : 2;
+
 // The first fault of one cell in the kc k of a staged chunk (as: its row, bs: its column, zeros or
 // their stands up to the next 16 k), kNoFault when there is none or `on` is false. `step`: the
 // first k's Multiply. ADDS: t carries the cell's sum from chunk to chunk, and every product and
-// sum is checked; else only for a tiny product, with zeros staged as kZeroStand. Sixteen k at a
+// sum is checked; else only for a tiny product, with zeros staged as kZeroStand. 64 bytes of k at a
 // time, whose smallest product (and sum, where subnormal ones are rejected) says whether they go
 // through the exact classifiers: a compare for each k would have cost three times the products.
 template <typename T, bool ADDS>
 __device__ __forceinline__ uint64_t chunk_first_fault(const T *as, const T *bs, int kc, T &t, bool on,
                                                       uint64_t step, int policy)
 {
-    constexpr int P = 16 / (int)sizeof(T), U = 16;
+    constexpr int P = 16 / (int)sizeof(T), U = 4 * P;
     const bool reject_sub = policy == kPolicyRejectSubnormal;
     for (int k = 0; k < kc; k += U) {
         uint4 qa[U / P], qb[U / P];
@@ -116,9 +125,10 @@ __device__ __forceinline__ uint64_t chunk_first_fault(const T *as, const T *bs, 
     return kNoFault;
 }
 
-// VA, VB: every row of the stored matrix is 16-byte aligned.
-template <typename T, bool TA, bool TB, bool VA, bool VB>
-__global__ __launch_bounds__(256, 2) void k_strict_gemm_small(
+// VA, VB: every row of the stored matrix is 16-byte aligned. L: 16-byte runs of each operand that a
+// thread stages at a time, 256 L bytes of k a row. ONE: all of K is one chunk, in one stage.
+template <typename T, bool TA, bool TB, bool VA, bool VB, int L, bool ONE>
+__global__ __launch_bounds__(256, (kSmallWaves<L, ONE>)) void k_strict_gemm_small(
     const T *__restrict__ A, const T *__restrict__ B, T *__restrict__ C, int M, int N, int K,
     int thr, int risk, int policy, unsigned long long *fault, NodeGate gate, ProgramClose close)
 {
@@ -127,13 +137,13 @@ __global__ __launch_bounds__(256, 2) void k_strict_gemm_small(
         return;
     }
     constexpr int P = 16 / (int)sizeof(T);     // elements of 16 bytes
-    constexpr int BK = 1024 / (int)sizeof(T);  // k of a chunk
+    constexpr int BK = 16 * P * L;             // k of a chunk
     constexpr int BKP = BK + P;                // row pitch: one 16-byte pad
-    constexpr int L = BK / (16 * P);           // 16-byte runs of each operand a thread stages
-    __shared__ __align__(16) T As[2][16][BKP];
-    __shared__ __align__(16) T Bs[2][16][BKP];
+    constexpr int kST = ONE ? 1 : 2;           // stages
+    __shared__ __align__(16) T As[kST][16][BKP];
+    __shared__ __align__(16) T Bs[kST][16][BKP];
     __shared__ uint32_t rkey[16], ckey[16];
-    __shared__ unsigned long long best; // this block's earliest fault
+    __shared__ unsigned long long best; // the earliest fault that this block knows of
     __shared__ int first_sus;           // its first suspect cell, and whether that is finite
     const int tid = threadIdx.x;
     const int ty = tid >> 4, tx = tid & 15; // the thread's cell
@@ -143,10 +153,8 @@ __global__ __launch_bounds__(256, 2) void k_strict_gemm_small(
         rkey[tid] = 0xffffffffu;
         ckey[tid] = 0xffffffffu;
     }
-    if (tid == 0) {
-        best = kNoFault;
+    if (tid == 0)
         first_sus = INT_MAX;
-    }
     // A thread stages runs of P k of one row of op(A) and one column of op(B), 16 P k apart, in
     // an order that keeps each global access coalesced: 16 threads along k where k is
     // contiguous, else 16 threads along the rows (columns).
@@ -156,42 +164,46 @@ __global__ __launch_bounds__(256, 2) void k_strict_gemm_small(
     const T *pa = TA ? A + (row < M ? row : M - 1) : A + (size_t)(row < M ? row : M - 1) * K;
     const T *pb = TB ? B + (size_t)(col < N ? col : N - 1) * K : B + (col < N ? col : N - 1);
     T va[L][P], vb[L][P];
-    // One operand's runs of the chunk at k0. FULL: the chunk lies inside K, no bound checks;
-    // else elements past K are +0.
+    // One operand's runs of the chunk at k0. FULL: the chunk lies inside K. Else what lies past K
+    // is loaded from its end, so that every load of the chunk is in flight at once (a load
+    // under a condition is waited for before the next), and is +0.
     auto fetch = [&](const T *p, size_t ld, auto kc_c, auto vec_c, auto full_c, int kt, int k0,
                      T (&v)[L][P]) __attribute__((always_inline)) {
-        constexpr bool KC = decltype(kc_c)::value, VEC = decltype(vec_c)::value;
+        constexpr bool KC = decltype(kc_c)::value, VEC = KC && decltype(vec_c)::value;
         constexpr bool FULL = decltype(full_c)::value;
+        uint4 q[L];
 #pragma unroll
         for (int j = 0; j < L; j++) {
             const int k = k0 + kt + 16 * P * j;
-            if (KC && VEC && (FULL || k + P <= K)) {
-                const uint4 q = *reinterpret_cast<const uint4 *>(p + k);
-                const T *e = reinterpret_cast<const T *>(&q);
-#pragma unroll
-                for (int c = 0; c < P; c++)
-                    v[j][c] = e[c];
+            if constexpr (VEC) { // K is a multiple of P
+                q[j] = *reinterpret_cast<const uint4 *>(p + (FULL || k < K ? k : K - P));
             } else {
-                const T *pk = KC ? p + k : p + (size_t)k * ld;
 #pragma unroll
-                for (int c = 0; c < P; c++)
-                    v[j][c] = FULL || k + c < K ? pk[KC ? (size_t)c : c * ld] : (T)0;
+                for (int c = 0; c < P; c++) {
+                    const int kk = FULL || k + c < K ? k + c : K - 1;
+                    v[j][c] = p[KC ? (size_t)kk : (size_t)kk * ld];
+                }
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < L; j++) {
+            const int k = k0 + kt + 16 * P * j;
+            const T *e = reinterpret_cast<const T *>(&q[j]);
+#pragma unroll
+            for (int c = 0; c < P; c++) {
+                if constexpr (VEC)
+                    v[j][c] = e[c];
+                if (!FULL && k + c >= K)
+                    v[j][c] = (T)0;
             }
         }
     };
-    auto fetch_chunk = [&](int k0) __attribute__((always_inline)) {
-        const std::integral_constant<bool, !TA> kca;
-        const std::integral_constant<bool, TB> kcb;
-        const std::integral_constant<bool, VA> veca;
-        const std::integral_constant<bool, VB> vecb;
-        if (k0 + BK <= K) {
-            fetch(pa, (size_t)M, kca, veca, std::true_type{}, ka, k0, va);
-            fetch(pb, (size_t)N, kcb, vecb, std::true_type{}, kb, k0, vb);
-        } else {
-            fetch(pa, (size_t)M, kca, veca, std::false_type{}, ka, k0, va);
-            fetch(pb, (size_t)N, kcb, vecb, std::false_type{}, kb, k0, vb);
-        }
+    auto fetch_chunk = [&](auto full_c, int k0) __attribute__((always_inline)) {
+        fetch(pa, (size_t)M, std::integral_constant<bool, !TA>{}, std::integral_constant<bool, VA>{}, full_c, ka, k0, va);
+        fetch(pb, (size_t)N, std::integral_constant<bool, TB>{}, std::integral_constant<bool, VB>{}, full_c, kb, k0, vb);
     };
+    const std::true_type yes;
+    const std::false_type no;
     uint32_t amin = 0xffffffffu, bmin = 0xffffffffu;
     // STAND: zeros are staged as kZeroStand.
     auto stash_chunk = [&](int buf, auto stand_c) __attribute__((always_inline)) {
@@ -269,38 +281,64 @@ __global__ __launch_bounds__(256, 2) void k_strict_gemm_small(
                 a[c] = an[c];
         }
     };
-    // The last, partial block: whole groups only (zeros pad the last).
+    // The last, partial block, four groups at a time (zeros pad the last), op(B) read four groups
+    // ahead.
     auto part_block = [&](const T *as, const T *bs, int left) __attribute__((always_inline)) {
-        T a[P];
+        T a[P], b[2][4][P];
         load16(as + P * tx, a);
-        each<16>([&](auto j_c) __attribute__((always_inline)) {
-            constexpr int j = decltype(j_c)::value;
-            if (j * P < left) {
-                T b[P], p[P];
-                load16(bs + P * j, b);
-                products(j_c, a, b, p);
 #pragma unroll
-                for (int c = 0; c < P; c++)
-                    acc = acc + p[c];
+        for (int g = 0; g < 4; g++)
+            load16(bs + P * g, b[0][g]);
+        each<4>([&](auto u_c) __attribute__((always_inline)) {
+            constexpr int u = decltype(u_c)::value;
+            if (4 * P * u < left) {
+                if constexpr (u < 3)
+#pragma unroll
+                    for (int g = 0; g < 4; g++)
+                        load16(bs + P * (4 * u + 4 + g), b[(u + 1) & 1][g]);
+                each<4>([&](auto g_c) __attribute__((always_inline)) {
+                    constexpr int g = decltype(g_c)::value;
+                    T p[P];
+                    products(std::integral_constant<int, 4 * u + g>{}, a, b[u & 1][g], p);
+#pragma unroll
+                    for (int c = 0; c < P; c++)
+                        acc = acc + p[c];
+                });
             }
         });
     };
-    fetch_chunk(0);
-    stash_chunk(0, std::false_type{});
-    __syncthreads();
-    for (int k0 = 0, buf = 0; k0 < K; k0 += BK, buf ^= 1) {
-        const int kc = K - k0 < BK ? K - k0 : BK;
-        const bool next = k0 + BK < K;
-        if (next)
-            fetch_chunk(k0 + BK);
+    auto last_chunk = [&](int buf, int kc) __attribute__((always_inline)) {
         if (kc >= BL)
             whole_blocks(&As[buf][ty][0], &Bs[buf][tx][0], kc / BL);
         if (kc % BL != 0)
             part_block(&As[buf][ty][kc / BL * BL], &Bs[buf][tx][kc / BL * BL], kc % BL);
-        if (next) {
-            stash_chunk(buf ^ 1, std::false_type{});
+    };
+    if constexpr (ONE) {
+        fetch_chunk(no, 0);
+        stash_chunk(0, no);
+        __syncthreads();
+        last_chunk(0, K);
+    } else {
+        // A chunk that another follows. The two kinds of next chunk are separate code: where their
+        // loads met, the compiler waited for them before the sums.
+        auto chunk = [&](auto full_c, int k0, int buf) __attribute__((always_inline)) {
+            fetch_chunk(full_c, k0 + BK);
+            whole_blocks(&As[buf][ty][0], &Bs[buf][tx][0], BK / BL);
+            stash_chunk(buf ^ 1, no);
             __syncthreads();
+        };
+        fetch_chunk(yes, 0); // K > BK
+        stash_chunk(0, no);
+        __syncthreads();
+        int k0 = 0, buf = 0;
+        for (; k0 + 2 * BK <= K; k0 += BK, buf ^= 1)
+            chunk(yes, k0, buf);
+        if (k0 + BK < K) {
+            chunk(no, k0, buf);
+            k0 += BK;
+            buf ^= 1;
         }
+        last_chunk(buf, K - k0);
     }
     if (amin != 0xffffffffu)
         atomicMin(&rkey[xa], amin);
@@ -317,17 +355,26 @@ __global__ __launch_bounds__(256, 2) void k_strict_gemm_small(
         program_close_block(close);
         return;
     }
-    // The search. A block whose first suspect cell is not finite has its first fault there (such a
-    // result comes of a fault), and a wave walks that cell alone.
+    // The search. Nothing is left to it where another block has already recorded a fault before this
+    // one's first suspect cell: a NaN in a row or column of many blocks costs few of them a walk and
+    // an atomic on the node's word. A block whose first suspect cell is not finite has its first
+    // fault there (such a result comes of a fault), and a wave walks that cell alone.
     const uint64_t mask = __ballot(sus);
     if (mask != 0 && (tid & 63) == __ffsll((long long)mask) - 1)
         atomicMin(&first_sus, 2 * tid + (int)finite_bits(acc));
+    if (tid == 0)
+        best = __atomic_load_n(fault, __ATOMIC_RELAXED);
     __syncthreads();
+    const int i = first_sus >> 1;
+    const uint64_t cell0 = (uint64_t)(m0 + (i >> 4)) * N + n0 + (i & 15);
+    if (best < pack_fault(cell0 * (uint64_t)K * 2, 0)) {
+        program_close_block(close);
+        return;
+    }
     if (!(first_sus & 1)) {
-        const int i = first_sus >> 1;
         if (tid < 64) {
             const uint64_t w = cell_first_fault(A, B, (uint64_t)M, (uint64_t)N, (uint64_t)K, (int)TA, (int)TB,
-                                                (uint64_t)(m0 + (i >> 4)) * N + n0 + (i & 15), policy, true);
+                                                cell0, policy, true);
             if (w != kNoFault && tid == 0) {
                 atomicMin(fault, (unsigned long long)w);
                 gate_record(gate);
@@ -345,12 +392,12 @@ __global__ __launch_bounds__(256, 2) void k_strict_gemm_small(
     const bool adds = policy == kPolicyRejectSubnormal || __syncthreads_or(sus && !finite_bits(acc));
     T t = (T)0;
     for (int k0 = 0; k0 < K; k0 += BK) {
-        if (!adds || K > BK) { // a single chunk still stands in its stage
-            fetch_chunk(k0);
+        if (!adds || !ONE) { // a single chunk still stands in its stage
+            fetch_chunk(no, k0);
             if (adds)
-                stash_chunk(0, std::false_type{});
+                stash_chunk(0, no);
             else
-                stash_chunk(0, std::true_type{});
+                stash_chunk(0, yes);
             __syncthreads();
         }
         uint64_t key = kNoFault;
@@ -384,10 +431,19 @@ static void small_launch(hipStream_t s, dim3 grid, const T *A, const T *B, T *C,
 {
     constexpr int P = 16 / (int)sizeof(T);
     const bool va = !TA && K % P == 0 && aligned16(A), vb = TB && K % P == 0 && aligned16(B);
+    auto form = [&](auto va_c, auto vb_c) {
+        constexpr bool VA = decltype(va_c)::value, VB = decltype(vb_c)::value;
+        if (K <= 16 * P)
+            hipLaunchKernelGGL((k_strict_gemm_small<T, TA, TB, VA, VB, 1, true>), grid, dim3(256), 0, s, A, B, C, M, N, K, thr, risk, policy, fault, gate, close);
+        else if (K <= 64 * P)
+            hipLaunchKernelGGL((k_strict_gemm_small<T, TA, TB, VA, VB, 4, true>), grid, dim3(256), 0, s, A, B, C, M, N, K, thr, risk, policy, fault, gate, close);
+        else
+            hipLaunchKernelGGL((k_strict_gemm_small<T, TA, TB, VA, VB, 4, false>), grid, dim3(256), 0, s, A, B, C, M, N, K, thr, risk, policy, fault, gate, close);
+    };
     if ((TA || va) && (!TB || vb))
-        hipLaunchKernelGGL((k_strict_gemm_small<T, TA, TB, !TA, TB>), grid, dim3(256), 0, s, A, B, C, M, N, K, thr, risk, policy, fault, gate, close);
+        form(std::integral_constant<bool, !TA>{}, std::integral_constant<bool, TB>{});
     else
-        hipLaunchKernelGGL((k_strict_gemm_small<T, TA, TB, false, false>), grid, dim3(256), 0, s, A, B, C, M, N, K, thr, risk, policy, fault, gate, close);
+        form(std::false_type{}, std::false_type{});
 }
 
 template <typename T>
@@ -405,26 +461,56 @@ static void small_layout(hipStream_t s, dim3 grid, bool ta, bool tb, const T *A,
         small_launch<T, true, true>(s, grid, A, B, C, M, N, K, thr, risk, policy, fault, gate, close);
 }
 
-// Estimated microseconds of this kernel and of the screened tile kernels, from measurements on
-// MI355X per 1024 k: up to two workgroups a CU run beside each other (binary32 12, 15; binary64
-// 22, 30), more take turns (6.1 and 13.2 each). The screened path adds a screen, a scan and a
-// replay launch (15 us). Its binary64 tiles: see mid_wanted_f64. Kernels at the lines: binary32
-// 256 x 1024 x 1024 (1024 workgroups) 27 us against 20 + 15, 256 x 4096 x 1024 95 against
-// 69 + 15; binary64 512 x 1024 x 512 53 against 88 + 15.
+// Estimated microseconds of this kernel, from kernel times on MI355X of 1 to 64 workgroups a CU and
+// K = 8 to 4096 (a fixed part, and each workgroup of the fullest CU its own): the forms of one chunk
+// have 4 to 6 workgroups of a CU beside each other, the two-stage form two. Kernels of 4 / 8 / 16
+// workgroups a CU: binary32 K = 8 4.4 / 5.7 / 9.7 us, K = 64 5.2 / 7.8 / 12.2, K = 256 10.9 / 15.4 /
+// 26.6, K = 1024 28.8 / 54.4 / 102.9; binary64 K = 8 4.4 / 6.3 / 9.5, K = 64 8.3 / 13.0 / 21.5, K =
+// 256 17.1 / 30.2 / 56.3, K = 1024 53.6 / 102 / 196.
+static double small_time(int dtype, double c, uint64_t inner)
+{
+    const double K = (double)inner, k = K / 1024.0;
+    if (dtype == 0) {
+        if (inner <= 64)
+            return 3.3 + c * (0.33 + 0.0033 * K);
+        if (inner <= 256)
+            return 4 + c * (0.62 + 0.0028 * K);
+        return c <= 1 ? 4.5 + 8.6 * k : 3 + c * (0.7 + 5.79 * k);
+    }
+    if (inner <= 32)
+        return 3.3 + c * (0.3 + 0.0085 * K);
+    if (inner <= 128)
+        return 4.5 + c * (0.6 + 0.0065 * K);
+    return c <= 1 ? 3.5 + 16.5 * k : 4 + c * (0.5 + 12.4 * k);
+}
+
+// Against the screened tile kernels: their screen (about 4.5 us, 2 more for each 1024 k of a row,
+// and both operands at 6 MB a us), the tiles as mid_time_f32 and mid_wanted_f64 put them, which leaves
+// out a fixed part and the store of the output, and the further launches (0.5 us; whole calls of
+// either route otherwise take their kernels and 11.5 us). Whole calls, this kernel against the tiles,
+// on both sides of the line: binary32 512 x 8 x 1024 18.0 / 21.0 us, 1024 x 8 x 1024 20.7 / 22.2, 4096
+// x 8 x 512 26.0 / 24.5, 1024 x 64 x 1024 23.8 / 24.9, 512 x 100 x 1024 23.2 / 23.8, 1024 x 100 x 1024
+// 30.4 / 26.7, 512 x 256 x 512 21.5 / 25.3, 512 x 1024 x 256 28.7 / 50; binary64 1024 x 8 x 1024 21.7
+// / 23.0, 4096 x 8 x 512 27.5 / 25.8, 512 x 128 x 1024 27.9 / 33.1, 1024 x 128 x 1024 44 / 34.
 bool gemm_small_wanted(int dtype, uint64_t rows, uint64_t inner, uint64_t cols)
 {
     const auto per_cu = [&](uint64_t t) {
         const uint64_t tiles = ((rows + t - 1) / t) * ((cols + t - 1) / t);
         return (double)((tiles + kGfx950Cus - 1) / kGfx950Cus);
     };
-    const double k = (double)inner / 1024.0, c = per_cu(16);
     // A launch holds fewer than 2^32 threads: one a cell.
     if (((rows + 15) / 16) * ((cols + 15) / 16) > UINT32_MAX / 256)
         return false;
-    if (dtype == 0)
-        return (c <= 2 ? 9 + 3 * c : 6.1 * c) * k + 3 < mid_time_f32(rows, cols, inner) + 15;
-    const double c64 = per_cu(64);
-    return (c <= 2 ? 14 + 8 * c : 13.2 * c) * k + 3 < (c64 <= 2 ? 26 + 65 * c64 : 74 * c64) * k + 18;
+    const double k = (double)inner / 1024.0, cells = (double)rows * (double)cols;
+    const double mb = ((double)rows + (double)cols) * (double)inner * (dtype == 0 ? 4e-6 : 8e-6);
+    double tiles = 4.5 + 2 * k + mb / 6 + 0.5;
+    if (dtype == 0) {
+        tiles += mid_time_f32(rows, cols, inner) + 2 + 1.2e-6 * cells;
+    } else {
+        const double c64 = per_cu(64);
+        tiles += (c64 <= 2 ? 26 + 65 * c64 : 74 * c64) * k + 3.5 + 1.8e-6 * cells;
+    }
+    return small_time(dtype, per_cu(16), inner) < tiles;
 }
 
 hipError_t launch_gemm_small(hipStream_t s, int dtype, int M, int N, int K, bool ta, bool tb,

@@ -41,6 +41,26 @@ def test_no_choice_launches_more_threads_than_a_grid_holds(tile):
                 assert m * n * threads[tile(dtype, m, k, n, policy=policy)] < 2 ** 32, (dtype, m, k, n)
 
 
+@pytest.mark.parametrize("dtype", ["f32", "f64"])
+def test_short_sums_of_many_cells_take_the_tiles(tile, dtype):
+    """One launch pays for each of its 16 x 16 workgroups, however short the sum; above some 30 of
+    them a CU the tile kernels are the faster at every K, at the smaller K of several too."""
+    for k in (1, 8, 15, 16, 30, 32, 64, 100, 128, 256, 1024, 4096):
+        for m, n in ((4096, 4096), (2048, 2048), (8192, 8192), (4096, 1024), (64, 65536)):
+            assert tile(dtype, m, k, n) != 16, (m, k, n)
+    for m, k, n in ((4096, 8, 512), (1024, 128, 1024), (1024, 256, 1024), (4096, 64, 512)):
+        assert tile(dtype, m, k, n) != 16, (m, k, n)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f64"])
+def test_few_cells_take_one_launch(tile, dtype):
+    for m, k, n in ((64, 256, 64), (1, 1, 1), (64, 4096, 1024), (512, 8, 512), (1024, 8, 1024), (512, 64, 1024),
+                    (256, 1024, 256), (64, 64, 2048), (100, 17, 300)):
+        for tl in (False, True):
+            for tr in (False, True):
+                assert tile(dtype, m, k, n, tl, tr) == 16, (m, k, n)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("name,engine", [("auto", AUTO), ("valu", VALU), ("mfma_products", MFMA)])
 def test_a_context_runs_with_the_engine_it_was_given(pcu_pkg, name, engine):
