@@ -185,6 +185,15 @@ __global__ __launch_bounds__(Cfg::kThreads, Cfg::kWavesPerSimd) void k_native_ge
     }
 }
 
+// Whether an operand's tiles load directly as whole ones: every row 16-byte aligned, and a lane's
+// byte offset from its run's base within 32 bits.
+static bool native_direct(const float *A, const float *B, uint64_t M, uint64_t N, uint64_t K, bool ta, bool tb)
+{
+    const uint64_t span_a = ta ? M + 128 : 64 * K, span_b = N + 128;
+    return (ta ? M : K) % 4 == 0 && (tb ? K : N) % 4 == 0 && aligned16(A) && aligned16(B) &&
+           4 * span_a <= UINT32_MAX && (tb || 4 * span_b <= UINT32_MAX);
+}
+
 template <class Cfg, bool TA, bool TB>
 static void native_dispatch(hipStream_t s, const float *A, const float *B, float *C, int M, int N,
                             int K, NodeGate gate)
@@ -193,10 +202,7 @@ static void native_dispatch(hipStream_t s, const float *A, const float *B, float
     const dim3 block(Cfg::kThreads);
     const bool va = (TA ? (M % 4 == 0) : (K % 4 == 0)) && aligned16(A);
     const bool vb = (TB ? (K % 4 == 0) : (N % 4 == 0)) && aligned16(B);
-    // Whole tiles load directly: a lane's byte offset from its run's base must fit 32 bits.
-    const uint64_t span_a = TA ? (uint64_t)M + 128 : 64 * (uint64_t)K, span_b = (uint64_t)N + 128;
-    const bool offsets32 = 4 * span_a <= UINT32_MAX && (TB || 4 * span_b <= UINT32_MAX);
-    const bool whole = va && vb && M % Cfg::BM == 0 && N % Cfg::BN == 0 && K % Cfg::BK == 0 && offsets32;
+    const bool whole = M % Cfg::BM == 0 && N % Cfg::BN == 0 && K % Cfg::BK == 0 && native_direct(A, B, M, N, K, TA, TB);
     if (whole)
         hipLaunchKernelGGL((k_native_gemm_mfma<Cfg, TA, TB, true, true, true>), grid, block, 0, s, A, B, C, M, N, K, gate);
     else if (va && vb)
@@ -252,8 +258,8 @@ static hipError_t launch_native_mid(hipStream_t s, MidTile tile, int M, int N, i
 
 // Estimated microseconds of each tile, from measurements on MI355X: the tiles of the fullest CU
 // times what one takes, per 1024 k and fixed. A whole 128 x 128 tile 68 alone on its CU, 59
-// beside others (a bound-checked one 85 and more: never chosen, 3001 x 2999 x 3003 took 1065 us
-// on them and 446 on 64 x 64 tiles). A 64 x 64 tile 17 + 1, alone 20 + 2.5; a 32 x 32 tile
+// beside others (a bound-checked one 85 and more: taken only where the smaller tiles cannot address
+// the operands, 3001 x 2999 x 3003 took 1065 us on them and 446 on 64 x 64 tiles). A 64 x 64 tile 17 + 1, alone 20 + 2.5; a 32 x 32 tile
 // 5.4 + 0.4, up to two 8.1 and 14 + 2.5 together. Against 128 x 128 tiles: 1024 x 2048 x 1024
 // 44 against 137 us, 1024 x 2048 x 2048 76 / 139, 64 x 4096 x 1024 35 / 348, 777 x 3000 x 555
 // 41 / 351; 4096^3 1038 / 957.
@@ -271,12 +277,27 @@ static MidTile native_tile(uint64_t M, uint64_t N, uint64_t K, bool whole)
     return t32 < t64 ? MidTile::k32 : MidTile::k64;
 }
 
+// The tile that a native MatMul of these operands takes.
+static MidTile native_choice(const float *A, const float *B, uint64_t M, uint64_t N, uint64_t K, bool ta, bool tb)
+{
+    const bool whole = M % NativeCfg::BM == 0 && N % NativeCfg::BN == 0 && K % NativeCfg::BK == 0 &&
+                       native_direct(A, B, M, N, K, ta, tb);
+    return mid_fits_f32(M, N, K, ta, tb) ? native_tile(M, N, K, whole) : MidTile::k128;
+}
+
+// native_choice as a tile side, for tests of the choice.
+extern "C" int pcu_internal_native_matmul_tile(const void *a, const void *b, uint64_t rows, uint64_t inner,
+                                               uint64_t cols, int ta, int tb)
+{
+    const MidTile t = native_choice((const float *)a, (const float *)b, rows, cols, inner, ta != 0, tb != 0);
+    return t == MidTile::k32 ? 32 : (t == MidTile::k64 ? 64 : 128);
+}
+
 hipError_t launch_native_gemm_f32(hipStream_t s, int M, int N, int K, bool ta, bool tb,
                                   const float *A, const float *B, float *C, NodeGate gate)
 {
-    const bool whole = M % NativeCfg::BM == 0 && N % NativeCfg::BN == 0 && K % NativeCfg::BK == 0;
-    const MidTile tile = native_tile((uint64_t)M, (uint64_t)N, (uint64_t)K, whole);
-    if (tile != MidTile::k128 && mid_fits_f32((uint64_t)M, (uint64_t)N, (uint64_t)K, ta, tb))
+    const MidTile tile = native_choice(A, B, (uint64_t)M, (uint64_t)N, (uint64_t)K, ta, tb);
+    if (tile != MidTile::k128)
         return launch_native_mid(s, tile, M, N, K, ta, tb, A, B, C, gate);
     if (!ta && !tb) native_dispatch<NativeCfg, false, false>(s, A, B, C, M, N, K, gate);
     else if (!ta && tb) native_dispatch<NativeCfg, false, true>(s, A, B, C, M, N, K, gate);

@@ -61,6 +61,18 @@ def test_few_cells_take_one_launch(tile, dtype):
                 assert tile(dtype, m, k, n, tl, tr) == 16, (m, k, n)
 
 
+def test_native_whole_tiles_need_aligned_operands(pcu_pkg):
+    """A grid of whole 128 x 128 tiles is one only where both operands' rows are 16-byte aligned:
+    the bound-checked form of that tile is slower than the 64 x 64 tiles at every size."""
+    f = pcu_pkg.lib().pcu_internal_native_matmul_tile
+    f.argtypes, f.restype = 2 * [ctypes.c_void_p] + 3 * [ctypes.c_uint64] + 2 * [ctypes.c_int], ctypes.c_int
+    for tl in (0, 1):
+        for tr in (0, 1):
+            assert f(0x10000, 0x20000, 4096, 4096, 4096, tl, tr) == 128
+            for a, b in ((0x10004, 0x20000), (0x10000, 0x20008), (0x10004, 0x20004)):
+                assert f(a, b, 4096, 4096, 4096, tl, tr) == 64
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("name,engine", [("auto", AUTO), ("valu", VALU), ("mfma_products", MFMA)])
 def test_a_context_runs_with_the_engine_it_was_given(pcu_pkg, name, engine):
