@@ -306,7 +306,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f64_mid(
         }
     }
     if constexpr (!NATIVE)
-        wave_record_fault(key, suspect);
+        wave_record_first(key, suspect);
 }
 
 static inline bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }

@@ -676,6 +676,20 @@ __device__ __forceinline__ void wave_record_fault(uint64_t key, unsigned long lo
     }
 }
 
+// Record the wave's earliest key, where the word does not hold an earlier one already: the tiles of
+// a grid are dispatched from its first cells on, so of many waves with a key most find one. The
+// binary64 64 x 64 tiles, four waves for the cells of one wave of a 128 x 128 tile, queued on the
+// word: a call with a NaN in every row 88 -> 60 us at 2048 x 32 x 2048 (73 on larger tiles), 122 ->
+// 112 at 2048 x 256 x 2048; clean calls unchanged.
+__device__ __forceinline__ void wave_record_first(uint64_t key, unsigned long long *word)
+{
+    if (__ballot(key != kNoFault) == 0)
+        return;
+    const uint64_t m = wave_min_u64(key);
+    if (__lane_id() == 0 && m < __atomic_load_n(word, __ATOMIC_RELAXED))
+        atomicMin(word, (unsigned long long)m);
+}
+
 // Record the workgroup's earliest key with one atomic: every thread of a workgroup of NW
 // waves calls it (it holds a barrier). A MatMul tile with a NaN operand marks whole rows or
 // columns suspect, and one atomic a wave on the one word then queues every wave of the grid
