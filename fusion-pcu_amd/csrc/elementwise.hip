@@ -635,6 +635,8 @@ template <> struct SumBits<double> {
 
 // Threads of a chunk's scan; a chunk is kPer elements for each.
 constexpr int kSumThreads = 512;
+// Inputs of up to kMseSerialMax elements are summed by one wave (k_mse_serial).
+constexpr uint64_t kMseSerialMax = 2048;
 constexpr int kQuarters = 4; // parts of a chunk that the squares kernel sums on their own
 
 template <typename T>
@@ -1651,6 +1653,162 @@ __global__ __launch_bounds__(kSumThreads) __attribute__((amdgpu_waves_per_eu(4))
     program_close_block(close);
 }
 
+// Inputs of at most kMseSerialMax elements, one workgroup. Its four waves form every difference and
+// square in parallel into LDS (all of a thread's loads are issued before it computes) and find the
+// first faulting Subtract or Multiply; then one wave folds the squares before that element in order,
+// a chunk of 60 (binary64 30) at a time, every lane holding the chunk in registers and the next
+// chunk's LDS reads in flight. A sum can only fault as in fold_run, so a chunk is folded with plain
+// adds (REJECT_SUB: each partial total is kept and checked after) and again exactly only when that
+// trips. The same results and first fault as below. What bounds it is the chain of adds, about
+// 4.4 ns each and no barrier among them; the kernel of one chunk below pays some 250 ns more for 64
+// of them and 2 us a window: whole calls, this one against that, binary32 300 squares 15.1 / 17.1 us,
+// 512 16.2 / 18.6, 1024 18.9 / 21.7, 2000 23.6 / 24.2, 4096 45 / 42; binary64 512 18.0 / 20.2, 1024
+// 21.4 / 23.9.
+template <typename T, bool REJECT_SUB>
+__device__ __forceinline__ void mse_serial(const T *__restrict__ p, const T *__restrict__ t, uint64_t n,
+                                           T count, int policy, T *__restrict__ out,
+                                           unsigned long long *fault, const NodeGate &gate)
+{
+    if (block_gate_closed(gate))
+        return;
+    constexpr int P = 16 / sizeof(T);              // squares per 16-byte LDS read
+    constexpr int R = (int)(kMseSerialMax / 256);  // elements a thread
+    __shared__ __align__(16) T sq[kMseSerialMax];
+    __shared__ unsigned long long first_sm; // earliest Subtract or Multiply fault word
+    const int tid = threadIdx.x;
+    if (tid == 0)
+        first_sm = kNoFault;
+    T pv[R], tv[R];
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+        const uint64_t i = (uint64_t)tid + 256u * (uint64_t)j;
+        if (i < n) {
+            pv[j] = p[i];
+            tv[j] = t[i];
+        }
+    }
+    __syncthreads();
+    uint64_t key = kNoFault;
+    bool any = false; // a square other than +0
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+        const uint64_t i = (uint64_t)tid + 256u * (uint64_t)j;
+        if (i < n) {
+            const T d = pv[j] - tv[j];
+            const T s = d * d;
+            sq[i] = s;
+            any |= !is_zero(s);
+            if (key == kNoFault) {
+                const uint32_t ks = classify_add(pv[j], tv[j], d, policy);
+                if (ks != kOk) {
+                    key = pack_fault(3 * i, ks);
+                } else {
+                    const uint32_t km = classify_mul(d, d, s, policy);
+                    if (km != kOk)
+                        key = pack_fault(3 * i + 1, km);
+                }
+            }
+        }
+    }
+    if (key != kNoFault)
+        atomicMin(&first_sm, (unsigned long long)key);
+    any = __syncthreads_or(any);
+    if (tid >= 64)
+        return;
+    const unsigned long long fsm = first_sm;
+    // Elements summed; squares that are all +0 leave the total at +0.
+    const uint64_t limit = fsm != kNoFault ? ((fsm >> 3) / 3) : (any ? n : 0);
+    T total = (T)0;
+    // The exact pass over squares i0 .. i0 + here - 1 from `total`: false when an Add faults
+    // (recorded).
+    auto exact = [&](uint64_t i0, uint32_t here) {
+        bool ok = true;
+        if (tid == 0)
+            ok = fold_exact<T>(total, here, i0, policy, fault, gate, [&](uint32_t i) { return sq[i0 + i]; });
+        return __ballot(!ok) == 0;
+    };
+    // A chunk is 15 LDS reads: with the next chunk's 15 reads issued before its adds, the wait for
+    // this chunk (in-order LDS counter, at most 15 outstanding) leaves all of them in flight.
+    constexpr int CH = 15 * P;
+    auto load = [&](T (&v)[CH], uint64_t i0) {
+#pragma unroll
+        for (int q = 0; q < CH / P; q++)
+            *reinterpret_cast<uint4 *>(&v[P * q]) = *reinterpret_cast<const uint4 *>(&sq[i0 + P * q]);
+    };
+    // Folds a whole chunk held in v; false when an Add faults (recorded).
+    auto fold = [&](T (&v)[CH], uint64_t i0) __attribute__((always_inline)) {
+        T sum = total;
+        bool trip = false;
+        if constexpr (!REJECT_SUB) {
+#pragma unroll
+            for (int j = 0; j < CH; j++)
+                sum = sum + v[j];
+        } else {
+#pragma unroll
+            for (int j = 0; j < CH; j++) {
+                sum = sum + v[j];
+                v[j] = sum;
+            }
+#pragma unroll
+            for (int j = 0; j < CH; j++)
+                trip |= subnormal(v[j]);
+        }
+        if ((!finite_bits(sum) || trip) && !exact(i0, CH))
+            return false;
+        total = sum;
+        return true;
+    };
+    const uint64_t full = limit / CH * CH;
+    T va[CH], vb[CH];
+    if (full > 0)
+        load(va, 0);
+    for (uint64_t i0 = 0; i0 < full; i0 += 2 * CH) {
+        const bool second = i0 + CH < full;
+        if (second)
+            load(vb, i0 + CH);
+        if (!fold(va, i0))
+            return;
+        if (!second)
+            break;
+        if (i0 + 2 * CH < full)
+            load(va, i0 + 2 * CH);
+        if (!fold(vb, i0 + CH))
+            return;
+    }
+    if (limit > full) {
+        const uint32_t here = (uint32_t)(limit - full);
+        T sum = total;
+        bool trip = false;
+        for (uint32_t j = 0; j < here; j++) {
+            sum = sum + sq[full + j];
+            trip |= REJECT_SUB && subnormal(sum);
+        }
+        if ((!finite_bits(sum) || trip) && !exact(full, here))
+            return;
+        total = sum;
+    }
+    if (tid != 0)
+        return;
+    const T r = total / count;
+    const uint32_t kind = fsm != kNoFault ? kOk : classify_div(total, count, r, policy);
+    if (fsm != kNoFault || kind != kOk) {
+        atomicMin(fault, fsm != kNoFault ? fsm : (unsigned long long)pack_fault(3 * n, kind));
+        gate_record(gate);
+    } else {
+        *out = r;
+    }
+}
+
+template <typename T, bool REJECT_SUB>
+__global__ __launch_bounds__(256) void k_mse_serial(const T *__restrict__ p, const T *__restrict__ t, uint64_t n,
+                                                    T count, int policy, T *__restrict__ out,
+                                                    unsigned long long *fault, NodeGate gate,
+                                                    ProgramClose close)
+{
+    mse_serial<T, REJECT_SUB>(p, t, n, count, policy, out, fault, gate);
+    program_close_block(close);
+}
+
 // Inputs of one chunk, one workgroup. Its waves form every difference and square in parallel into
 // LDS (each thread issues all of its loads before it computes, so the inputs arrive in one round
 // trip), find the first faulting Subtract or Multiply and estimate the mean; then the squares
@@ -2200,7 +2358,16 @@ hipError_t launch_mse_one(hipStream_t s, int dtype, uint64_t n, const void *p, c
 {
     if (n == 0 || n > mse_one_max(dtype))
         return hipErrorInvalidValue;
-    if (dtype == 0)
+    const bool reject = policy == kPolicyRejectSubnormal;
+    if (n <= kMseSerialMax && dtype == 0 && reject)
+        hipLaunchKernelGGL((k_mse_serial<float, true>), dim3(1), dim3(256), 0, s, (const float *)p, (const float *)t, n, (float)count, policy, (float *)out, fault, gate, close);
+    else if (n <= kMseSerialMax && dtype == 0)
+        hipLaunchKernelGGL((k_mse_serial<float, false>), dim3(1), dim3(256), 0, s, (const float *)p, (const float *)t, n, (float)count, policy, (float *)out, fault, gate, close);
+    else if (n <= kMseSerialMax && reject)
+        hipLaunchKernelGGL((k_mse_serial<double, true>), dim3(1), dim3(256), 0, s, (const double *)p, (const double *)t, n, count, policy, (double *)out, fault, gate, close);
+    else if (n <= kMseSerialMax)
+        hipLaunchKernelGGL((k_mse_serial<double, false>), dim3(1), dim3(256), 0, s, (const double *)p, (const double *)t, n, count, policy, (double *)out, fault, gate, close);
+    else if (dtype == 0)
         hipLaunchKernelGGL((k_mse_one<float>), dim3(1), dim3(kSumThreads), 0, s, (const float *)p, (const float *)t, n, (float)count, policy, (float *)out, fault, gate, close);
     else
         hipLaunchKernelGGL((k_mse_one<double>), dim3(1), dim3(kSumThreads), 0, s, (const double *)p, (const double *)t, n, count, policy, (double *)out, fault, gate, close);

@@ -73,3 +73,34 @@ def test_lengths_about_the_one_workgroup_kernel(ctx, pcu_pkg, dtype):
             p = rng.normal(0, 1, n).astype(dtype)
             p[at] = np.inf
             _check(ctx, pcu_pkg, p, 0)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("policy", [0, 1, 2])
+@pytest.mark.parametrize("n", [61, 121, 2048, 2049])
+def test_first_squares_of_short_inputs(ctx, pcu_pkg, dtype, policy, n):
+    test_first_squares(ctx, pcu_pkg, dtype, policy, n)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("policy", [0, 1, 2])
+def test_lengths_about_the_one_wave_kernel(ctx, pcu_pkg, dtype, policy):
+    """Lengths about its chunks of 60 (binary64 30) squares, its four waves and its limit: random,
+    whole counts, squares all zero, a first fault of each kind at the first, a middle and the last
+    element."""
+    rng = np.random.default_rng(13)
+    info = np.finfo(dtype)
+    for n in (1, 2, 29, 30, 31, 59, 60, 61, 119, 120, 121, 255, 256, 257, 2047, 2048, 2049):
+        p = rng.normal(0, 1, n).astype(dtype)
+        _check(ctx, pcu_pkg, p, policy)
+        _check(ctx, pcu_pkg, np.ones(n, dtype), policy)
+        _check(ctx, pcu_pkg, np.zeros(n, dtype), policy)
+        for at in {0, n // 2, n - 1}:
+            # Subtract of a NaN; a square that overflows, is tiny, is exactly subnormal; a mean that is.
+            for special in (np.nan, info.max, np.sqrt(info.tiny) * dtype(0.7), dtype(2.0 ** ((info.minexp - 3) // 2))):
+                q = p.copy()
+                q[at] = special
+                _check(ctx, pcu_pkg, q, policy)
+                q[:] = 0
+                q[at] = special
+                _check(ctx, pcu_pkg, q, policy)
