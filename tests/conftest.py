@@ -1,3 +1,4 @@
+import ctypes
 import importlib.util
 import os
 import sys
@@ -32,6 +33,21 @@ def pytest_configure(config):
 @pytest.fixture(scope="session")
 def pcu_pkg():
     return _load_package()
+
+
+@pytest.fixture(scope="session")
+def strict_tile(pcu_pkg):
+    """The side of the output tile that a strict MatMul of these sizes takes (16: the one launch of
+    few cells), so that a test can say which kernel it reaches."""
+    f = pcu_pkg.lib().pcu_internal_strict_matmul_tile
+    f.argtypes = [ctypes.c_int] + 3 * [ctypes.c_uint64] + 4 * [ctypes.c_int]
+    f.restype = ctypes.c_int
+    engines = {"auto": 0, "valu": 1, "mfma_products": 2}
+
+    def call(dtype, m, k, n, tl=False, tr=False, policy=0, engine="auto"):
+        return f(int(dtype().itemsize == 8), m, k, n, int(tl), int(tr), policy, engines[engine])
+
+    return call
 
 
 @pytest.fixture(scope="session")

@@ -515,7 +515,7 @@ def test_matmul_relu_epilogue_fault_order(G, pcu_pkg, dtype):
     tiny = dtype(2.0 ** -70) if dtype == np.float32 else dtype(2.0 ** -530)
     ctx = G.default_context()
     rng = np.random.default_rng(37)
-    for m, k, n in ((2048, 64, 2048), (2048, 128, 2176), (2048, 64, 2050), (256, 64, 256)):
+    for m, k, n in ((2048, 64, 2048), (2048, 128, 2176), (2048, 64, 2050), (2040, 64, 1930), (256, 64, 256)):
         g = G.Graph()
         g.set_numerical_mode(True)
         a, b = g.input((m, k), dtype), g.input((k, n), dtype)

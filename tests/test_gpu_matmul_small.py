@@ -2,8 +2,6 @@
 16 x 16 blocks, of the chunks it stages (256 k for F32, 128 for F64), of the blocks it computes
 (64 and 32 k) and of the groups in them, rows that are and are not 16-byte aligned, in every
 layout, under every policy, with and without faults. Bit-exact against the oracle."""
-import ctypes
-
 import numpy as np
 import pytest
 
@@ -139,19 +137,17 @@ def test_search_of_many_suspect_cells(ctx, pcu_pkg, dtype, layout, policy):
 
 @DTYPES
 @pytest.mark.parametrize("layout", [(False, False), (True, True)], ids=["nn", "tt"])
-def test_many_workgroups_of_short_sums(ctx, pcu_pkg, dtype, layout):
+def test_many_workgroups_of_short_sums(ctx, pcu_pkg, strict_tile, dtype, layout):
     """Grids of more workgroups than run at once, at sums that stand in one chunk of each form and
     just past it: clean, a row of NaN after a tiny product in an earlier workgroup, and faults in
     several workgroups of which the last to be dispatched holds none of the first cells."""
     tl, tr = layout
     rng = np.random.default_rng(31)
     low = dtype(2.0 ** (-120 if dtype == np.float32 else -1016))
-    tile = ctx._lib.pcu_internal_strict_matmul_tile
-    tile.argtypes = [ctypes.c_int] + 3 * [ctypes.c_uint64] + 4 * [ctypes.c_int]
     per = 16 // np.dtype(dtype).itemsize
     for m, k, n in ((1000, 7, 1000), (33, 16 * per, 5000), (700, 16 * per + 1, 600), (500, 64 * per, 600),
                     (300, 64 * per + 3, 400)):
-        assert tile(0 if dtype == np.float32 else 1, m, k, n, int(tl), int(tr), 0, 0) == 16
+        assert strict_tile(dtype, m, k, n, tl, tr) == 16
         a, b = _operands(rng, m, k, n, tl, tr, dtype)
         av, bv = (a.T if tl else a), (b.T if tr else b)
         _check(ctx, pcu_pkg, a, b, tl, tr, 0)

@@ -1,5 +1,5 @@
-"""The strict F32 MatMul's smaller tiles at the sizes where they can go wrong: the edges of the
-32 x 32 and 64 x 64 tiles, slabs of 32 k and their remainders, operands whose rows are and are
+"""The strict F32 MatMul's tiles at the sizes where they can go wrong: the edges of the 32 x 32, 64 x
+64 and bound-checked 128 x 128 tiles, slabs of 32 (16) k and their remainders, operands whose rows are and are
 not 16-byte aligned, in every layout, under every policy, with and without faults. Outputs are
 bit-exact and first faults exact against the oracle."""
 import numpy as np
@@ -13,8 +13,8 @@ pytestmark = pytest.mark.gpu
 @pytest.fixture(scope="module")
 def ctx(pcu_pkg):
     c = pcu_pkg.Context(0)
-    # The screened tile kernels at every size (the default engine computes the smallest
-    # outputs in one fused launch).
+    # The screened tile kernels at every size (the default engine computes outputs of few cells
+    # in one launch).
     c.set_matmul_engine("mfma_products")
     yield c
     c.close()
@@ -40,28 +40,33 @@ def _operands(rng, m, k, n, tl, tr):
     return a, b
 
 
-# 32 x 32 tiles (few cells) and 64 x 64 tiles (more than three 32 x 32 tiles a CU).
-@pytest.mark.parametrize("m,n", [(1, 1), (31, 33), (32, 64), (36, 68), (65, 127), (896, 1024),
-                                 (900, 1028), (897, 1031)])
+# 32 x 32 tiles, up to three a CU and more; 64 x 64 tiles, two a CU; 128 x 128 tiles, one a CU.
+@pytest.mark.parametrize("m,n,tile", [(1, 1, 32), (31, 33, 32), (32, 64, 32), (36, 68, 32), (65, 127, 32),
+                                      (896, 1024, 32), (900, 1028, 32), (897, 1031, 32), (1408, 1408, 64),
+                                      (1400, 1404, 64), (1393, 1427, 64), (2040, 1932, 128), (2047, 1929, 128)])
 @pytest.mark.parametrize("tl", [False, True])
 @pytest.mark.parametrize("tr", [False, True])
-def test_tile_edges_and_slab_remainders(ctx, pcu_pkg, m, n, tl, tr):
+def test_tile_edges_and_slab_remainders(ctx, pcu_pkg, strict_tile, m, n, tile, tl, tr):
     rng = np.random.default_rng(m * 7 + n)
     small = m * n < 100000
     # None, one, two, three, four and five slabs of 32, whole and with 1 to 31 k over.
     for k in (1, 4, 31, 32, 33, 64, 68, 95, 96, 100, 127, 128, 132, 161) if small else (4, 61, 96, 132, 163):
+        assert strict_tile(np.float32, m, k, n, tl, tr, engine="mfma_products") == tile
         a, b = _operands(rng, m, k, n, tl, tr)
         _check(ctx, pcu_pkg, a, b, tl, tr, 0)
 
 
-@pytest.mark.parametrize("m,k,n", [(70, 100, 90), (68, 132, 92), (901, 70, 1030), (904, 100, 1032)])
+@pytest.mark.parametrize("m,k,n,tile", [(70, 100, 90, 32), (68, 132, 92, 32), (901, 70, 1030, 32),
+                                        (904, 100, 1032, 32), (1401, 70, 1405, 64), (1408, 100, 1404, 64),
+                                        (2041, 50, 1931, 128), (2044, 52, 1932, 128)])
 @pytest.mark.parametrize("policy", [0, 1, 2])
 @pytest.mark.parametrize("layout", [(False, False), (False, True), (True, False), (True, True)])
-def test_tiles_first_fault_and_partial_sums(ctx, pcu_pkg, m, k, n, policy, layout):
+def test_tiles_first_fault_and_partial_sums(ctx, pcu_pkg, strict_tile, m, k, n, tile, policy, layout):
     """Operands next to the tiles' edges replaced by values that fault (not a number, an
     overflow, a tiny product) or leave a subnormal partial sum (rejected under policy 1 only):
     in the last row, column and k, inside the slab remainder."""
     tl, tr = layout
+    assert strict_tile(np.float32, m, k, n, tl, tr, policy, "mfma_products") == tile
     rng = np.random.default_rng(m + 10 * policy + 100 * tl + 1000 * tr)
     for special in (np.nan, np.float32(3e38), np.float32(1e-30), None):
         a, b = _operands(rng, m, k, n, tl, tr)
@@ -81,10 +86,11 @@ def test_tiles_first_fault_and_partial_sums(ctx, pcu_pkg, m, k, n, policy, layou
 # F64: 64 x 64 tiles of its own, slabs of 16 k.
 @pytest.mark.parametrize("m,n", [(63, 1025), (64, 1024), (65, 1026), (513, 515)])
 @pytest.mark.parametrize("layout", [(False, False), (False, True), (True, False), (True, True)])
-def test_f64_tile_edges_and_slab_remainders(ctx, m, n, layout):
+def test_f64_tile_edges_and_slab_remainders(ctx, strict_tile, m, n, layout):
     tl, tr = layout
     rng = np.random.default_rng(m + n)
     for k in (1, 2, 15, 16, 17, 32, 47, 48, 50, 64, 65, 98):
+        assert strict_tile(np.float64, m, k, n, tl, tr, engine="mfma_products") == 64
         a = rng.uniform(-1, 1, (k, m) if tl else (m, k))
         b = rng.uniform(-1, 1, (n, k) if tr else (k, n))
         got = ctx.strict_matmul(ctx.upload(a), ctx.upload(b), tl, tr).numpy()

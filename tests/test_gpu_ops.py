@@ -397,9 +397,9 @@ ENGINES = ["auto", "valu", "mfma_products"]
 @pytest.fixture(params=ENGINES)
 def engine(request, ctx):
     """Runs a MatMul test once per engine; every engine must give the oracle's bits and
-    first fault. "auto" runs outputs of at most 256 x 256 cells (F32) or 512 x 512 (F64) as
-    one fused launch; "valu" and "mfma_products" always take the screened tile kernels
-    (F64 uses the vector unit under both)."""
+    first fault. "auto" runs outputs of few cells, where one launch is estimated to be the
+    faster way, as one launch; "valu" and "mfma_products" always take the screened tile
+    kernels (F64 uses the vector unit under both)."""
     ctx.set_matmul_engine(request.param)
     yield request.param
     ctx.set_matmul_engine("auto")
@@ -414,7 +414,7 @@ def engine(request, ctx):
                                    # whole, with 3, 4 and 6 slabs (every trip count of the
                                    # three-stage slab loop)
                                    (128, 48, 128), (256, 64, 128), (128, 96, 256),
-                                   # whole 64 x 64 tiles of 16 x 16 waves: 1, 5 and 17 slabs
+                                   # multiples of 64 cells: 1, 5 and 17 slabs of 16 k
                                    (64, 16, 64), (192, 80, 320), (448, 272, 512)])
 def test_matmul_parity_all_transposes(ctx, pcu_pkg, dtype, shape, engine):
     m, k, n = shape
@@ -526,12 +526,11 @@ def test_matmul_random_fault_placement_fuzz(ctx, pcu_pkg, dtype, engine):
 
 @pytest.mark.parametrize("grid", ["small", "full"])
 @pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
-def test_matmul_whole_tile_fuzz(ctx, pcu_pkg, dtype, engine, grid):
+def test_matmul_whole_tile_fuzz(ctx, pcu_pkg, strict_tile, dtype, engine, grid):
     """The same first-fault fuzz over whole tiles only (M and N multiples of 128, K of 16),
     where the main kernels load operands straight into LDS in per-layout arrangements and run
-    three slabs a trip. "small" outputs have fewer 128 x 128 tiles than the GPU has CUs (F32
-    runs 64 x 64 tiles, F64 its narrow tile); "full" ones have at least as many (the 128 x
-    128 kernels). 12 seeded cases over every layout and policy, a third clean (bits
+    three slabs a trip. "small" outputs run on the smaller tiles or, under "auto", in one
+    launch; "full" ones on the 128 x 128 kernels. 12 seeded cases over every layout and policy, a third clean (bits
     compared) and the rest with up to five special operands, so faults land in different
     slabs and stages; the GPU must give the oracle's first fault or, without one, its bits."""
     rng = np.random.default_rng((31 if dtype == np.float32 else 32) + (grid == "full") * 10)
@@ -539,7 +538,8 @@ def test_matmul_whole_tile_fuzz(ctx, pcu_pkg, dtype, engine, grid):
     specials = np.array([np.nan, np.inf, -np.inf, info.max, -info.max,
                          info.tiny * dtype(2.0 ** 20), -info.tiny * dtype(3.0),
                          info.smallest_subnormal * dtype(3.0)], dtype=dtype)
-    full_shapes = [(2048, 2048), (4096, 1024), (1024, 4096), (2048, 2560)]
+    full_shapes = ([(2048, 2048), (4096, 1024), (1024, 4096), (4096, 2048)] if dtype == np.float32 else
+                   [(2816, 2816), (4096, 2048), (2048, 4096), (3584, 2176)])
     for case in range(12):
         if grid == "small":
             m, n = (128 * int(v) for v in rng.integers(1, 4, size=2))
@@ -549,6 +549,8 @@ def test_matmul_whole_tile_fuzz(ctx, pcu_pkg, dtype, engine, grid):
             k = 16 * int(rng.integers(1, 9))
         tl, tr = case % 2 == 1, (case // 2) % 2 == 1
         policy = int(rng.integers(3))
+        if grid == "full":
+            assert strict_tile(dtype, m, k, n, tl, tr, policy, engine) == 128
         a = rng.uniform(-1, 1, (k, m) if tl else (m, k)).astype(dtype)
         b = rng.uniform(-1, 1, (n, k) if tr else (k, n)).astype(dtype)
         for x in (a, b):
@@ -1028,15 +1030,26 @@ def test_matmul_replay_paths_for_marked_cells(ctx, pcu_pkg, dtype, engine):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
-@pytest.mark.parametrize("shape", [(128, 32, 128), (128, 32, 144), (512, 64, 512), (640, 64, 640)],
-                         ids=["fused64", "fused72", "mid", "large"])
-def test_matmul_call_end_paths(ctx, pcu_pkg, dtype, shape):
+@pytest.mark.parametrize("shape,engine", [((128, 32, 128), "auto"), ((128, 32, 144), "auto"),
+                                          ((512, 64, 512), "mfma_products"), ((640, 64, 640), "mfma_products")],
+                         ids=["one64", "one72", "mid", "large"])
+def test_matmul_call_end_paths(ctx, pcu_pkg, strict_tile, dtype, shape, engine):
     """A single strict MatMul call ends its one-node program in one of its own kernels: the
-    one-launch small-output kernel when its grid has at most 64 workgroups (128 x 128: 64),
-    else a publication launch (128 x 144: 72); on the screened path the tiny scan when no
-    cell is suspect and the replay otherwise (512 x 512 binary32; binary64 takes the
-    one-launch kernel up to 512 x 512, so 640 x 640 reaches its screened path). Clean, a NaN
-    operand, a tiny-inexact product and clean again, back to back, against the oracle."""
+    one-launch kernel of few cells when its grid has at most 64 workgroups (128 x 128: 64),
+    else a publication launch (128 x 144: 72); on the screened path (512 x 512 and 640 x 640
+    under an engine that always takes it) the tiny scan when no cell is suspect and the replay
+    otherwise. Clean, a NaN operand, a tiny-inexact product and clean again, back to back,
+    against the oracle."""
+    m, k, n = shape
+    assert (strict_tile(dtype, m, k, n, engine=engine) == 16) == (engine == "auto")
+    ctx.set_matmul_engine(engine)
+    try:
+        _call_end_paths(ctx, pcu_pkg, dtype, shape)
+    finally:
+        ctx.set_matmul_engine("auto")
+
+
+def _call_end_paths(ctx, pcu_pkg, dtype, shape):
     m, k, n = shape
     rng = np.random.default_rng(m * 7 + n + k)
     tiny_a, tiny_b = (-100, -30) if dtype == np.float32 else (-1000, -40)
@@ -1144,12 +1157,15 @@ def test_matmul_screen_after_calls_of_other_shapes(ctx, pcu_pkg, policy, engine)
     assert _ofault(rf) == (cols - 1, 3, 1, 4)
 
 
-@pytest.mark.parametrize("shape", [(2048, 64, 2048), (2080, 33, 2050)], ids=["whole", "ragged"])
-def test_matmul_f64_full_grid_tile(ctx, pcu_pkg, shape):
-    """Binary64 outputs of at least 256 tiles of 128 x 128 take the 8 x 8-per-thread tile
-    (smaller ones the 8 x 4 tile that the other tests reach): every layout, clean and with
+@pytest.mark.parametrize("shape,tile", [((2816, 32, 2816), 128), ((2760, 33, 2750), 128),
+                                        ((2048, 64, 2048), 64), ((2080, 33, 2050), 64)],
+                         ids=["whole", "ragged", "whole64", "ragged64"])
+def test_matmul_f64_full_grid_tile(ctx, pcu_pkg, strict_tile, shape, tile):
+    """Binary64 outputs whose 128 x 128 tiles fill the CUs evenly enough take the 8 x
+    8-per-thread tile, others of that size the 64 x 64 one: every layout, clean and with
     planted NaN, overflow and tiny-inexact operands, against the oracle."""
     m, k, n = shape
+    assert strict_tile(np.float64, m, k, n) == tile
     rng = np.random.default_rng(m + k + n)
     for tl in (False, True):
         for tr in (False, True):

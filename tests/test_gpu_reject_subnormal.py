@@ -66,14 +66,28 @@ def _plant_cancellation(a, b, r, c, k1, k2, dtype):
     b[k1, c] = b[k2, c] = dtype(1.0)
 
 
-SHAPES = [  # (M, K, N, dtype, engine): the tile kernel each reaches
+SHAPES = [  # (M, K, N, dtype, engine): the tile kernel each reaches (see TILES)
     (2048, 64, 2048, np.float32, "mfma_products"),   # 128 x 128 whole tiles, three stages
-    (1024, 48, 1024, np.float32, "mfma_products"),   # 16 x 16 waves, whole 64 x 64 tiles
-    (1000, 40, 700, np.float32, "mfma_products"),    # 64 x 64 tiles with bound checks
+    (1024, 48, 1024, np.float32, "mfma_products"),   # 32 x 32 tiles
+    (1000, 40, 700, np.float32, "mfma_products"),    # 32 x 32 tiles, ragged
     (512, 64, 640, np.float32, "valu"),              # vector-unit binary32
     (2048, 32, 2048, np.float64, "valu"),            # binary64 8 x 8 block, full grid
+    (1408, 64, 1408, np.float32, "mfma_products"),   # 64 x 64 tiles
+    (1401, 41, 1405, np.float32, "mfma_products"),   # 64 x 64 tiles, ragged
+    (2040, 50, 1930, np.float32, "mfma_products"),   # 128 x 128 tiles with bound checks
 ]
-IDS = ["mfma128", "mfma16", "mfma64-ragged", "valu-f32", "valu-f64"]
+IDS = ["mfma128", "mfma32", "mfma32-ragged", "valu-f32", "valu-f64", "mfma64", "mfma64-ragged", "mfma128-ragged"]
+TILES = [128, 32, 32, 128, 128, 64, 64, 128]
+
+
+@pytest.mark.parametrize("i", range(len(TILES)), ids=IDS)
+def test_shapes_reach_their_tile_kernels(strict_tile, i):
+    for m, k, n, dtype, engine in (SHAPES[i], DEEP[i]):
+        for tl, tr in ((False, False), (True, False), (False, True)):
+            assert strict_tile(dtype, m, k, n, tl, tr, 1, engine) == TILES[i], (m, k, n)
+    m, n, ks, dtype, engine = FUZZ_FAMILIES[i]
+    for k in ks:
+        assert strict_tile(dtype, m, k, n, policy=1, engine=engine) == TILES[i], (m, k, n)
 
 
 @pytest.mark.parametrize("shape", SHAPES, ids=IDS)
@@ -166,6 +180,9 @@ DEEP = [  # (M, K, N, dtype, engine): the same tile kernels over four superslabs
     (1000, 200, 700, np.float32, "mfma_products"),
     (512, 256, 640, np.float32, "valu"),
     (2048, 256, 2048, np.float64, "valu"),
+    (1408, 256, 1408, np.float32, "mfma_products"),
+    (1401, 201, 1405, np.float32, "mfma_products"),
+    (2040, 200, 1930, np.float32, "mfma_products"),
 ]
 
 
@@ -268,13 +285,16 @@ def test_tiny_products_through_superslab_tables(ctx, pcu_pkg, shape):
 
 FUZZ_FAMILIES = [  # (M, N, K choices, dtype, engine): each reaches one tile kernel
     (2048, 2048, (64, 144, 256), np.float32, "mfma_products"),  # whole 128 x 128, three stages
-    (2100, 2000, (48, 200), np.float32, "mfma_products"),       # 128 x 128 with bound checks
-    (1024, 1024, (112, 256), np.float32, "mfma_products"),      # 16 x 16 waves, 64 x 64 tiles
-    (1000, 700, (40, 177), np.float32, "mfma_products"),        # 64 x 64 with bound checks
+    (1024, 1024, (112, 256), np.float32, "mfma_products"),      # 32 x 32 tiles
+    (1000, 700, (40, 177), np.float32, "mfma_products"),        # 32 x 32, ragged
     (640, 520, (96, 250), np.float32, "valu"),                  # vector-unit binary32
     (2048, 2048, (80, 192), np.float64, "valu"),                # binary64 full grid
+    (1408, 1408, (112, 256), np.float32, "mfma_products"),      # 64 x 64 tiles
+    (1401, 1405, (40, 177), np.float32, "mfma_products"),       # 64 x 64, ragged
+    (2040, 1930, (50, 200), np.float32, "mfma_products"),       # 128 x 128 with bound checks
+    (2100, 2000, (48, 200), np.float32, "mfma_products"),       # 32 x 32, many tiles a CU
 ]
-FUZZ_IDS = ["mfma128", "mfma128-ragged", "mfma16", "mfma64-ragged", "valu-f32", "valu-f64"]
+FUZZ_IDS = IDS + ["mfma32-many"]
 
 
 @pytest.mark.parametrize("family", FUZZ_FAMILIES, ids=FUZZ_IDS)

@@ -2,25 +2,19 @@
 cells). The choice is made on the host, so it is checked without a GPU."""
 import ctypes
 
+import numpy as np
 import pytest
 
-AUTO, VALU, MFMA = 0, 1, 2
 IEEE, REJECT, GRADUAL = 0, 1, 2
 
 
 @pytest.fixture(scope="module")
-def tile(pcu_pkg):
-    f = pcu_pkg.lib().pcu_internal_strict_matmul_tile
-    f.argtypes = [ctypes.c_int] + 3 * [ctypes.c_uint64] + 4 * [ctypes.c_int]
-    f.restype = ctypes.c_int
-
-    def call(dtype, m, k, n, tl=False, tr=False, policy=IEEE, engine=AUTO):
-        return f({"f32": 0, "f64": 1}[dtype], m, k, n, int(tl), int(tr), policy, engine)
-
-    return call
+def tile(strict_tile):
+    types = {"f32": np.float32, "f64": np.float64}
+    return lambda dtype, *args, **kw: strict_tile(types[dtype], *args, **kw)
 
 
-@pytest.mark.parametrize("engine", [VALU, MFMA])
+@pytest.mark.parametrize("engine", ["valu", "mfma_products"])
 def test_a_chosen_engine_always_takes_the_tile_kernels(tile, engine):
     for dtype in ("f32", "f64"):
         for m in (1, 16, 64, 256, 1000, 4096):
@@ -74,7 +68,7 @@ def test_native_whole_tiles_need_aligned_operands(pcu_pkg):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("name,engine", [("auto", AUTO), ("valu", VALU), ("mfma_products", MFMA)])
+@pytest.mark.parametrize("name,engine", [("auto", 0), ("valu", 1), ("mfma_products", 2)])
 def test_a_context_runs_with_the_engine_it_was_given(pcu_pkg, name, engine):
     f = pcu_pkg.lib().pcu_internal_matmul_engine
     f.argtypes, f.restype = [ctypes.c_void_p], ctypes.c_int
