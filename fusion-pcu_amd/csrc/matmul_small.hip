@@ -172,6 +172,7 @@ __global__ __launch_bounds__(256, (kSmallWaves<L, ONE>)) void k_strict_gemm_smal
         constexpr bool KC = decltype(kc_c)::value, VEC = KC && decltype(vec_c)::value;
         constexpr bool FULL = decltype(full_c)::value;
         uint4 q[L];
+        const size_t first = KC ? 0 : (size_t)(k0 + kt) * ld, last = KC ? 0 : (size_t)(K - 1) * ld;
 #pragma unroll
         for (int j = 0; j < L; j++) {
             const int k = k0 + kt + 16 * P * j;
@@ -180,8 +181,8 @@ __global__ __launch_bounds__(256, (kSmallWaves<L, ONE>)) void k_strict_gemm_smal
             } else {
 #pragma unroll
                 for (int c = 0; c < P; c++) {
-                    const int kk = FULL || k + c < K ? k + c : K - 1;
-                    v[j][c] = p[KC ? (size_t)kk : (size_t)kk * ld];
+                    const bool in = FULL || k + c < K;
+                    v[j][c] = p[KC ? (size_t)(in ? k + c : K - 1) : (in ? first + (size_t)(16 * P * j + c) * ld : last)];
                 }
             }
         }
