@@ -908,21 +908,15 @@ hipError_t launch_fill_u32(hipStream_t s, unsigned int *p, uint64_t n, uint32_t 
 static inline bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
 
 // A stored R x C matrix copied into C x R (R and C multiples of 4, both pointers 16-byte
-// aligned): 64 x 64 tiles through LDS, runs of four elements (one or two 16-byte loads and
-// stores), rows of the tile padded by one element. Used for a transposed op(B) that the
-// tile kernel then loads as an untransposed one: the copy holds the same values, so every
-// product, sum and fault of the MatMul is unchanged.
-template <typename T> struct alignas(16) Run4 {
-    T v[4];
-};
-
-template <typename T>
-__global__ __launch_bounds__(256) void k_transpose(const T *__restrict__ X, T *__restrict__ Y,
+// aligned): 64 x 64 tiles through LDS, 16-byte loads and stores, rows of the tile padded by one
+// element. Used for a transposed op(B) that the tile kernel then loads as an untransposed one:
+// the copy holds the same values, so every product, sum and fault of the MatMul is unchanged.
+__global__ __launch_bounds__(256) void k_transpose(const float *__restrict__ X, float *__restrict__ Y,
                                                    int R, int C, NodeGate gate)
 {
     if (block_gate_closed(gate))
         return;
-    __shared__ T t[64][65];
+    __shared__ float t[64][65];
     const int tiles_c = (C + 63) / 64;
     const int r0 = (int)(blockIdx.x / tiles_c) * 64, c0 = (int)(blockIdx.x % tiles_c) * 64;
     const int q = threadIdx.x & 15, row = threadIdx.x >> 4; // 16 runs of 4 floats x 16 rows
@@ -930,23 +924,20 @@ __global__ __launch_bounds__(256) void k_transpose(const T *__restrict__ X, T *_
     for (int p = 0; p < 4; p++) {
         const int i = row + 16 * p, r = r0 + i, c = c0 + 4 * q;
         if (r < R && c < C) {
-            const Run4<T> v = *reinterpret_cast<const Run4<T> *>(X + (size_t)r * C + c);
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-                t[i][4 * q + e] = v.v[e];
+            const float4 v = *reinterpret_cast<const float4 *>(X + (size_t)r * C + c);
+            t[i][4 * q] = v.x;
+            t[i][4 * q + 1] = v.y;
+            t[i][4 * q + 2] = v.z;
+            t[i][4 * q + 3] = v.w;
         }
     }
     __syncthreads();
 #pragma unroll
     for (int p = 0; p < 4; p++) {
         const int j = row + 16 * p, c = c0 + j, r = r0 + 4 * q;
-        if (c < C && r < R) {
-            Run4<T> v;
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-                v.v[e] = t[4 * q + e][j];
-            *reinterpret_cast<Run4<T> *>(Y + (size_t)c * R + r) = v;
-        }
+        if (c < C && r < R)
+            *reinterpret_cast<float4 *>(Y + (size_t)c * R + r) =
+                make_float4(t[4 * q][j], t[4 * q + 1][j], t[4 * q + 2][j], t[4 * q + 3][j]);
     }
 }
 
@@ -964,8 +955,7 @@ bool matmul_bt_wanted(int dtype, uint64_t rows, uint64_t inner, uint64_t cols, b
         return false; // the launch for few cells reads B in place
     // Whole 128 x 128 tiles filling at least one workgroup a CU: the copy measured 2-2.5%
     // faster there (NT 4096^3 1973 against 2021 us, 4096 x 1024 x 4096 510 against 521, TT
-    // 4096^3 -2%), and 4.5-7% slower on the 64 x 64 tiles of smaller grids (1024^3 NT 57.1
-    // against 54.6 us).
+    // 4096^3 -2%). The smaller tiles load either layout straight into LDS and read B in place.
     return rows % 128 == 0 && cols % 128 == 0 && (rows / 128) * (cols / 128) >= 256 &&
            inner * cols <= kBtMaxElems && mid_tile_f32(rows, cols, inner, true) == MidTile::k128;
 }
@@ -1111,7 +1101,7 @@ static hipError_t strict_matmul_t(hipStream_t s, uint64_t M, uint64_t K, uint64_
         bool tbt = tb;
         if (tb && sc.bt && aligned16(B)) {
             const unsigned tiles = (unsigned)(((N + 63) / 64) * ((K + 63) / 64));
-            hipLaunchKernelGGL(k_transpose<float>, dim3(tiles), dim3(256), 0, s, (const float *)B,
+            hipLaunchKernelGGL(k_transpose, dim3(tiles), dim3(256), 0, s, (const float *)B,
                                (float *)sc.bt, n, k, gate);
             Bt = (const float *)sc.bt;
             tbt = false;
