@@ -944,14 +944,15 @@ __global__ __launch_bounds__(256) void k_transpose(const float *__restrict__ X, 
 // Largest op(B) copied out (2^28 elements); larger ones are read in place.
 constexpr uint64_t kBtMaxElems = 1ull << 28;
 
-bool matmul_bt_wanted(int dtype, uint64_t rows, uint64_t inner, uint64_t cols, bool tr, int engine)
+bool matmul_bt_wanted(int dtype, uint64_t rows, uint64_t inner, uint64_t cols, bool tr, int policy,
+                      int engine)
 {
     // Binary64 reads it in place: with the copy NT 4096^3 took 4727 to 4847 us a call against 4547
     // to 4739, 4096 x 1024 x 4096 1306 against 1279, 4096 x 512 x 4096 717 against 702, and
     // RejectSubnormal NT 2048^3 784 against 699.
     if (dtype != 0 || !tr || engine == kEngineValu || inner == 0 || inner % 16 != 0)
         return false;
-    if (engine == kEngineAuto && gemm_small_wanted(dtype, rows, inner, cols))
+    if (engine == kEngineAuto && gemm_small_wanted(dtype, rows, inner, cols, policy))
         return false; // the launch for few cells reads B in place
     // Whole 128 x 128 tiles filling at least one workgroup a CU: the copy measured 2-2.5%
     // faster there (NT 4096^3 1973 against 2021 us, 4096 x 1024 x 4096 510 against 521, TT
@@ -999,7 +1000,7 @@ static bool sum_check_wanted(int dtype, uint64_t M, uint64_t K, uint64_t N, int 
 int strict_matmul_tile(int dtype, uint64_t rows, uint64_t inner, uint64_t cols, bool ta, bool tb,
                        int policy, int engine, bool sum_flags)
 {
-    if (engine == kEngineAuto && inner > 0 && gemm_small_wanted(dtype, rows, inner, cols))
+    if (engine == kEngineAuto && inner > 0 && gemm_small_wanted(dtype, rows, inner, cols, policy))
         return 16;
     if (dtype == 0 && engine != kEngineValu) {
         const MidTile t = mfma_tile_f32(rows, cols, inner, ta, tb);

@@ -482,18 +482,20 @@ static double small_time(int dtype, double c, uint64_t inner)
         return 3.3 + c * (0.3 + 0.0085 * K);
     if (inner <= 128)
         return 4.5 + c * (0.6 + 0.0065 * K);
-    return c <= 1 ? 3.5 + 16.5 * k : 4 + c * (0.5 + 12.4 * k);
+    return c <= 1 ? 3.5 + 16.5 * k : 4 + c * (0.15 + 12.5 * k);
 }
 
 // Against the screened tile kernels: their screen (about 4.5 us, 2 more for each 1024 k of a row,
 // and both operands at 6 MB a us), the tiles as mid_time_f32 and mid_wanted_f64 put them, which leaves
 // out a fixed part and the store of the output, and the further launches (0.5 us; whole calls of
-// either route otherwise take their kernels and 11.5 us). Whole calls, this kernel against the tiles,
+// either route otherwise take their kernels and 11.5 us). AllowGradual needs no screen, only a
+// launch that opens the words (2.5 to 3.2 us: binary32 768 x 19 x 2270 25.0 us on tiles, 26.2 here;
+// 512 x 256 x 1024 24.1 / 25.9, 26.5 / 26.5 under IEEE). Whole calls, this kernel against the tiles,
 // on both sides of the line: binary32 512 x 8 x 1024 18.0 / 21.0 us, 1024 x 8 x 1024 20.7 / 22.2, 4096
 // x 8 x 512 26.0 / 24.5, 1024 x 64 x 1024 23.8 / 24.9, 512 x 100 x 1024 23.2 / 23.8, 1024 x 100 x 1024
 // 30.4 / 26.7, 512 x 256 x 512 21.5 / 25.3, 512 x 1024 x 256 28.7 / 50; binary64 1024 x 8 x 1024 21.7
 // / 23.0, 4096 x 8 x 512 27.5 / 25.8, 512 x 128 x 1024 27.9 / 33.1, 1024 x 128 x 1024 44 / 34.
-bool gemm_small_wanted(int dtype, uint64_t rows, uint64_t inner, uint64_t cols)
+bool gemm_small_wanted(int dtype, uint64_t rows, uint64_t inner, uint64_t cols, int policy)
 {
     const auto per_cu = [&](uint64_t t) {
         const uint64_t tiles = ((rows + t - 1) / t) * ((cols + t - 1) / t);
@@ -504,7 +506,7 @@ bool gemm_small_wanted(int dtype, uint64_t rows, uint64_t inner, uint64_t cols)
         return false;
     const double k = (double)inner / 1024.0, cells = (double)rows * (double)cols;
     const double mb = ((double)rows + (double)cols) * (double)inner * (dtype == 0 ? 4e-6 : 8e-6);
-    double tiles = 4.5 + 2 * k + mb / 6 + 0.5;
+    double tiles = policy == kPolicyAllowGradual ? (dtype == 0 ? 2.5 : 3.2) : 4.5 + 2 * k + mb / 6 + 0.5;
     if (dtype == 0) {
         tiles += mid_time_f32(rows, cols, inner) + 2 + 1.2e-6 * cells;
     } else {

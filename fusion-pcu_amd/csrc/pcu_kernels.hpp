@@ -170,7 +170,8 @@ struct SumCheck {
 // transposed op(B) stored K x N (grids of whole 128 x 128 tiles, K a multiple of 16): the tile
 // kernel loads an untransposed op(B) straight into LDS but stages a transposed one through
 // registers.
-bool matmul_bt_wanted(int dtype, uint64_t rows, uint64_t inner, uint64_t cols, bool tr, int engine);
+bool matmul_bt_wanted(int dtype, uint64_t rows, uint64_t inner, uint64_t cols, bool tr, int policy,
+                      int engine);
 // `sum_flags`: the scratch also carries the partial-sum block words. The superslab tables
 // take a buffer of their own of slab_table_bytes() bytes (0: too large, none), or none.
 size_t matmul_scratch_bytes(uint64_t rows, uint64_t cols, bool sum_flags);
@@ -223,7 +224,7 @@ hipError_t launch_gemm_mid_f64(hipStream_t s, bool native, int M, int N, int K, 
 
 // Strict MatMul of few cells in one launch (matmul_small.hip): screen, products, ordered sums
 // and the exact first-fault search. `wanted`: whether it is the faster route (inner > 0).
-bool gemm_small_wanted(int dtype, uint64_t rows, uint64_t inner, uint64_t cols);
+bool gemm_small_wanted(int dtype, uint64_t rows, uint64_t inner, uint64_t cols, int policy);
 hipError_t launch_gemm_small(hipStream_t s, int dtype, int M, int N, int K, bool ta, bool tb,
                              const void *A, const void *B, void *C, int thr, int risk, int policy,
                              unsigned long long *fault, NodeGate gate, ProgramClose close,

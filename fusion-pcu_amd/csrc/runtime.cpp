@@ -824,7 +824,7 @@ pcu_status Ctx::op_matmul(int dtype, uint64_t rows, uint64_t inner, uint64_t col
     // place.
     // The copy is only a speed-up: when it cannot be allocated the tile kernel reads B in
     // place, as for every other layout.
-    if (!noalloc && matmul_bt_wanted(dtype, rows, inner, cols, tr != 0, matmul_engine))
+    if (!noalloc && matmul_bt_wanted(dtype, rows, inner, cols, tr != 0, policy, matmul_engine))
         s.bt = optional_scratch(bt_scratch, (size_t)(inner * cols * dsize(dtype)));
 
     // Per-kernel timing takes events from a pool that may grow, so the no-allocation call

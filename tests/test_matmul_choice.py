@@ -46,6 +46,15 @@ def test_short_sums_of_many_cells_take_the_tiles(tile, dtype):
         assert tile(dtype, m, k, n) != 16, (m, k, n)
 
 
+def test_the_choice_counts_the_screen_where_there_is_one(tile):
+    """AllowGradual needs no exponent screen, so its tiles are the faster way a little earlier."""
+    for m, k, n in ((512, 256, 1024), (768, 19, 2270), (1024, 64, 1024), (512, 300, 512)):
+        assert tile("f32", m, k, n, policy=GRADUAL) != 16
+    for m, k, n in ((512, 8, 512), (512, 256, 512), (64, 4096, 1024)):
+        for policy in (IEEE, REJECT, GRADUAL):
+            assert tile("f32", m, k, n, policy=policy) == 16 and tile("f64", m, k, n, policy=policy) == 16
+
+
 @pytest.mark.parametrize("dtype", ["f32", "f64"])
 def test_few_cells_take_one_launch(tile, dtype):
     for m, k, n in ((64, 256, 64), (1, 1, 1), (64, 4096, 1024), (512, 8, 512), (1024, 8, 1024), (512, 64, 1024),
