@@ -56,14 +56,16 @@ static void mid_layout(hipStream_t s, MidTile tile, int M, int N, int K, const f
 }
 
 // Estimated microseconds of each tile, from measurements on MI355X: the tiles of the fullest
-// CU times what one takes, per 1024 k and fixed. A 128 x 128 tile: 118 (whole tiles) or 131
-// (bound checks; 140 alone on its CU) + 4. A 64 x 64 tile: 32.5 + 2, alone 36 + 4. Up to three
-// 32 x 32 tiles run at once, 16 / 22.5 / 29 + 3 together; more, 9.3 + 0.5 each. The estimates
-// pick the faster tile or one within 2% of it over 1024^3, 1500^3, 2050^3, 3001^3, 4000^3,
-// 1536 x 1024 x 1536, 1920 x 1024 x 1920, 100 x 2000 x 9000, 8190 x 512 x 8190 and the shapes
-// above: no single bound on the number of tiles does (a 2050 x 2050 output takes 541 us on
-// 289 128 x 128 tiles, two rounds for one, and 329 on 4225 of 32 x 32; 8190 x 8190 takes 1119
-// and 1303).
+// CU times what one takes, per 1024 k and fixed, and a fixed part. A 128 x 128 tile: 118 + 2.5
+// (whole tiles) or 131 + 4 (bound checks; 140 alone on its CU), and 8. A 64 x 64 tile: 32.5 + 2 and
+// 2.5, alone 36 and 5.5. Up to three 32 x 32 tiles run at once, 16 / 22.5 / 29 together and 4.5;
+// more, 9.3 + 0.7 each and 2.5. The fixed parts decide short sums: kernels on 32 x 32 / 64 x 64 /
+// 128 x 128 tiles, 768 x 19 x 2270 10.5 / 8.8 / 17.2 us, 1000 x 8 x 1500 9.3 / 7.7 / 14.4, 2048 x 19
+// x 2048 20.6 / 16.2 / 18.5, 4096 x 32 x 2048 29.4 / 26.0 / 20.1, 3000 x 64 x 3000 41.6 / 39.0 /
+// 43.4. Over K = 8 to 4000 and 512^2 to 8192^2 cells the estimates pick the fastest tile or one
+// within 4% of it: 1500^3 125 / 154 / 216, 2050^3 315 / 341 / 602 (289 128 x 128 tiles are two
+// rounds for one), 2048 x 256 x 2048 48.8 / 45.2 / 43.6, 2040 x 1024 x 2040 153 / 143 / 158, 4000^3
+// 2393 / 2110 / 2230, 8190 x 512 x 8190 1346 / 1171 / 1098.
 static MidTile mid_choose(uint64_t M, uint64_t N, uint64_t K, bool whole, double &us)
 {
     const auto per_cu = [&](uint64_t t) {
@@ -71,9 +73,9 @@ static MidTile mid_choose(uint64_t M, uint64_t N, uint64_t K, bool whole, double
         return (double)((tiles + kGfx950Cus - 1) / kGfx950Cus);
     };
     const double k = (double)K / 1024.0, c32 = per_cu(32), c64 = per_cu(64), c128 = per_cu(128);
-    const double t32 = c32 <= 3 ? (9.5 + 6.5 * c32) * k + 3 : c32 * (9.3 * k + 0.5);
-    const double t64 = c64 <= 1 ? 36 * k + 4 : c64 * (32.5 * k + 2);
-    const double t128 = c128 * ((whole ? 118 : c128 <= 1 ? 140 : 131) * k + 4);
+    const double t32 = c32 <= 3 ? (9.5 + 6.5 * c32) * k + 4.5 : c32 * (9.3 * k + 0.7) + 2.5;
+    const double t64 = c64 <= 1 ? 36 * k + 5.5 : c64 * (32.5 * k + 2) + 2.5;
+    const double t128 = 8 + c128 * (whole ? 118 * k + 2.5 : (c128 <= 1 ? 140 : 131) * k + 4);
     us = t32 < t64 ? t32 : t64;
     if (t128 <= us) {
         us = t128;

@@ -486,8 +486,8 @@ static double small_time(int dtype, double c, uint64_t inner)
 }
 
 // Against the screened tile kernels: their screen (about 4.5 us, 2 more for each 1024 k of a row,
-// and both operands at 6 MB a us), the tiles as mid_time_f32 and mid_wanted_f64 put them, which leaves
-// out a fixed part and the store of the output, and the further launches (0.5 us; whole calls of
+// and both operands at 6 MB a us), the tiles as mid_time_f32 and mid_wanted_f64 put them with the store
+// of the output (and, binary64, a fixed part), and the further launches (0.5 us; whole calls of
 // either route otherwise take their kernels and 11.5 us). AllowGradual needs no screen, only a
 // launch that opens the words (2.5 to 3.2 us: binary32 768 x 19 x 2270 25.0 us on tiles, 26.2 here;
 // 512 x 256 x 1024 24.1 / 25.9, 26.5 / 26.5 under IEEE). Whole calls, this kernel against the tiles,
@@ -508,7 +508,7 @@ bool gemm_small_wanted(int dtype, uint64_t rows, uint64_t inner, uint64_t cols, 
     const double mb = ((double)rows + (double)cols) * (double)inner * (dtype == 0 ? 4e-6 : 8e-6);
     double tiles = policy == kPolicyAllowGradual ? (dtype == 0 ? 2.5 : 3.2) : 4.5 + 2 * k + mb / 6 + 0.5;
     if (dtype == 0) {
-        tiles += mid_time_f32(rows, cols, inner) + 2 + 1.2e-6 * cells;
+        tiles += mid_time_f32(rows, cols, inner) + 0.5 + 1e-6 * cells;
     } else {
         const double c64 = per_cu(64);
         tiles += (c64 <= 2 ? 26 + 65 * c64 : 74 * c64) * k + 3.5 + 1.8e-6 * cells;

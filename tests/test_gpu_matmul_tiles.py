@@ -40,10 +40,10 @@ def _operands(rng, m, k, n, tl, tr):
     return a, b
 
 
-# 32 x 32 tiles, up to three a CU and more; 64 x 64 tiles, two a CU; 128 x 128 tiles, one a CU.
+# 32 x 32 tiles, up to three a CU and more; 64 x 64 tiles, two a CU; 128 x 128 tiles, two a CU.
 @pytest.mark.parametrize("m,n,tile", [(1, 1, 32), (31, 33, 32), (32, 64, 32), (36, 68, 32), (65, 127, 32),
                                       (896, 1024, 32), (900, 1028, 32), (897, 1031, 32), (1408, 1408, 64),
-                                      (1400, 1404, 64), (1393, 1427, 64), (2040, 1932, 128), (2047, 1929, 128)])
+                                      (1400, 1404, 64), (1393, 1427, 64), (4092, 2036, 128), (4089, 2041, 128)])
 @pytest.mark.parametrize("tl", [False, True])
 @pytest.mark.parametrize("tr", [False, True])
 def test_tile_edges_and_slab_remainders(ctx, pcu_pkg, strict_tile, m, n, tile, tl, tr):
@@ -58,7 +58,7 @@ def test_tile_edges_and_slab_remainders(ctx, pcu_pkg, strict_tile, m, n, tile, t
 
 @pytest.mark.parametrize("m,k,n,tile", [(70, 100, 90, 32), (68, 132, 92, 32), (901, 70, 1030, 32),
                                         (904, 100, 1032, 32), (1401, 70, 1405, 64), (1408, 100, 1404, 64),
-                                        (2041, 50, 1931, 128), (2044, 52, 1932, 128)])
+                                        (4089, 50, 2041, 128), (4092, 52, 2036, 128)])
 @pytest.mark.parametrize("policy", [0, 1, 2])
 @pytest.mark.parametrize("layout", [(False, False), (False, True), (True, False), (True, True)])
 def test_tiles_first_fault_and_partial_sums(ctx, pcu_pkg, strict_tile, m, k, n, tile, policy, layout):

@@ -74,7 +74,7 @@ SHAPES = [  # (M, K, N, dtype, engine): the tile kernel each reaches (see TILES)
     (2048, 32, 2048, np.float64, "valu"),            # binary64 8 x 8 block, full grid
     (1408, 64, 1408, np.float32, "mfma_products"),   # 64 x 64 tiles
     (1401, 41, 1405, np.float32, "mfma_products"),   # 64 x 64 tiles, ragged
-    (2040, 50, 1930, np.float32, "mfma_products"),   # 128 x 128 tiles with bound checks
+    (4089, 50, 2036, np.float32, "mfma_products"),   # 128 x 128 tiles with bound checks
 ]
 IDS = ["mfma128", "mfma32", "mfma32-ragged", "valu-f32", "valu-f64", "mfma64", "mfma64-ragged", "mfma128-ragged"]
 TILES = [128, 32, 32, 128, 128, 64, 64, 128]
@@ -176,13 +176,13 @@ def test_reject_subnormal_after_calls_of_other_shapes(pcu_pkg):
 
 DEEP = [  # (M, K, N, dtype, engine): the same tile kernels over four superslabs of 64 k
     (2048, 256, 2048, np.float32, "mfma_products"),
-    (1024, 256, 1024, np.float32, "mfma_products"),
+    (768, 256, 1024, np.float32, "mfma_products"),
     (1000, 200, 700, np.float32, "mfma_products"),
     (512, 256, 640, np.float32, "valu"),
     (2048, 256, 2048, np.float64, "valu"),
     (1408, 256, 1408, np.float32, "mfma_products"),
     (1401, 201, 1405, np.float32, "mfma_products"),
-    (2040, 200, 1930, np.float32, "mfma_products"),
+    (4089, 200, 2036, np.float32, "mfma_products"),
 ]
 
 
@@ -285,13 +285,13 @@ def test_tiny_products_through_superslab_tables(ctx, pcu_pkg, shape):
 
 FUZZ_FAMILIES = [  # (M, N, K choices, dtype, engine): each reaches one tile kernel
     (2048, 2048, (64, 144, 256), np.float32, "mfma_products"),  # whole 128 x 128, three stages
-    (1024, 1024, (112, 256), np.float32, "mfma_products"),      # 32 x 32 tiles
+    (1024, 1024, (112, 160), np.float32, "mfma_products"),      # 32 x 32 tiles
     (1000, 700, (40, 177), np.float32, "mfma_products"),        # 32 x 32, ragged
     (640, 520, (96, 250), np.float32, "valu"),                  # vector-unit binary32
     (2048, 2048, (80, 192), np.float64, "valu"),                # binary64 full grid
     (1408, 1408, (112, 256), np.float32, "mfma_products"),      # 64 x 64 tiles
     (1401, 1405, (40, 177), np.float32, "mfma_products"),       # 64 x 64, ragged
-    (2040, 1930, (50, 200), np.float32, "mfma_products"),       # 128 x 128 with bound checks
+    (4089, 2036, (50, 200), np.float32, "mfma_products"),       # 128 x 128 with bound checks
     (2100, 2000, (48, 200), np.float32, "mfma_products"),       # 32 x 32, many tiles a CU
 ]
 FUZZ_IDS = IDS + ["mfma32-many"]
